@@ -2,101 +2,235 @@
 // dense_mm / mat_vec_mul (3d/mat_vec_mul_dense.h:25-73: gemv with alpha = 1,
 // beta = 0, leading dimension lda).
 //
-// N (y = A x): a thread owns a row and walks a slab of columns, so a
-// wavefront reads 64 consecutive entries of one column (coalesced); the
-// column range is split over gridDim.y slabs and the slab partials are summed
-// in a fixed order by a second kernel (deterministic, no atomics).
-// T (y = A^T x): a wavefront owns a column; lanes read it contiguously.
+// Both are bound by reading A once, so both load it 16 bytes a lane (W = 16 /
+// sizeof(V) entries of one column; a wavefront load is 1 KB of one column).
+// Measured against one entry a lane and load: 8192 x 16384 BF16, N 108 + 36
+// (partial sums) -> 40 + 5 us, T 107 -> 50 us (6.7 and 5.4 TB/s of a matrix
+// partly in the memory-side cache); 1638 x 4096 FP32, N 20 + 17 -> 6.6 + 2.6
+// us, T 10.3 -> 6.9 us.
+// Columns start at any multiple of the element size (lda and the caller's
+// matrix decide), so the loads are declared with the element's alignment.
+//
+// N (y = A x): a wavefront owns 64 W rows and walks columns, eight loads in
+// flight; the four wavefronts of a workgroup walk neighbouring column runs of
+// the same rows and add up in LDS; gridDim.y column slabs fill the chip and
+// their partial sums are added by a second kernel.  Fixed orders, no atomics.
+// T (y = A^T x): a wavefront owns C columns and walks their rows, so that W
+// values of x in registers serve C loads of A (with one column, x is 2 bytes
+// of L1 traffic per byte of a BF16 matrix and set the pace).
+#include <algorithm>
+
+#include "lanes.hpp"
 #include "tv3_internal.hpp"
 
 namespace tv3 {
 
-template <typename V> __device__ __forceinline__ float ldv(const V *p, int64_t k);
-template <> __device__ __forceinline__ float ldv<float>(const float *p, int64_t k) { return p[k]; }
-template <> __device__ __forceinline__ float ldv<__half>(const __half *p, int64_t k) {
-    return __half2float(p[k]);
-}
-template <> __device__ __forceinline__ float ldv<__hip_bfloat16>(const __hip_bfloat16 *p, int64_t k) {
-    return __bfloat162float(p[k]);
-}
-__device__ __forceinline__ double ldd(const double *p, int64_t k) { return p[k]; }
-__device__ __forceinline__ double ldd(const float *p, int64_t k) { return (double)p[k]; }
+namespace {
 
-template <typename V, typename AccT>
-__device__ __forceinline__ AccT loadA(const V *A, int64_t k) {
-    if constexpr (std::is_same<V, double>::value) return (AccT)A[k];
-    else if constexpr (std::is_same<V, float>::value) return (AccT)A[k];
-    else return (AccT)ldv<V>(A, k);
+// W consecutive values at any multiple of their own size
+template <typename V, int W>
+struct __attribute__((packed, aligned(alignof(V)))) Run {
+    V v[W];
+};
+
+template <typename V, int W>
+__device__ __forceinline__ Run<V, W> load_run(const V *p) {
+    return *reinterpret_cast<const Run<V, W> *>(p);
 }
 
-template <typename V, typename T, typename AccT>
+template <typename AccT, typename V>
+__device__ __forceinline__ AccT up(V v) {
+    if constexpr (std::is_same<V, __half>::value) return (AccT)__half2float(v);
+    else if constexpr (std::is_same<V, __hip_bfloat16>::value) return (AccT)__bfloat162float(v);
+    else return (AccT)v;
+}
+
+// entries per lane and load: 16 bytes' worth
+template <typename V> constexpr int run_of() { return 16 / (int)sizeof(V); }
+
+constexpr int kColsInFlight = 8;
+
+// Rows beyond the last whole run are covered by moving the last lanes' runs
+// back to end at row m (m >= W): a row held by two lanes gets the same sum
+// twice and both store it.
+template <typename V, int W, typename T, typename AccT>
 __global__ __launch_bounds__(256) void k_gemv_n_part(int64_t m, int64_t n, int64_t lda,
                                                      const V *__restrict__ A,
                                                      const T *__restrict__ x,
-                                                     AccT *__restrict__ part, int64_t cols_per) {
-    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    int64_t j0 = (int64_t)blockIdx.y * cols_per, j1 = j0 + cols_per < n ? j0 + cols_per : n;
-    if (i >= m) return;
-    AccT s = 0;
-    for (int64_t j = j0; j < j1; ++j) s += loadA<V, AccT>(A, i + j * lda) * (AccT)x[j];
-    part[(int64_t)blockIdx.y * m + i] = s;
+                                                     AccT *__restrict__ part, T *__restrict__ y,
+                                                     int64_t cols_per) {
+    __shared__ AccT sh[3][64 * W];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t i = min(((int64_t)blockIdx.x * 64 + lane) * W, m - W);
+    const int64_t s0 = (int64_t)blockIdx.y * cols_per, s1 = min(s0 + cols_per, n);
+    const int64_t per = (cols_per + 3) / 4;
+    const int64_t j0 = min(s0 + wave * per, s1), j1 = min(j0 + per, s1);
+    AccT s[W] = {};
+    const V *a = A + i + j0 * lda;
+    int64_t j = j0;
+    for (; j + kColsInFlight <= j1; j += kColsInFlight, a += kColsInFlight * lda) {
+        Run<V, W> r[kColsInFlight];
+#pragma unroll
+        for (int c = 0; c < kColsInFlight; ++c) r[c] = load_run<V, W>(a + c * lda);
+#pragma unroll
+        for (int c = 0; c < kColsInFlight; ++c) {
+            const AccT xj = (AccT)x[j + c];
+#pragma unroll
+            for (int e = 0; e < W; ++e) s[e] += up<AccT>(r[c].v[e]) * xj;
+        }
+    }
+    for (; j < j1; ++j, a += lda) {
+        const Run<V, W> r = load_run<V, W>(a);
+        const AccT xj = (AccT)x[j];
+#pragma unroll
+        for (int e = 0; e < W; ++e) s[e] += up<AccT>(r.v[e]) * xj;
+    }
+    if (wave > 0) {
+#pragma unroll
+        for (int e = 0; e < W; ++e) sh[wave - 1][e * 64 + lane] = s[e];
+    }
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int e = 0; e < W; ++e) {
+        const AccT t = (s[e] + sh[0][e * 64 + lane]) + (sh[1][e * 64 + lane] + sh[2][e * 64 + lane]);
+        if (gridDim.y == 1) y[i + e] = (T)t;
+        else part[(int64_t)blockIdx.y * m + i + e] = t;
+    }
 }
 
+// y = sum of the ks slab partials: 64 rows a workgroup, its wavefronts each a
+// quarter of the slabs (one thread summing all slabs of a row was a chain of
+// up to 128 dependent loads).
 template <typename T, typename AccT>
-__global__ void k_gemv_n_sum(int64_t m, int ks, const AccT *part, T *y) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
+__global__ __launch_bounds__(256) void k_gemv_n_sum(int64_t m, int ks,
+                                                    const AccT *__restrict__ part,
+                                                    T *__restrict__ y) {
+    __shared__ AccT sh[3][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t i = min((int64_t)blockIdx.x * 64 + lane, m - 1);
     AccT s = 0;
-    for (int k = 0; k < ks; ++k) s += part[(int64_t)k * m + i];
-    y[i] = (T)s;
+    int k = wave;
+    for (; k + 28 < ks; k += 32) {
+        AccT v[8];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) v[c] = part[(int64_t)(k + 4 * c) * m + i];
+        s += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+    }
+    for (; k < ks; k += 4) s += part[(int64_t)k * m + i];
+    if (wave > 0) sh[wave - 1][lane] = s;
+    __syncthreads();
+    if (wave == 0) y[i] = (T)((s + sh[0][lane]) + (sh[1][lane] + sh[2][lane]));
 }
 
-template <typename V, typename T, typename AccT>
+template <typename V, int W, int C, typename T, typename AccT>
 __global__ __launch_bounds__(256) void k_gemv_t(int64_t m, int64_t n, int64_t lda,
                                                 const V *__restrict__ A,
                                                 const T *__restrict__ x, T *__restrict__ y) {
-    int64_t j = ((int64_t)blockIdx.x * 256 + threadIdx.x) / 64;
-    int lane = threadIdx.x & 63;
-    if (j >= n) return;
-    const V *col = A + j * lda;
-    AccT s = 0;
-    for (int64_t i = lane; i < m; i += 64) s += loadA<V, AccT>(col, i) * (AccT)x[i];
+    const int lane = threadIdx.x & 63;
+    const int64_t j0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * C;
+    if (j0 >= n) return;
+    const V *col[C];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    if (lane == 0) y[j] = (T)s;
+    for (int c = 0; c < C; ++c) col[c] = A + min(j0 + c, n - 1) * lda;
+    AccT s[C] = {}, s2[C] = {};
+    auto add = [&](const Run<V, W> &r, const Run<T, W> &xv, AccT &sum) {
+        AccT p = 0;
+#pragma unroll
+        for (int e = 0; e < W; ++e) p += up<AccT>(r.v[e]) * (AccT)xv.v[e];
+        sum += p;
+    };
+    const int64_t step = 64 * W, whole = m / step * step;
+    int64_t i = (int64_t)lane * W;
+    for (; i + step < whole; i += 2 * step) {
+        Run<V, W> r[C], r2[C];
+        const Run<T, W> xv = load_run<T, W>(x + i), xv2 = load_run<T, W>(x + i + step);
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            r[c] = load_run<V, W>(col[c] + i);
+            r2[c] = load_run<V, W>(col[c] + i + step);
+        }
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            add(r[c], xv, s[c]);
+            add(r2[c], xv2, s2[c]);
+        }
+    }
+    for (; i + W <= m; i += step) {
+        const Run<T, W> xv = load_run<T, W>(x + i);
+#pragma unroll
+        for (int c = 0; c < C; ++c) add(load_run<V, W>(col[c] + i), xv, s[c]);
+    }
+    // the rows after the last whole run: one a lane
+    const int64_t tail = m / W * W + lane;
+    if (tail < m) {
+        const AccT xv = (AccT)x[tail];
+#pragma unroll
+        for (int c = 0; c < C; ++c) s2[c] += up<AccT>(col[c][tail]) * xv;
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const AccT t = lane_sum<64>(s[c] + s2[c]);
+        if (lane == 0 && j0 + c < n) y[j0 + c] = (T)t;
+    }
 }
+
+}  // namespace
 
 // ws: the split-K partials of A x go to this workspace of ws_bytes (the
 // allocation-free path) instead of the context's, which grows on demand
+template <typename V, int W, typename T, typename AccT>
+static void gemv_n(tv3_op *op, const T *x, T *y, hipStream_t s, void *ws, size_t ws_bytes) {
+    const V *A = reinterpret_cast<const V *>(op->dense.p);
+    const int64_t m = op->m, n = op->n, lda = op->lda;
+    // the workspace a caller provides is checked for min(128, ceil(n / 64))
+    // slabs; the launch uses no more than those
+    int64_t slabs = std::min<int64_t>(128, (n + 63) / 64);
+    slabs = (n + (n + slabs - 1) / slabs - 1) / ((n + slabs - 1) / slabs);
+    const size_t need = sizeof(AccT) * (size_t)slabs * (size_t)m;
+    if (ws)
+        TV3_REQUIRE(need <= ws_bytes, TV3_E_UNSUPPORTED,
+                    "dense A x needs " + std::to_string(need) + " bytes of partial sums; the "
+                    "allocation-free path holds " + std::to_string(ws_bytes));
+    // enough workgroups for four a CU, as far as the columns go
+    const int64_t tiles = (m + 64 * W - 1) / (64 * W);
+    int64_t ks = std::min(slabs, std::max<int64_t>(1, (4 * op->ctx->num_cus + tiles - 1) / tiles));
+    const int64_t cols_per = (n + ks - 1) / ks;
+    ks = (n + cols_per - 1) / cols_per;
+    AccT *part = reinterpret_cast<AccT *>(ws);
+    if (!ws && ks > 1) {
+        if (op->ctx->scratch.bytes() < need) op->ctx->scratch.alloc(need);
+        part = reinterpret_cast<AccT *>(op->ctx->scratch.p);
+    }
+    hipLaunchKernelGGL((k_gemv_n_part<V, W, T, AccT>), dim3((unsigned)tiles, (unsigned)ks),
+                       dim3(256), 0, s, m, n, lda, A, x, part, y, cols_per);
+    if (ks > 1)
+        hipLaunchKernelGGL((k_gemv_n_sum<T, AccT>), dim3((unsigned)((m + 63) / 64)), dim3(256), 0,
+                           s, m, (int)ks, part, y);
+}
+
+template <typename V, int C, typename T, typename AccT>
+static void gemv_t(tv3_op *op, const T *x, T *y, hipStream_t s) {
+    constexpr int W = run_of<V>();
+    hipLaunchKernelGGL((k_gemv_t<V, W, C, T, AccT>), dim3((unsigned)((op->n + 4 * C - 1) / (4 * C))),
+                       dim3(256), 0, s, op->m, op->n, op->lda,
+                       reinterpret_cast<const V *>(op->dense.p), x, y);
+}
+
 template <typename V, typename T, typename AccT>
 static void gemv(tv3_op *op, bool trans, const T *x, T *y, hipStream_t s, void *ws = nullptr,
                  size_t ws_bytes = 0) {
-    const V *A = reinterpret_cast<const V *>(op->dense.p);
-    int64_t m = op->m, n = op->n, lda = op->lda;
+    constexpr int W = run_of<V>();
     if (!trans) {
-        int ks = (int)((n + 63) / 64);
-        if (ks > 128) ks = 128;
-        if (ks < 1) ks = 1;
-        int64_t cols_per = (n + ks - 1) / ks;
-        ks = (int)((n + cols_per - 1) / cols_per);
-        size_t need = sizeof(AccT) * (size_t)ks * (size_t)m;
-        AccT *part;
-        if (ws) {
-            TV3_REQUIRE(need <= ws_bytes, TV3_E_UNSUPPORTED,
-                        "dense A x needs " + std::to_string(need) + " bytes of partial sums; the "
-                        "allocation-free path holds " + std::to_string(ws_bytes));
-            part = reinterpret_cast<AccT *>(ws);
-        } else {
-            if (op->ctx->scratch.bytes() < need) op->ctx->scratch.alloc(need);
-            part = reinterpret_cast<AccT *>(op->ctx->scratch.p);
-        }
-        hipLaunchKernelGGL((k_gemv_n_part<V, T, AccT>), dim3((unsigned)((m + 255) / 256), ks), dim3(256),
-                           0, s, m, n, lda, A, x, part, cols_per);
-        hipLaunchKernelGGL((k_gemv_n_sum<T, AccT>), dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, m,
-                           ks, part, y);
+        if (op->m >= W) gemv_n<V, W, T, AccT>(op, x, y, s, ws, ws_bytes);
+        else gemv_n<V, 1, T, AccT>(op, x, y, s, ws, ws_bytes);
     } else {
-        hipLaunchKernelGGL((k_gemv_t<V, T, AccT>), dim3((unsigned)((n * 64 + 255) / 256)), dim3(256), 0,
-                           s, m, n, lda, A, x, y);
+        // columns per wavefront: as many as leave eight wavefronts a CU
+        const int64_t waves = 8 * (int64_t)op->ctx->num_cus;
+        if (op->n >= 4 * waves) gemv_t<V, 4, T, AccT>(op, x, y, s);
+        else if (op->n >= 2 * waves) gemv_t<V, 2, T, AccT>(op, x, y, s);
+        else gemv_t<V, 1, T, AccT>(op, x, y, s);
     }
     TV3_HIP(hipGetLastError());
 }
