@@ -15,32 +15,31 @@
 //
 // FP32 products of a Siddon operator whose dimensions are multiples of 4
 // run as tile products (dyntile.hip, panels.hpp: deterministic, no
-// atomics).  The others -- Bresenham, FP64, other shapes -- run here: one
-// thread walks one ray; N gathers x along the ray (x stays resident in L2 /
-// MALL) and writes y[ray] once; T scatters x[ray]*w into y with FP32
-// hardware atomics (no replicated sub-volumes).  The same walk, with FP
+// atomics).  The others -- Bresenham, FP64, other shapes -- run here.  N: one
+// thread walks one ray and gathers x along it, several gathers in flight.  T:
+// the rays' parts inside boxes of 16 x 8 x 8 voxels, listed on the device at
+// creation (RayBoxes), add into the box in LDS; nothing is scattered to
+// memory.  Neither keeps scratch between calls.  A Bresenham operator with
+// transducers outside the grid keeps the clamping per-ray kernels.  The same
+// walk, with FP
 // contraction disabled, fills the CSR in dynamic_materialize so a
 // precomputed matrix holds exactly the weights the dynamic product uses.
-#include "siddon.hpp"
-#include "tv3_internal.hpp"
-
+#include <algorithm>
 #include <cmath>
+#include <numeric>
+
+#include "panels.hpp"
 
 namespace tv3 {
 
 __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
-// Bresenham walk; emit(linear voxel index) for each visited voxel.
+// Bresenham walk; emit(x, y, z) for each visited voxel (not clamped).
 template <typename F>
-__device__ __forceinline__ void bresenham_walk(int x0, int y0, int z0, int x1, int y1, int z1,
-                                               int rvx, int rvy, int rvz, F emit) {
+__device__ __forceinline__ void bresenham_steps(int x0, int y0, int z0, int x1, int y1, int z1,
+                                                F emit) {
     int c[3] = {x0, y0, z0};
-    auto visit = [&]() {
-        int xx = clampi(c[0], 0, rvx - 1), yy = clampi(c[1], 0, rvy - 1),
-            zz = clampi(c[2], 0, rvz - 1);
-        emit((int64_t)zz * rvx * rvy + (int64_t)xx * rvy + yy);
-    };
-    visit();
+    emit(c[0], c[1], c[2]);
     int d1 = x1 - x0, d2 = y1 - y0, d3 = z1 - z0;
     int m1 = abs(d1), m2 = abs(d2), m3 = abs(d3);
     int a1, a2, a3;
@@ -61,9 +60,61 @@ __device__ __forceinline__ void bresenham_walk(int x0, int y0, int z0, int x1, i
         if (e2 > 0) { c[a3] += inc3; e2 -= 2 * m1; }
         e1 += 2 * m2; e2 += 2 * m3;
         c[a1] += inc1;
-        visit();
+        emit(c[0], c[1], c[2]);
     }
 }
+
+// The walk clamped into the grid; emit(linear voxel index).
+template <typename F>
+__device__ __forceinline__ void bresenham_walk(int x0, int y0, int z0, int x1, int y1, int z1,
+                                               int rvx, int rvy, int rvz, F emit) {
+    bresenham_steps(x0, y0, z0, x1, y1, z1, [&](int x, int y, int z) {
+        emit((int64_t)clampi(z, 0, rvz - 1) * rvx * rvy + (int64_t)clampi(x, 0, rvx - 1) * rvy +
+             clampi(y, 0, rvy - 1));
+    });
+}
+
+// A Bresenham walk that can start at any step (transducers inside the grid).
+// After j steps the leading axis has moved j voxels and a slower one, with
+// differences m along it and M along the leading axis, floor((2 m j + M - 1)
+// / (2 M)): its error term passes 0 that often.  off advances by the strides
+// the caller gives; with all coordinates below 2^15 every term fits 32 bits.
+struct BresWalk {
+    int off, s1, s2, s3;     // offset, signed strides along the leading and slower axes
+    int e1, e2, d1, d2, dm;  // error terms, 2 m2, 2 m3, 2 M
+    int x, y, z, steps;      // voxel at the start; steps of the whole walk
+    __device__ __forceinline__ BresWalk(const int4 w, int j0, int sx, int sy, int sz) {
+        const int dx = w.y >> 16, dy = (int)(int16_t)w.z, dz = w.z >> 16;
+        const int mx = abs(dx), my = abs(dy), mz = abs(dz);
+        const int ix = dx < 0 ? -1 : 1, iy = dy < 0 ? -1 : 1, iz = dz < 0 ? -1 : 1;
+        const int lead = mx >= my && mx >= mz ? 0 : (my >= mx && my >= mz ? 1 : 2);
+        const int M = lead == 0 ? mx : (lead == 1 ? my : mz);
+        const int m2 = lead == 0 ? my : mx, m3 = lead == 2 ? my : mz;
+        d1 = 2 * m2; d2 = 2 * m3; dm = 2 * M;
+        int k2 = 0, k3 = 0;
+        if (j0 > 0) {        // then M > 0
+            k2 = (int)((unsigned)(d1 * j0 + M - 1) / (unsigned)dm);
+            k3 = (int)((unsigned)(d2 * j0 + M - 1) / (unsigned)dm);
+        }
+        e1 = d1 * (j0 + 1) - M - dm * k2;
+        e2 = d2 * (j0 + 1) - M - dm * k3;
+        x = (int)(int16_t)w.x + ix * (lead == 0 ? j0 : k2);
+        y = (w.x >> 16) + iy * (lead == 1 ? j0 : (lead == 0 ? k2 : k3));
+        z = (int)(int16_t)w.y + iz * (lead == 2 ? j0 : k3);
+        sx *= ix; sy *= iy; sz *= iz;
+        s1 = lead == 0 ? sx : (lead == 1 ? sy : sz);
+        s2 = lead == 0 ? sy : sx;
+        s3 = lead == 2 ? sy : sz;
+        off = 0;
+        steps = M + 1;
+    }
+    __device__ __forceinline__ void next() {
+        const bool a = e1 > 0, b = e2 > 0;
+        off += s1 + (a ? s2 : 0) + (b ? s3 : 0);
+        e1 += d1 - (a ? dm : 0);
+        e2 += d2 - (b ? dm : 0);
+    }
+};
 
 // Siddon traversal of p0->p1 through [org, org + N*h] (siddon.hpp);
 // emit(linear voxel index, length) in traversal order.
@@ -98,6 +149,13 @@ static GeoView view(const DynGeom &g) {
     return v;
 }
 
+// Boxes of the A^T product (RayBoxes) and its workgroup.  Measured, Bresenham
+// at 128^3 and Siddon at 77 x 101 x 90 (us): 16 x 8 x 8 voxels, 512 threads,
+// items of at most 8192 segments 44, 27; 4096 segments 51, 27; 256 threads
+// and 4096 52, 28; 8^3 voxels 55, 25; 16^3 voxels 60-67, 34-44.
+constexpr int kRayBoxY = 16, kRayBoxXZ = 8, kBoxThreads = 512;
+constexpr int kBoxSegs = 8192, kLenClasses = 16;
+
 template <typename R>
 __device__ __forceinline__ void ray_ends(const GeoView &g, int64_t k, R p0[3], R p1[3]) {
     int e = g.path[2 * k], r = g.path[2 * k + 1];
@@ -105,30 +163,202 @@ __device__ __forceinline__ void ray_ends(const GeoView &g, int64_t k, R p0[3], R
     for (int a = 0; a < 3; ++a) { p0[a] = (R)g.ep[3 * e + a]; p1[a] = (R)g.rp[3 * r + a]; }
 }
 
-// The Siddon operator is the FP32 traversal: FP64 products accumulate its
-// weights in FP64 (the same matrix in both precisions).
+// N of a Bresenham operator with every transducer in the grid: a thread owns
+// a ray (in bundles of neighbours, so the lanes of a wavefront gather near
+// each other) and gathers eight voxels at a time; one at a time, each step
+// waited for its gather.  At 128^3 with 262,144 rays 206 -> 77 us, now bound
+// by the gathers' cache lines (4 to 32 at a time, bundles of 4^2 to 32^2 rays
+// and workgroups of 64 to 1024 threads all take 77-79 us).
 template <typename T, typename AccT>
-__global__ __launch_bounds__(256) void k_dyn_N(GeoView g, int siddon, const T *__restrict__ x,
-                                               T *__restrict__ y) {
-    int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (k >= g.P) return;
+__global__ __launch_bounds__(64) void k_bres_N(GeoView g, const int32_t *__restrict__ bundle,
+                                               const int4 *__restrict__ walk,
+                                               const T *__restrict__ x, T *__restrict__ y) {
+    const int64_t i = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * 64 + threadIdx.x;
+    if (i >= g.P) return;
+    const int64_t k = bundle ? bundle[i] : i;
+    BresWalk w(walk[k], 0, g.rvy, 1, g.rvx * g.rvy);
+    w.off = (w.z * g.rvx + w.x) * g.rvy + w.y;
+    const AccT wt = (AccT)(T)g.scale;
     AccT acc = 0;
-    if (siddon) {
-        float p0[3], p1[3];
-        int N[3] = {g.rvx, g.rvy, g.rvz};
-        ray_ends<float>(g, k, p0, p1);
-        siddon_walk<float>(p0, p1, g.org, g.h, N, g.rvy,
-                           [&](int64_t v, float w) { acc += (AccT)w * (AccT)x[v]; });
-    } else {
-        int e = g.path[2 * k], r = g.path[2 * k + 1];
-        T w = (T)g.scale;
-        bresenham_walk(g.ec[3 * e], g.ec[3 * e + 1], g.ec[3 * e + 2], g.rc[3 * r], g.rc[3 * r + 1],
-                       g.rc[3 * r + 2], g.rvx, g.rvy, g.rvz,
-                       [&](int64_t v) { acc += (AccT)x[v] * (AccT)w; });
+    for (int j = 0; j < w.steps; j += 8) {
+        T v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            v[u] = x[w.off];
+            if (j + u + 1 < w.steps) w.next();   // stays at the receiver's voxel
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (j + u < w.steps) acc += (AccT)v[u] * wt;
     }
     y[k] = (T)acc;
 }
 
+// N of a Siddon operator likewise: sid_walk's steps with eight gathers at a
+// time (77 x 101 x 90 voxels, 90,150 rays: 73 -> 32 us).  The Siddon operator is the FP32 traversal: FP64 products accumulate
+// its weights in FP64 (the same matrix in both precisions).
+template <typename T, typename AccT>
+__global__ __launch_bounds__(64) void k_sid_N(GeoView g, const int32_t *__restrict__ bundle,
+                                              const T *__restrict__ x, T *__restrict__ y) {
+#pragma clang fp contract(off)
+    const int64_t i = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * 64 + threadIdx.x;
+    if (i >= g.P) return;
+    const int64_t k = bundle ? bundle[i] : i;
+    float p0[3], p1[3];
+    const int N[3] = {g.rvx, g.rvy, g.rvz};
+    const int64_t stride[3] = {g.rvy, 1, (int64_t)g.rvx * g.rvy};
+    ray_ends<float>(g, k, p0, p1);
+    SidRay<float> s;
+    sid_setup(s, p0, p1, g.org, g.h, N);
+    AccT acc = 0;
+    if (s.hit) {
+        // next plane (as a float) and its parameter per axis; a plane beyond
+        // the grid lies at or beyond amax, so it is never taken
+        float kf[3], tk[3], st[3], tcur = s.amin;
+        int64_t step[3], off = 0;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const bool par = s.st[a] == 0;
+            const int kn = par ? 0 : sid_next_plane(s, a, s.amin);
+            const int c = par ? s.cfix[a] : (s.st[a] > 0 ? kn - 1 : kn);
+            kf[a] = (float)kn;
+            st[a] = (float)s.st[a];
+            tk[a] = par ? INFINITY : sid_fma(kf[a], s.A[a], s.B[a]);
+            step[a] = s.st[a] * stride[a];
+            off += c * stride[a];
+        }
+        bool on = true;
+        for (int left = N[0] + N[1] + N[2] + 4; on && left > 0; left -= 8) {
+            float w[8];
+            T v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                float tnext = s.amax;
+#pragma unroll
+                for (int a = 0; a < 3; ++a) tnext = tk[a] < tnext ? tk[a] : tnext;
+                w[u] = on ? (tnext - tcur) * s.L : 0.f;
+                v[u] = x[off];
+                on = on && tnext < s.amax;
+#pragma unroll
+                for (int a = 0; a < 3; ++a) {
+                    const bool m = on && tk[a] == tnext;
+                    kf[a] += m ? st[a] : 0.f;
+                    off += m ? step[a] : 0;
+                    tk[a] = m ? sid_fma(kf[a], s.A[a], s.B[a]) : tk[a];
+                }
+                tcur = on ? tnext : tcur;
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (w[u] > 0) acc = fma((AccT)w[u], (AccT)v[u], acc);
+        }
+    }
+    y[k] = (T)acc;
+}
+
+// T from the rays' parts inside boxes: a workgroup adds the parts of one work
+// item into the box in LDS, then writes the box (a box with several items:
+// adds it to a cleared y, whole lines at a time).  The sums are FP64 for FP32
+// vectors too: an LDS FP64 add serves a wavefront in 22 clocks, an FP32 add
+// in 196 (measured, random addresses), which at first bound the kernel: 134
+// us at 128^3 with 262,144 Bresenham rays against 44 us now (1025 us with one
+// memory atomic per entry).  Parts of equal length are neighbours in the
+// list, so the lanes of a wavefront end together.
+template <bool SID, typename T>
+__global__ __launch_bounds__(kBoxThreads) void k_box_T(GeoView g, int nby, int nbx,
+                                                       const int4 *__restrict__ items,
+                                                       const uint2 *__restrict__ seg,
+                                                       const int4 *__restrict__ walk,
+                                                       const float *__restrict__ rec,
+                                                       const T *__restrict__ x,
+                                                       T *__restrict__ y) {
+    constexpr int NV = kRayBoxY * kRayBoxXZ * kRayBoxXZ, NT = kBoxThreads;
+    __shared__ double box[NV];
+    const int4 it = items[blockIdx.x];
+    const int t = threadIdx.x;
+    DynPan P = {};
+    P.by = it.x % nby * kRayBoxY;
+    P.bx = it.x / nby % nbx * kRayBoxXZ;
+    P.bz = it.x / nby / nbx * kRayBoxXZ;
+    P.bs = kRayBoxXZ;
+    P.ey = kRayBoxY;
+    for (int i = t; i < NV; i += NT) box[i] = 0;
+    __syncthreads();
+    // a part needs two loads in turn, its segment and then its ray's record
+    // and value: segments are requested two parts ahead, records one
+    struct Part {
+        uint2 sg;
+        T xr;
+        int4 w;            // Bresenham
+        float4 ra, rb;     // Siddon
+        float amax;
+    };
+    auto segment = [&](int k) { return seg[min(k, it.z - 1)]; };
+    auto fetch = [&](uint2 sg) {
+        Part p = {};
+        p.sg = sg;
+        p.xr = x[sg.x];
+        if constexpr (SID) {
+            const float4 *q = reinterpret_cast<const float4 *>(rec + 12 * (int64_t)sg.x);
+            p.ra = q[0];
+            p.rb = q[1];
+            p.amax = q[2].x;
+        } else {
+            p.w = walk[sg.x];
+        }
+        return p;
+    };
+    int k = it.y + t;
+    if (k < it.z) {
+        Part cur = fetch(segment(k));
+        uint2 ahead = segment(k + NT);
+        for (; k < it.z; k += NT) {
+            const Part nxt = fetch(ahead);
+            ahead = segment(k + 2 * NT);
+            if (cur.xr != 0) {
+                if constexpr (SID) {
+                    dyn_seg_walk(DynSeg{cur.ra, cur.rb, cur.amax, (int)cur.sg.y}, P,
+                                 [&](int i, float w) { atomicAdd(&box[i], (double)((T)w * cur.xr)); });
+                } else {
+                    const double v = (double)(cur.xr * (T)g.scale);
+                    BresWalk w(cur.w, cur.sg.y & 0xffff, kRayBoxY, 1, kRayBoxY * kRayBoxXZ);
+                    w.off = (w.y - P.by) + kRayBoxY * ((w.x - P.bx) + kRayBoxXZ * (w.z - P.bz));
+                    for (int j = cur.sg.y >> 16; j > 0; --j) {
+                        atomicAdd(&box[w.off & (NV - 1)], v);
+                        w.next();
+                    }
+                }
+            }
+            cur = nxt;
+        }
+    }
+    __syncthreads();
+    for (int i = t; i < NV; i += NT) {
+        const int yy = P.by + (i & (kRayBoxY - 1)), xx = P.bx + i / kRayBoxY % kRayBoxXZ,
+                  zz = P.bz + i / (kRayBoxY * kRayBoxXZ);
+        if (yy >= g.rvy || xx >= g.rvx || zz >= g.rvz) continue;
+        const int64_t o = ((int64_t)zz * g.rvx + xx) * g.rvy + yy;
+        if (it.w) atomicAdd(&y[o], (T)box[i]);
+        else y[o] = (T)box[i];
+    }
+}
+
+// Bresenham with transducers outside the grid (coordinates clamped)
+template <typename T, typename AccT>
+__global__ __launch_bounds__(256) void k_clamped_N(GeoView g, const T *__restrict__ x,
+                                                   T *__restrict__ y) {
+    int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (k >= g.P) return;
+    AccT acc = 0;
+    int e = g.path[2 * k], r = g.path[2 * k + 1];
+    T w = (T)g.scale;
+    bresenham_walk(g.ec[3 * e], g.ec[3 * e + 1], g.ec[3 * e + 2], g.rc[3 * r], g.rc[3 * r + 1],
+                   g.rc[3 * r + 2], g.rvx, g.rvy, g.rvz,
+                   [&](int64_t v) { acc += (AccT)x[v] * (AccT)w; });
+    y[k] = (T)acc;
+}
+
+// T per ray: FP32 (FP64) hardware atomics on y
 template <typename T>
 __global__ __launch_bounds__(256) void k_dyn_T(GeoView g, int siddon, const T *__restrict__ x,
                                                T *__restrict__ y) {
@@ -150,16 +380,43 @@ __global__ __launch_bounds__(256) void k_dyn_T(GeoView g, int siddon, const T *_
     }
 }
 
+template <typename T>
+__global__ void k_clear(int64_t n, T *y) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) y[i] = 0;
+}
+
+static int boxes_along(int n, int edge) { return (n + edge - 1) / edge; }
+
 template <typename T, typename AccT>
 static void dyn_apply(tv3_op *op, bool trans, const T *x, T *y, hipStream_t s) {
-    GeoView g = view(op->geo);
-    int sid = op->geo.mode == TV3_WEIGHT_SIDDON;
-    unsigned blocks = (unsigned)((g.P + 255) / 256);
+    const DynGeom &G = op->geo;
+    const GeoView g = view(G);
+    const int sid = G.mode == TV3_WEIGHT_SIDDON;
+    const unsigned rays64 = (unsigned)((g.P + 63) / 64), rays256 = (unsigned)((g.P + 255) / 256);
     if (!trans) {
-        if (blocks) hipLaunchKernelGGL((k_dyn_N<T, AccT>), dim3(blocks), dim3(256), 0, s, g, sid, x, y);
+        if (sid)
+            hipLaunchKernelGGL((k_sid_N<T, AccT>), dim3(rays64), dim3(64), 0, s, g, G.bundle.p, x,
+                               y);
+        else if (G.inside)
+            hipLaunchKernelGGL((k_bres_N<T, AccT>), dim3(rays64), dim3(64), 0, s, g, G.bundle.p,
+                               G.walk.p, x, y);
+        else
+            hipLaunchKernelGGL((k_clamped_N<T, AccT>), dim3(rays256), dim3(256), 0, s, g, x, y);
     } else {
-        TV3_HIP(hipMemsetAsync(y, 0, sizeof(T) * op->n, s));
-        if (blocks) hipLaunchKernelGGL((k_dyn_T<T>), dim3(blocks), dim3(256), 0, s, g, sid, x, y);
+        if (G.boxes.nitem == 0 || G.boxes.split)
+            hipLaunchKernelGGL(k_clear<T>, dim3((unsigned)((op->n + 255) / 256)), dim3(256), 0, s,
+                               op->n, y);
+        const dim3 items((unsigned)G.boxes.nitem);
+        const int nby = boxes_along(g.rvy, kRayBoxY), nbx = boxes_along(g.rvx, kRayBoxXZ);
+        if (G.boxes.nitem && sid)
+            hipLaunchKernelGGL((k_box_T<true, T>), items, dim3(kBoxThreads), 0, s, g, nby, nbx,
+                               G.boxes.item.p, G.boxes.seg.p, G.walk.p, G.rec.p, x, y);
+        else if (G.boxes.nitem)
+            hipLaunchKernelGGL((k_box_T<false, T>), items, dim3(kBoxThreads), 0, s, g, nby, nbx,
+                               G.boxes.item.p, G.boxes.seg.p, G.walk.p, G.rec.p, x, y);
+        else
+            hipLaunchKernelGGL((k_dyn_T<T>), dim3(rays256), dim3(256), 0, s, g, sid, x, y);
     }
     TV3_HIP(hipGetLastError());
 }
@@ -171,6 +428,161 @@ void dynamic_apply(tv3_op *op, bool trans, const float *x, float *y, hipStream_t
 }
 void dynamic_apply(tv3_op *op, bool trans, const double *x, double *y, hipStream_t s, bool) {
     dyn_apply<double, double>(op, trans, x, y, s);
+}
+
+// ------------------------------------------------------------- ray boxes
+// Per ray: the walk's record (Bresenham) or the traversal's (Siddon).
+__global__ __launch_bounds__(256) void k_ray_records(GeoView g, int siddon, int4 *walk,
+                                                     float *rec) {
+    const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (k >= g.P) return;
+    if (siddon) {
+        float p0[3], p1[3];
+        const int N[3] = {g.rvx, g.rvy, g.rvz};
+        ray_ends<float>(g, k, p0, p1);
+        SidRay<float> s;
+        sid_setup(s, p0, p1, g.org, g.h, N);
+        float4 *o = reinterpret_cast<float4 *>(rec + 12 * k);
+        o[0] = make_float4(s.A[0], s.A[1], s.A[2], s.L);
+        o[1] = make_float4(s.B[0], s.B[1], s.B[2], s.amin);
+        o[2] = make_float4(s.amax, 0.f, 0.f, 0.f);
+    } else {
+        const int32_t *a = g.ec + 3 * (int64_t)g.path[2 * k], *b = g.rc + 3 * (int64_t)g.path[2 * k + 1];
+        auto two = [](int lo, int hi) { return (int)((unsigned)(lo & 0xffff) | (unsigned)hi << 16); };
+        walk[k] = make_int4(two(a[0], a[1]), two(a[2], b[0] - a[0]), two(b[1] - a[1], b[2] - a[2]),
+                            0);
+    }
+}
+
+// Every ray's walk cut at box faces (a box is convex: one part per ray and
+// box).  FILL = false: counts the parts; FILL = true: cnt holds the next free
+// segment.  A box has a counter for each of kLenClasses lengths, longest
+// first (Siddon, whose parts are longer, in steps of two).
+template <bool FILL>
+__global__ __launch_bounds__(64) void k_box_parts(GeoView g, int siddon,
+                                                  const int32_t *__restrict__ bundle, int nby,
+                                                  int nbx, int32_t *cnt, uint2 *seg) {
+    const int64_t i = (int64_t)blockIdx.x * 64 + threadIdx.x;
+    if (i >= g.P) return;
+    const int64_t k = bundle ? bundle[i] : i;
+    int cur = -1, j = 0;
+    unsigned first = 0;
+    auto close = [&]() {
+        if (cur < 0) return;
+        const int len = siddon ? j >> 1 : j - (int)first;
+        const int cls = max(kLenClasses - 1 - len, 0);
+        const int at = atomicAdd(&cnt[(int64_t)cur * kLenClasses + cls], 1);
+        if (FILL)
+            seg[at] = make_uint2((unsigned)k, siddon ? first : first | (unsigned)len << 16);
+    };
+    auto visit = [&](int x, int y, int z) {
+        const int b = (z / kRayBoxXZ * nbx + x / kRayBoxXZ) * nby + y / kRayBoxY;
+        if (b != cur) {
+            close();
+            cur = b;
+            if (siddon) {
+                first = (unsigned)(x % kRayBoxXZ | y % kRayBoxY << 4 | z % kRayBoxXZ << 8);
+                j = 0;
+            } else {
+                first = (unsigned)j;
+            }
+        }
+        ++j;
+    };
+    if (siddon) {
+        float p0[3], p1[3];
+        const int N[3] = {g.rvx, g.rvy, g.rvz};
+        ray_ends<float>(g, k, p0, p1);
+        SidRay<float> s;
+        sid_setup(s, p0, p1, g.org, g.h, N);
+        if (s.hit)
+            sid_walk(s, s.amin, s.amax, [&](int x, int y, int z, float) { visit(x, y, z); });
+    } else {
+        const int32_t *a = g.ec + 3 * (int64_t)g.path[2 * k], *b = g.rc + 3 * (int64_t)g.path[2 * k + 1];
+        bresenham_steps(a[0], a[1], a[2], b[0], b[1], b[2], visit);
+    }
+    close();
+}
+
+// the boxes' segments and work items
+static void build_ray_boxes(tv3_ctx *ctx, DynGeom &G) {
+    hipStream_t s = ctx->stream;
+    const GeoView g = view(G);
+    const int sid = G.mode == TV3_WEIGHT_SIDDON;
+    const unsigned rays64 = (unsigned)((g.P + 63) / 64);
+    const int nby = boxes_along(g.rvy, kRayBoxY), nbx = boxes_along(g.rvx, kRayBoxXZ);
+    const int64_t nbox = (int64_t)nby * nbx * boxes_along(g.rvz, kRayBoxXZ);
+    const int64_t ncnt = nbox * kLenClasses;
+    DevBuf<int32_t> cnt(ncnt), ptr(ncnt + 1);
+    TV3_HIP(hipMemsetAsync(cnt.p, 0, cnt.bytes(), s));
+    hipLaunchKernelGGL(k_box_parts<false>, dim3(rays64), dim3(64), 0, s, g, sid, G.bundle.p, nby,
+                       nbx, cnt.p, (uint2 *)nullptr);
+    const int64_t nseg = exclusive_scan_i32(ctx, cnt.p, ptr.p, ncnt);
+    G.boxes.seg.alloc(nseg > 0 ? nseg : 1);
+    TV3_HIP(hipMemcpyAsync(cnt.p, ptr.p, sizeof(int32_t) * ncnt, hipMemcpyDeviceToDevice, s));
+    hipLaunchKernelGGL(k_box_parts<true>, dim3(rays64), dim3(64), 0, s, g, sid, G.bundle.p, nby,
+                       nbx, cnt.p, G.boxes.seg.p);
+    std::vector<int32_t> q(ncnt + 1), p(nbox + 1);
+    TV3_HIP(hipMemcpyAsync(q.data(), ptr.p, sizeof(int32_t) * (ncnt + 1), hipMemcpyDeviceToHost, s));
+    TV3_HIP(hipStreamSynchronize(s));
+    for (int64_t b = 0; b <= nbox; ++b) p[b] = q[b * kLenClasses];
+    std::vector<int4> items;
+    for (int64_t b = 0; b < nbox; ++b) {
+        const int32_t c = p[b + 1] - p[b], k = std::max(1, (c + kBoxSegs - 1) / kBoxSegs);
+        for (int32_t i = 0; i < k; ++i)
+            items.push_back(int4{(int)b, (int)(p[b] + (int64_t)c * i / k),
+                                 (int)(p[b] + (int64_t)c * (i + 1) / k), k > 1});
+        G.boxes.split = G.boxes.split || k > 1;
+    }
+    std::stable_sort(items.begin(), items.end(),
+                     [](const int4 &a, const int4 &b) { return a.z - a.y > b.z - b.y; });
+    G.boxes.item.alloc(items.size());
+    TV3_HIP(hipMemcpyAsync(G.boxes.item.p, items.data(), sizeof(int4) * items.size(),
+                           hipMemcpyHostToDevice, s));
+    TV3_HIP(hipStreamSynchronize(s));
+    G.boxes.nitem = (int64_t)items.size();
+}
+
+void dynamic_prepare(tv3_op *op, bool boxes) {
+    DynGeom &G = op->geo;
+    tv3_ctx *ctx = op->ctx;
+    hipStream_t s = ctx->stream;
+    const int sid = G.mode == TV3_WEIGHT_SIDDON;
+    // 8 x 8 transducers: the lanes of one wavefront
+    const std::vector<int32_t> bundle = ray_bundles(G, 8);
+    if (!bundle.empty()) {
+        G.bundle.alloc(bundle.size());
+        TV3_HIP(hipMemcpyAsync(G.bundle.p, bundle.data(), sizeof(int32_t) * bundle.size(),
+                               hipMemcpyHostToDevice, s));
+    }
+    if (!sid) {
+        // epos_h / rpos_h hold the voxel coordinates
+        const int lim[3] = {G.rv_x, G.rv_y, G.rv_z};
+        G.inside = std::max({G.rv_x, G.rv_y, G.rv_z}) < 32768 && op->n < (int64_t(1) << 31);
+        for (const std::vector<float> *c : {&G.epos_h, &G.rpos_h})
+            for (size_t k = 0; k < c->size(); ++k)
+                G.inside = G.inside && (*c)[k] >= 0 && (*c)[k] < lim[k % 3];
+    }
+    const GeoView g = view(G);
+    const unsigned rays256 = (unsigned)((g.P + 255) / 256);
+    if (!sid && G.inside) G.walk.alloc(g.P);
+    if (sid && boxes) G.rec.alloc(12 * g.P);
+    if (G.walk.p || G.rec.p)
+        hipLaunchKernelGGL(k_ray_records, dim3(rays256), dim3(256), 0, s, g, sid, G.walk.p,
+                           G.rec.p);
+    // at most one part per ray and box face crossed: their count must fit 32 bits
+    const int64_t parts = boxes_along(g.rvy, kRayBoxY) + boxes_along(g.rvx, kRayBoxXZ) +
+                          (int64_t)boxes_along(g.rvz, kRayBoxXZ);
+    if (boxes && (sid || G.inside) && op->n < (int64_t(1) << 31) && g.P * parts < (int64_t(1) << 31)) {
+        try {
+            build_ray_boxes(ctx, G);
+        } catch (const tv3_error &e) {
+            if (e.status != TV3_E_NOMEM) throw;
+            G.boxes = RayBoxes();      // the per-ray kernel needs no memory
+        }
+    }
+    TV3_HIP(hipGetLastError());
+    TV3_HIP(hipStreamSynchronize(s));
 }
 
 // ------------------------------------------------------------- materialize

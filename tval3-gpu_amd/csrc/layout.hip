@@ -42,35 +42,64 @@ static std::vector<int32_t> spatial_rank(const std::vector<float> &pos) {
     return rank;
 }
 
-// Rays in bundles: 4 emitters x 4 receivers neighbouring in spatial rank
+// Rays in bundles of neighbours: the rays of one measurement position by
+// (emitter rank / bundle, receiver rank / bundle, emitter rank, receiver
+// rank), ranks being spatial.  path_h lists a position's rays by emitter,
+// then receiver, so the order is read off a table of each pair's place.
+std::vector<int32_t> ray_bundles(const DynGeom &g, int bundle) {
+    std::vector<int32_t> order;
+    const int64_t P = g.num_paths;
+    if (P == 0 || g.epos_h.empty() || g.rpos_h.empty() || (int64_t)g.path_h.size() != 2 * P)
+        return order;
+    const std::vector<int32_t> er = spatial_rank(g.epos_h), rr = spatial_rank(g.rpos_h);
+    order.reserve(P);
+    // indices first .. first + count in rank order
+    auto sorted = [](const std::vector<int32_t> &rank, int64_t first, int64_t count) {
+        std::vector<int32_t> id(count);
+        std::iota(id.begin(), id.end(), (int32_t)first);
+        std::sort(id.begin(), id.end(), [&](int32_t a, int32_t b) { return rank[a] < rank[b]; });
+        return id;
+    };
+    // end of the run of equal rank / bundle that starts at i
+    auto run_end = [bundle](const std::vector<int32_t> &id, const std::vector<int32_t> &rank,
+                            size_t i) {
+        const int32_t k = rank[id[i]] / bundle;
+        while (i < id.size() && rank[id[i]] / bundle == k) ++i;
+        return i;
+    };
+    std::vector<int32_t> place((size_t)g.E * g.R);
+    int64_t k = 0;
+    for (int32_t mp = 0; mp < g.mps; ++mp) {
+        std::fill(place.begin(), place.end(), -1);
+        for (; k < P && g.path_h[2 * k] / g.E == mp; ++k)
+            place[(size_t)(g.path_h[2 * k] - (int64_t)mp * g.E) * g.R +
+                  (g.path_h[2 * k + 1] - (int64_t)mp * g.R)] = (int32_t)k;
+        const std::vector<int32_t> es = sorted(er, (int64_t)mp * g.E, g.E),
+                                   rs = sorted(rr, (int64_t)mp * g.R, g.R);
+        for (size_t e0 = 0, e1; e0 < es.size(); e0 = e1) {
+            e1 = run_end(es, er, e0);
+            for (size_t r0 = 0, r1; r0 < rs.size(); r0 = r1) {
+                r1 = run_end(rs, rr, r0);
+                for (size_t e = e0; e < e1; ++e)
+                    for (size_t r = r0; r < r1; ++r) {
+                        const int32_t ray = place[(size_t)(es[e] - (int64_t)mp * g.E) * g.R +
+                                                  (rs[r] - (int64_t)mp * g.R)];
+                        if (ray >= 0) order.push_back(ray);
+                    }
+            }
+        }
+    }
+    return order;
+}
+
+// The fused solver's ray order: 4 emitters x 4 receivers
 // form a thin tube whose 16 rays cross nearly the same tiles, so a tile's
 // rays (ascending internal number) come in runs that share cache lines, in
 // A^T's staging of the residual and in the per-ray sums of A's segment
 // partials.  At 128^3 with 256 x 1024 rays this cuts the 64-byte lines those
 // gathers touch from 0.39 to 0.29 (A^T) and from 0.34 to 0.23 (A) per
 // segment against ordering by emitter, then receiver.
-std::vector<int32_t> geometry_ray_order(const DynGeom &g) {
-    std::vector<int32_t> order;
-    const int64_t P = g.num_paths;
-    if (P == 0 || g.epos_h.empty() || g.rpos_h.empty() || (int64_t)g.path_h.size() != 2 * P)
-        return order;
-    std::vector<int32_t> er = spatial_rank(g.epos_h), rr = spatial_rank(g.rpos_h);
-    constexpr int kBundle = 4;
-    order.resize(P);
-    std::iota(order.begin(), order.end(), 0);
-    std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) {
-        const int32_t ea = g.path_h[2 * a], eb = g.path_h[2 * b];
-        const int32_t ma = ea / g.E, mb = eb / g.E;
-        if (ma != mb) return ma < mb;
-        const int32_t xa = er[ea], xb = er[eb];
-        const int32_t ya = rr[g.path_h[2 * a + 1]], yb = rr[g.path_h[2 * b + 1]];
-        if (xa / kBundle != xb / kBundle) return xa / kBundle < xb / kBundle;
-        if (ya / kBundle != yb / kBundle) return ya / kBundle < yb / kBundle;
-        if (xa != xb) return xa < xb;
-        return ya < yb;
-    });
-    return order;
-}
+std::vector<int32_t> geometry_ray_order(const DynGeom &g) { return ray_bundles(g, 4); }
 
 __global__ void k_vox_maps(int p, int q, int r, int B, int nby, int nbx, int32_t *nat2int,
                            int32_t *int2nat) {

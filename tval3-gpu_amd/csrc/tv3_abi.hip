@@ -412,6 +412,7 @@ tv3_status tv3_op_dynamic_create(tv3_ctx *ctx, const tv3_geometry *geom, tv3_wei
         op->device = ctx->device;
         op->kind = OpKind::DYNAMIC;
         fill_geometry(ctx, geom, mode, op.get());
+        dynamic_prepare(op.get(), true);
         op->fused = build_dyn_layout(op.get());   // Siddon, dims multiples of 4: tile products
         *out = op.release();
     });
@@ -432,6 +433,7 @@ tv3_status tv3_op_hybrid_create(tv3_ctx *ctx, const tv3_geometry *geom, tv3_weig
         op->device = ctx->device;
         op->kind = OpKind::HYBRID;
         fill_geometry(ctx, geom, mode, op.get());
+        dynamic_prepare(op.get(), false);
         const int64_t m = op->m, n = op->n;
         SparseRows A;                        // freed after the stream has drained
         if (cptr) {                          // the caller's CSC is A^T's rows

@@ -137,6 +137,18 @@ struct SparseRows {
 void build_row_blocks(tv3_ctx *ctx, SparseRows &S, int blk_nnz,
                       const std::vector<int64_t> *starts = nullptr);
 
+// The parts of a geometry's rays inside boxes of kRayBox{Y,X,Z} voxels, for
+// the A^T products of dynamic.hip: built on the device when a matrix-free
+// operator is created, read only afterwards (any number of streams).
+struct RayBoxes {
+    int64_t nitem = 0;         // 0: not built (the per-ray kernels serve)
+    bool split = false;        // some box has several work items
+    DevBuf<int4> item;         // box, first and end segment, 1 if the box is split;
+                               // most segments first
+    DevBuf<uint2> seg;         // per segment: ray; Bresenham: first step | steps << 16,
+                               // Siddon: box-local first voxel x | y << 4 | z << 8
+};
+
 struct DynGeom {
     int32_t E = 0, R = 0, mps = 0, rv_x = 0, rv_y = 0, rv_z = 0;
     float scale = 1.f;
@@ -147,6 +159,11 @@ struct DynGeom {
     DevBuf<int32_t> ecoord;    // 3 * mps*E  (x, y, z) Bresenham
     DevBuf<int32_t> rcoord;    // 3 * mps*R
     DevBuf<float> epos, rpos;  // 3 * mps*E / 3 * mps*R world coordinates, Siddon
+    bool inside = false;       // Bresenham: every transducer lies in the grid
+    DevBuf<int32_t> bundle;    // rays in bundles of neighbours (empty: natural order)
+    DevBuf<int4> walk;         // Bresenham: emitter x | y << 16, z | dx << 16, dy | dz << 16
+    DevBuf<float> rec;         // Siddon: A[3], L, B[3], amin, amax, 3 unused, per ray
+    RayBoxes boxes;
     float origin[3] = {0, 0, 0}, voxel[3] = {1, 1, 1};
     // host copies used to order rays for cache locality
     std::vector<float> epos_h, rpos_h;   // 3 per transducer (voxel coords for Bresenham)
@@ -157,6 +174,7 @@ struct DynGeom {
 // transducers sorted by polar band and serpentine azimuth, rays sorted by
 // (measurement position, emitter rank, receiver rank).
 std::vector<int32_t> geometry_ray_order(const DynGeom &g);
+std::vector<int32_t> ray_bundles(const DynGeom &g, int bundle);
 
 // Internal index of voxel (y, x, z) in the fused solver's numbering.
 //   B = 1: natural order (y fastest, then x, then z).
@@ -401,6 +419,9 @@ void dynamic_apply(tv3_op *op, bool trans, const float *x, float *y, hipStream_t
 void dynamic_apply(tv3_op *op, bool trans, const double *x, double *y, hipStream_t s,
                    bool acc64 = true);
 void dynamic_materialize(tv3_op *op, tv3_dtype vt, SparseRows &A);
+// what the products of op->geo keep besides the geometry: ray order and
+// records, and with boxes the A^T product's RayBoxes
+void dynamic_prepare(tv3_op *op, bool boxes);
 
 // generic apply: y = op x (trans = 0) or op^T x
 void op_apply(tv3_op *op, bool trans, const float *x, float *y, hipStream_t s,
