@@ -11,6 +11,8 @@
 // consecutive memory: the col/val streams are fully coalesced whatever L is.
 // x is gathered (it stays in L2 / MALL); the group sum is a butterfly over L
 // lanes.  L is chosen from the mean row length or by the autotuner.
+#include <algorithm>
+
 #include "spmv_stream.hpp"
 
 namespace tv3 {
@@ -205,6 +207,166 @@ void spmv_csr(const SparseRows &S, const double *x, double *y, hipStream_t s, in
     case TV3_F32: launch_f64<float>(S, x, y, s, L); break;
     default: throw tv3_error(TV3_E_FORMAT, "FP64 products need F64 or F32 values");
     }
+}
+
+// ------------------------------------------------- several right-hand sides
+// Xt[i][j] = X[i + j ldx] for j < G, 0 for G <= j < KT: one gather then brings
+// an entry's values for all columns.
+template <int KT>
+__global__ __launch_bounds__(256) void k_columns_to_rows(int64_t n, int G,
+                                                         const float *__restrict__ X, int64_t ldx,
+                                                         float *__restrict__ Xt) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    float v[KT];
+#pragma unroll
+    for (int j = 0; j < KT; ++j) v[j] = j < G ? X[i + j * ldx] : 0.f;
+#pragma unroll
+    for (int j = 0; j < KT; j += 4)
+        *reinterpret_cast<float4 *>(Xt + i * KT + j) = make_float4(v[j], v[j + 1], v[j + 2], v[j + 3]);
+}
+
+__device__ __forceinline__ float4 operator*(float a, const float4 &b) {
+    return make_float4(a * b.x, a * b.y, a * b.z, a * b.w);
+}
+
+// row_sum of four columns at once: each column's additions in row_sum's order
+template <int NB>
+__device__ __forceinline__ float4 row_sum4(const float4 *prod, int a, int e, int lane, int L) {
+    float4 s0 = make_float4(0, 0, 0, 0), s1 = s0;
+    for (int k = a + lane; k < e; k += 4 * L) {
+        float4 v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[i] = prod[min(k + i * L, NB - 1)];
+            if (i > 0 && k + i * L >= e) v[i] = make_float4(0, 0, 0, 0);
+        }
+        s0.x += v[0].x + v[2].x; s0.y += v[0].y + v[2].y;
+        s0.z += v[0].z + v[2].z; s0.w += v[0].w + v[2].w;
+        s1.x += v[1].x + v[3].x; s1.y += v[1].y + v[3].y;
+        s1.z += v[1].z + v[3].z; s1.w += v[1].w + v[3].w;
+    }
+    return make_float4(s0.x + s1.x, s0.y + s1.y, s0.z + s1.z, s0.w + s1.w);
+}
+
+// k_csr_stream for KT columns: a row block's entries are read once, KT / 4
+// neighbouring lanes gather one entry's KT values (one line look-up serves
+// them), the products go to LDS, and 256 threads per four columns sum the
+// rows.  Every column is summed as k_csr_stream sums it (same bits).  Bound
+// by the gathers of Xt: at 64^3 voxels and 65,536 rays, 8 columns, FP32
+// weights, A 30 us and A^T 59 us, Xt 3-7 us, against eight launches of 17 and
+// 27 us (43 and 81 us when a lane gathered an entry's values in turn).
+template <int NB, int KT, typename V>
+__global__ __launch_bounds__(64 * KT) void k_csr_multi(const BlkDesc *__restrict__ desc,
+                                                       const int32_t *__restrict__ ptr,
+                                                       const int32_t *__restrict__ ind,
+                                                       const V *__restrict__ val,
+                                                       const float *__restrict__ Xt,
+                                                       float *__restrict__ Y, int64_t ldy, int G) {
+    constexpr int Q = KT / 4;                // quads of columns
+    __shared__ float4 prod[Q][NB];
+    const BlkDesc d = desc[xcd_remap(blockIdx.x, gridDim.x)];
+    const int t = threadIdx.x & 255, q2 = threadIdx.x >> 8;      // phase 2: thread, quad
+    const int L = 1 << d.lg, rr = t >> d.lg, lane = t & (L - 1);
+    const bool has = rr < d.nr;
+    const int row = d.r0 + (has ? rr : d.nr - 1);
+    if (d.len <= NB) {
+        constexpr int J = NB / 256;
+        const int a = ptr[row] - d.p0, e = ptr[row + 1] - d.p0;
+        if (d.len > 0) {
+            const int q = threadIdx.x % Q, slot = threadIdx.x / Q, last = d.p0 + d.len - 1;
+            int c[J];
+            float w[J];
+#pragma unroll
+            for (int j = 0; j < J; ++j) {
+                const int k = min(d.p0 + j * 256 + slot, last);
+                c[j] = ind[k];
+                w[j] = ld_weight<V>(val, k);
+            }
+#pragma unroll
+            for (int j = 0; j < J; ++j)
+                prod[q][j * 256 + slot] =
+                    w[j] * *reinterpret_cast<const float4 *>(Xt + (int64_t)c[j] * KT + 4 * q);
+        }
+        __syncthreads();
+        float4 s = make_float4(0, 0, 0, 0);
+        if (has) s = row_sum4<NB>(prod[q2], a, e, lane, L);
+        const float o[4] = {lane_sum(s.x, L), lane_sum(s.y, L), lane_sum(s.z, L), lane_sum(s.w, L)};
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (has && lane == 0 && 4 * q2 + j < G) Y[row + (4 * q2 + j) * ldy] = o[j];
+    } else {
+        // one row longer than NB
+        float s[4] = {};
+        for (int k = d.p0 + t; k < d.p0 + d.len; k += 256) {
+            const float w = ld_weight<V>(val, k);
+            const float *x = Xt + (int64_t)ind[k] * KT + 4 * q2;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s[j] += w * x[j];
+        }
+        float *sh = reinterpret_cast<float *>(prod);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            s[j] = lane_sum<64>(s[j]);
+            if ((t & 63) == 0) sh[4 * (4 * q2 + j) + (t >> 6)] = s[j];
+        }
+        __syncthreads();
+        const int g = threadIdx.x;
+        if (g < G) Y[d.r0 + g * ldy] = (sh[4 * g] + sh[4 * g + 1]) + (sh[4 * g + 2] + sh[4 * g + 3]);
+    }
+}
+
+bool spmv_multi_ok(const SparseRows &S) {
+    return S.blk_nnz != 0 && (S.vtype == TV3_F32 || S.vtype == TV3_F16 || S.vtype == TV3_BF16);
+}
+
+size_t spmv_multi_scratch(const SparseRows &S) { return (size_t)S.cols * 8; }
+
+template <int KT, typename V>
+static void launch_multi(const SparseRows &S, int G, const float *xt, float *Y, int64_t ldy,
+                         hipStream_t s) {
+    const dim3 g((unsigned)S.nblk);
+    const V *val = reinterpret_cast<const V *>(S.val.p);
+#define TV3_MCASE(NBV)                                                                        \
+    case NBV:                                                                                 \
+        hipLaunchKernelGGL((k_csr_multi<NBV, KT, V>), g, dim3(64 * KT), 0, s, S.desc.p,        \
+                           S.ptr.p, S.ind.p, val, xt, Y, ldy, G);                             \
+        return;
+    switch (S.blk_nnz) {
+        TV3_MCASE(1024) TV3_MCASE(2048)
+    case 4096:           // 64 KB of products for four columns
+        if constexpr (KT == 4) {
+            hipLaunchKernelGGL((k_csr_multi<4096, KT, V>), g, dim3(64 * KT), 0, s, S.desc.p, S.ptr.p,
+                               S.ind.p, val, xt, Y, ldy, G);
+            return;
+        }
+    default: throw tv3_error(TV3_E_ARG, "stream block size must be 1024, 2048 or 4096");
+    }
+#undef TV3_MCASE
+}
+
+template <int KT>
+static void multi(const SparseRows &S, int G, const float *X, int64_t ldx, float *Y, int64_t ldy,
+                  float *xt, hipStream_t s) {
+    hipLaunchKernelGGL(k_columns_to_rows<KT>, dim3((unsigned)((S.cols + 255) / 256)), dim3(256), 0,
+                       s, S.cols, G, X, ldx, xt);
+    if (S.nblk == 0) return;
+    switch (S.vtype) {
+    case TV3_F32: launch_multi<KT, float>(S, G, xt, Y, ldy, s); break;
+    case TV3_F16: launch_multi<KT, __half>(S, G, xt, Y, ldy, s); break;
+    default: launch_multi<KT, __hip_bfloat16>(S, G, xt, Y, ldy, s); break;
+    }
+}
+
+void spmv_multi(const SparseRows &S, int nrhs, const float *X, int64_t ldx, float *Y, int64_t ldy,
+                float *xt, hipStream_t s) {
+    if (nrhs > 4 && S.blk_nnz <= 2048) {
+        multi<8>(S, nrhs, X, ldx, Y, ldy, xt, s);
+    } else {
+        multi<4>(S, std::min(nrhs, 4), X, ldx, Y, ldy, xt, s);
+        if (nrhs > 4) multi<4>(S, nrhs - 4, X + 4 * ldx, ldx, Y + 4 * ldy, ldy, xt, s);
+    }
+    TV3_HIP(hipGetLastError());
 }
 
 // ------------------------------------------------------------------ scan

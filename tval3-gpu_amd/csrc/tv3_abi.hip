@@ -562,6 +562,20 @@ tv3_status tv3_matvec_multi(tv3_op *op, tv3_trans trans, int32_t nrhs, const flo
         const int64_t R = yl, K = xl;
         const bool mfma = op->kind == OpKind::DENSE && op->dtype == TV3_BF16 && R % 256 == 0 &&
                           K % 64 == 0 && op->lda % 8 == 0 && ldx % 4 == 0;
+        // a sparse matrix in row blocks is read once for up to eight vectors; the
+        // workspace needs its order kept over streams, which a capture cannot
+        const SparseRows *S = op->kind == OpKind::CSR ? (T ? &op->AT : &op->A)
+                              : op->kind == OpKind::HYBRID && T ? &op->AT : nullptr;
+        if (S && nrhs > 1 && spmv_multi_ok(*S) && !capturing(s)) {
+            float *xt = reinterpret_cast<float *>(
+                op->multi_ws.acquire(s, spmv_multi_scratch(*S) * sizeof(float)));
+            int32_t j = 0;
+            for (; nrhs - j > 1; j += 8)
+                spmv_multi(*S, std::min(8, nrhs - j), X + j * ldx, ldx, Y + j * ldy, ldy, xt, s);
+            if (j < nrhs) spmv_csr(*S, X + j * ldx, Y + j * ldy, s);
+            op->multi_ws.release(s);
+            return;
+        }
         if (!mfma) {
             for (int32_t j = 0; j < nrhs; ++j) op_apply(op, T, X + j * ldx, Y + j * ldy, s);
             TV3_HIP(hipGetLastError());

@@ -92,6 +92,39 @@ struct PinnedBuf {
     }
 };
 
+// Workspace of an object's calls that may run on several streams: acquire
+// makes the stream wait for the last use, release marks the end of this one.
+// Grown on demand (freeing the smaller buffer waits for the device), kept
+// until the object is destroyed.  Not for a stream that is being captured.
+struct SharedScratch {
+    DevBuf<uint8_t> buf;
+    hipEvent_t done = nullptr;
+    bool used = false;
+    SharedScratch() = default;
+    SharedScratch(const SharedScratch &) = delete;
+    SharedScratch &operator=(const SharedScratch &) = delete;
+    ~SharedScratch() { if (done) (void)hipEventDestroy(done); }
+    uint8_t *acquire(hipStream_t s, size_t bytes) {
+        if (!done) TV3_HIP(hipEventCreateWithFlags(&done, hipEventDisableTiming));
+        if (used) TV3_HIP(hipStreamWaitEvent(s, done, 0));
+        if (buf.bytes() < bytes) buf.alloc(bytes);
+        return buf.p;
+    }
+    void release(hipStream_t s) {
+        TV3_HIP(hipEventRecord(done, s));
+        used = true;
+    }
+};
+
+inline bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
 inline size_t dtype_size(tv3_dtype t) {
     switch (t) {
     case TV3_F32: return 4;
@@ -364,6 +397,7 @@ struct tv3_op {
     int64_t lda = 0;
     tv3::DevBuf<uint8_t> dense_oN, dense_oT;   // A and A^T in MFMA operand order (multi-RHS
                                                // products), built on demand
+    tv3::SharedScratch multi_ws;               // sparse products of several vectors
     // DYNAMIC / HYBRID
     tv3::DynGeom geo;
     // CSR built from a geometry: the locality order of its rays (may be empty)
@@ -382,6 +416,12 @@ void spmv_csr(const SparseRows &S, const float *x, float *y, hipStream_t s, int 
 void spmv_csr(const SparseRows &S, const double *x, double *y, hipStream_t s, int lanes = 0,
               bool acc64 = true);
 int default_lanes(int64_t rows, int64_t nnz);
+// Y[:, j] = S X[:, j], j < nrhs <= 8, from one reading of S; xt: workspace of
+// spmv_multi_scratch floats.  S in row blocks, F32, F16 or BF16
+bool spmv_multi_ok(const SparseRows &S);
+size_t spmv_multi_scratch(const SparseRows &S);
+void spmv_multi(const SparseRows &S, int nrhs, const float *X, int64_t ldx, float *Y, int64_t ldy,
+                float *xt, hipStream_t s);
 // Stable device transpose of a CSR (rows ordered ascending within each column).
 void build_transpose(tv3_ctx *ctx, const SparseRows &A, SparseRows &AT);
 // exclusive scan of cnt[0..n) into out[0..n] (out[n] = total); returns total
