@@ -220,10 +220,11 @@ tv3_status tv3_matvec_noalloc(tv3_op *op, tv3_trans trans, const float *x_dev, f
  * product (each FP32 value of X split into three BF16 terms, hi + mid + lo,
  * FP32 accumulation; the first such call builds copies of A and A^T in the
  * matrix cores' operand order, 2 m n bytes each, kept with the operator);
- * any other operator gives tv3_matvec's result per column, a sparse one in
- * row blocks from one reading of the matrix for up to eight columns (with a
- * workspace of eight vectors kept with the operator; not under stream
- * capture).  Asynchronous on stream. */
+ * any other operator gives tv3_matvec's result per column, a dense one and a
+ * sparse one in row blocks from one reading of the matrix for up to eight
+ * columns (the sparse one with a workspace of eight vectors kept with the
+ * operator; one column at a time under stream capture).  Asynchronous on
+ * stream. */
 tv3_status tv3_matvec_multi(tv3_op *op, tv3_trans trans, int32_t nrhs, const float *X_dev,
                             int64_t ldx, float *Y_dev, int64_t ldy, void *stream);
 

@@ -53,6 +53,14 @@ def test_sparse_columns_equal_matvec(ctx, dtype, nrhs):
         _check(op, nrhs, nrhs)
 
 
+@pytest.mark.parametrize("nrhs", [2, 3, 4, 5, 8, 11])
+@pytest.mark.parametrize("dtype,m,n", [("f32", 6, 40), ("f32", 519, 301), ("f16", 130, 4099),
+                                       ("bf16", 1027, 513), ("bf16", 300, 8200)])
+def test_dense_columns_equal_matvec(ctx, dtype, m, n, nrhs):
+    A = np.random.default_rng(m).normal(size=(m, n)).astype(np.float32)
+    _check(api.DenseOperator(ctx, np.asfortranarray(A), dtype), nrhs, nrhs)
+
+
 def test_sparse_on_two_streams(ctx):
     import torch
     op = _sparse(ctx, "f32")

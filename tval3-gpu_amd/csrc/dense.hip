@@ -53,12 +53,12 @@ constexpr int kColsInFlight = 8;
 // Rows beyond the last whole run are covered by moving the last lanes' runs
 // back to end at row m (m >= W): a row held by two lanes gets the same sum
 // twice and both store it.
-template <typename V, int W, typename T, typename AccT>
+template <typename V, int W, int KT, typename T, typename AccT>
 __global__ __launch_bounds__(256) void k_gemv_n_part(int64_t m, int64_t n, int64_t lda,
                                                      const V *__restrict__ A,
-                                                     const T *__restrict__ x,
+                                                     const T *__restrict__ x, int64_t ldx, int G,
                                                      AccT *__restrict__ part, T *__restrict__ y,
-                                                     int64_t cols_per) {
+                                                     int64_t ldy, int64_t cols_per) {
     __shared__ AccT sh[3][64 * W];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -66,48 +66,63 @@ __global__ __launch_bounds__(256) void k_gemv_n_part(int64_t m, int64_t n, int64
     const int64_t s0 = (int64_t)blockIdx.y * cols_per, s1 = min(s0 + cols_per, n);
     const int64_t per = (cols_per + 3) / 4;
     const int64_t j0 = min(s0 + wave * per, s1), j1 = min(j0 + per, s1);
-    AccT s[W] = {};
+    AccT s[KT][W] = {};
     const V *a = A + i + j0 * lda;
+    const T *xk[KT];
+#pragma unroll
+    for (int k = 0; k < KT; ++k) xk[k] = x + (int64_t)min(k, G - 1) * ldx;
     int64_t j = j0;
     for (; j + kColsInFlight <= j1; j += kColsInFlight, a += kColsInFlight * lda) {
         Run<V, W> r[kColsInFlight];
 #pragma unroll
         for (int c = 0; c < kColsInFlight; ++c) r[c] = load_run<V, W>(a + c * lda);
 #pragma unroll
-        for (int c = 0; c < kColsInFlight; ++c) {
-            const AccT xj = (AccT)x[j + c];
+        for (int c = 0; c < kColsInFlight; ++c)
 #pragma unroll
-            for (int e = 0; e < W; ++e) s[e] += up<AccT>(r[c].v[e]) * xj;
-        }
+            for (int k = 0; k < KT; ++k) {
+                const AccT xj = (AccT)xk[k][j + c];
+#pragma unroll
+                for (int e = 0; e < W; ++e) s[k][e] += up<AccT>(r[c].v[e]) * xj;
+            }
     }
     for (; j < j1; ++j, a += lda) {
         const Run<V, W> r = load_run<V, W>(a);
-        const AccT xj = (AccT)x[j];
 #pragma unroll
-        for (int e = 0; e < W; ++e) s[e] += up<AccT>(r.v[e]) * xj;
+        for (int k = 0; k < KT; ++k) {
+            const AccT xj = (AccT)xk[k][j];
+#pragma unroll
+            for (int e = 0; e < W; ++e) s[k][e] += up<AccT>(r.v[e]) * xj;
+        }
     }
-    if (wave > 0) {
 #pragma unroll
-        for (int e = 0; e < W; ++e) sh[wave - 1][e * 64 + lane] = s[e];
-    }
-    __syncthreads();
-    if (wave > 0) return;
+    for (int k = 0; k < KT; ++k) {
+        if (k > 0) __syncthreads();          // the previous vector's sums have been read
+        if (wave > 0) {
 #pragma unroll
-    for (int e = 0; e < W; ++e) {
-        const AccT t = (s[e] + sh[0][e * 64 + lane]) + (sh[1][e * 64 + lane] + sh[2][e * 64 + lane]);
-        if (gridDim.y == 1) y[i + e] = (T)t;
-        else part[(int64_t)blockIdx.y * m + i + e] = t;
+            for (int e = 0; e < W; ++e) sh[wave - 1][e * 64 + lane] = s[k][e];
+        }
+        __syncthreads();
+        if (wave > 0 || k >= G) continue;
+#pragma unroll
+        for (int e = 0; e < W; ++e) {
+            const AccT t = (s[k][e] + sh[0][e * 64 + lane]) +
+                           (sh[1][e * 64 + lane] + sh[2][e * 64 + lane]);
+            if (gridDim.y == 1) y[k * ldy + i + e] = (T)t;
+            else part[((int64_t)k * gridDim.y + blockIdx.y) * m + i + e] = t;
+        }
     }
 }
 
 // y = sum of the ks slab partials: 64 rows a workgroup, its wavefronts each a
 // quarter of the slabs (one thread summing all slabs of a row was a chain of
-// up to 128 dependent loads).
+// up to 128 dependent loads); blockIdx.y is the vector.
 template <typename T, typename AccT>
 __global__ __launch_bounds__(256) void k_gemv_n_sum(int64_t m, int ks,
                                                     const AccT *__restrict__ part,
-                                                    T *__restrict__ y) {
+                                                    T *__restrict__ y, int64_t ldy) {
     __shared__ AccT sh[3][64];
+    part += (int64_t)blockIdx.y * ks * m;
+    y += blockIdx.y * ldy;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t i = min((int64_t)blockIdx.x * 64 + lane, m - 1);
     AccT s = 0;
@@ -124,17 +139,21 @@ __global__ __launch_bounds__(256) void k_gemv_n_sum(int64_t m, int ks,
     if (wave == 0) y[i] = (T)((s + sh[0][lane]) + (sh[1][lane] + sh[2][lane]));
 }
 
-template <typename V, int W, int C, typename T, typename AccT>
+template <typename V, int W, int C, int KT, typename T, typename AccT>
 __global__ __launch_bounds__(256) void k_gemv_t(int64_t m, int64_t n, int64_t lda,
                                                 const V *__restrict__ A,
-                                                const T *__restrict__ x, T *__restrict__ y) {
+                                                const T *__restrict__ x, int64_t ldx, int G,
+                                                T *__restrict__ y, int64_t ldy) {
     const int lane = threadIdx.x & 63;
     const int64_t j0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * C;
     if (j0 >= n) return;
     const V *col[C];
 #pragma unroll
     for (int c = 0; c < C; ++c) col[c] = A + min(j0 + c, n - 1) * lda;
-    AccT s[C] = {}, s2[C] = {};
+    const T *xk[KT];
+#pragma unroll
+    for (int k = 0; k < KT; ++k) xk[k] = x + (int64_t)min(k, G - 1) * ldx;
+    AccT s[C][KT] = {}, s2[C][KT] = {};
     auto add = [&](const Run<V, W> &r, const Run<T, W> &xv, AccT &sum) {
         AccT p = 0;
 #pragma unroll
@@ -145,43 +164,63 @@ __global__ __launch_bounds__(256) void k_gemv_t(int64_t m, int64_t n, int64_t ld
     int64_t i = (int64_t)lane * W;
     for (; i + step < whole; i += 2 * step) {
         Run<V, W> r[C], r2[C];
-        const Run<T, W> xv = load_run<T, W>(x + i), xv2 = load_run<T, W>(x + i + step);
+        Run<T, W> xv[KT], xv2[KT];
+#pragma unroll
+        for (int k = 0; k < KT; ++k) {
+            xv[k] = load_run<T, W>(xk[k] + i);
+            xv2[k] = load_run<T, W>(xk[k] + i + step);
+        }
 #pragma unroll
         for (int c = 0; c < C; ++c) {
             r[c] = load_run<V, W>(col[c] + i);
             r2[c] = load_run<V, W>(col[c] + i + step);
         }
 #pragma unroll
-        for (int c = 0; c < C; ++c) {
-            add(r[c], xv, s[c]);
-            add(r2[c], xv2, s2[c]);
-        }
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int k = 0; k < KT; ++k) {
+                add(r[c], xv[k], s[c][k]);
+                add(r2[c], xv2[k], s2[c][k]);
+            }
     }
     for (; i + W <= m; i += step) {
-        const Run<T, W> xv = load_run<T, W>(x + i);
+        Run<T, W> xv[KT];
 #pragma unroll
-        for (int c = 0; c < C; ++c) add(load_run<V, W>(col[c] + i), xv, s[c]);
+        for (int k = 0; k < KT; ++k) xv[k] = load_run<T, W>(xk[k] + i);
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const Run<V, W> r = load_run<V, W>(col[c] + i);
+#pragma unroll
+            for (int k = 0; k < KT; ++k) add(r, xv[k], s[c][k]);
+        }
     }
     // the rows after the last whole run: one a lane
     const int64_t tail = m / W * W + lane;
     if (tail < m) {
-        const AccT xv = (AccT)x[tail];
 #pragma unroll
-        for (int c = 0; c < C; ++c) s2[c] += up<AccT>(col[c][tail]) * xv;
+        for (int k = 0; k < KT; ++k) {
+            const AccT xv = (AccT)xk[k][tail];
+#pragma unroll
+            for (int c = 0; c < C; ++c) s2[c][k] += up<AccT>(col[c][tail]) * xv;
+        }
     }
 #pragma unroll
-    for (int c = 0; c < C; ++c) {
-        const AccT t = lane_sum<64>(s[c] + s2[c]);
-        if (lane == 0 && j0 + c < n) y[j0 + c] = (T)t;
-    }
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int k = 0; k < KT; ++k) {
+            const AccT t = lane_sum<64>(s[c][k] + s2[c][k]);
+            if (lane == 0 && j0 + c < n && k < G) y[k * ldy + j0 + c] = (T)t;
+        }
 }
 
 }  // namespace
 
-// ws: the split-K partials of A x go to this workspace of ws_bytes (the
-// allocation-free path) instead of the context's, which grows on demand
-template <typename V, int W, typename T, typename AccT>
-static void gemv_n(tv3_op *op, const T *x, T *y, hipStream_t s, void *ws, size_t ws_bytes) {
+// G vectors (1 <= G <= KT).  ws: the split-K partials of A x go to this
+// workspace of ws_bytes (the allocation-free path, one vector) instead of the
+// context's, which grows on demand.
+template <typename V, int W, int KT, typename T, typename AccT>
+static void gemv_n(tv3_op *op, int G, const T *x, int64_t ldx, T *y, int64_t ldy, hipStream_t s,
+                   void *ws, size_t ws_bytes) {
     const V *A = reinterpret_cast<const V *>(op->dense.p);
     const int64_t m = op->m, n = op->n, lda = op->lda;
     // the workspace a caller provides is checked for min(128, ceil(n / 64))
@@ -200,39 +239,81 @@ static void gemv_n(tv3_op *op, const T *x, T *y, hipStream_t s, void *ws, size_t
     ks = (n + cols_per - 1) / cols_per;
     AccT *part = reinterpret_cast<AccT *>(ws);
     if (!ws && ks > 1) {
-        if (op->ctx->scratch.bytes() < need) op->ctx->scratch.alloc(need);
+        if (op->ctx->scratch.bytes() < KT * need) op->ctx->scratch.alloc(KT * need);
         part = reinterpret_cast<AccT *>(op->ctx->scratch.p);
     }
-    hipLaunchKernelGGL((k_gemv_n_part<V, W, T, AccT>), dim3((unsigned)tiles, (unsigned)ks),
-                       dim3(256), 0, s, m, n, lda, A, x, part, y, cols_per);
+    hipLaunchKernelGGL((k_gemv_n_part<V, W, KT, T, AccT>), dim3((unsigned)tiles, (unsigned)ks),
+                       dim3(256), 0, s, m, n, lda, A, x, ldx, G, part, y, ldy, cols_per);
     if (ks > 1)
-        hipLaunchKernelGGL((k_gemv_n_sum<T, AccT>), dim3((unsigned)((m + 63) / 64)), dim3(256), 0,
-                           s, m, (int)ks, part, y);
+        hipLaunchKernelGGL((k_gemv_n_sum<T, AccT>), dim3((unsigned)((m + 63) / 64), (unsigned)G),
+                           dim3(256), 0, s, m, (int)ks, part, y, ldy);
 }
 
-template <typename V, int C, typename T, typename AccT>
-static void gemv_t(tv3_op *op, const T *x, T *y, hipStream_t s) {
+template <typename V, int C, int KT, typename T, typename AccT>
+static void gemv_t(tv3_op *op, int G, const T *x, int64_t ldx, T *y, int64_t ldy, hipStream_t s) {
     constexpr int W = run_of<V>();
-    hipLaunchKernelGGL((k_gemv_t<V, W, C, T, AccT>), dim3((unsigned)((op->n + 4 * C - 1) / (4 * C))),
-                       dim3(256), 0, s, op->m, op->n, op->lda,
-                       reinterpret_cast<const V *>(op->dense.p), x, y);
+    hipLaunchKernelGGL((k_gemv_t<V, W, C, KT, T, AccT>),
+                       dim3((unsigned)((op->n + 4 * C - 1) / (4 * C))), dim3(256), 0, s, op->m,
+                       op->n, op->lda, reinterpret_cast<const V *>(op->dense.p), x, ldx, G, y, ldy);
 }
 
-template <typename V, typename T, typename AccT>
-static void gemv(tv3_op *op, bool trans, const T *x, T *y, hipStream_t s, void *ws = nullptr,
-                 size_t ws_bytes = 0) {
+template <typename V, int KT, typename T, typename AccT>
+static void gemv(tv3_op *op, bool trans, int G, const T *x, int64_t ldx, T *y, int64_t ldy,
+                 hipStream_t s, void *ws = nullptr, size_t ws_bytes = 0) {
     constexpr int W = run_of<V>();
     if (!trans) {
-        if (op->m >= W) gemv_n<V, W, T, AccT>(op, x, y, s, ws, ws_bytes);
-        else gemv_n<V, 1, T, AccT>(op, x, y, s, ws, ws_bytes);
+        if (op->m >= W) gemv_n<V, W, KT, T, AccT>(op, G, x, ldx, y, ldy, s, ws, ws_bytes);
+        else gemv_n<V, 1, KT, T, AccT>(op, G, x, ldx, y, ldy, s, ws, ws_bytes);
     } else {
         // columns per wavefront: as many as leave eight wavefronts a CU
         const int64_t waves = 8 * (int64_t)op->ctx->num_cus;
-        if (op->n >= 4 * waves) gemv_t<V, 4, T, AccT>(op, x, y, s);
-        else if (op->n >= 2 * waves) gemv_t<V, 2, T, AccT>(op, x, y, s);
-        else gemv_t<V, 1, T, AccT>(op, x, y, s);
+        if (op->n >= 4 * waves) gemv_t<V, 4, KT, T, AccT>(op, G, x, ldx, y, ldy, s);
+        else if (op->n >= 2 * waves) gemv_t<V, 2, KT, T, AccT>(op, G, x, ldx, y, ldy, s);
+        else gemv_t<V, 1, KT, T, AccT>(op, G, x, ldx, y, ldy, s);
     }
     TV3_HIP(hipGetLastError());
+}
+
+// one vector
+template <typename V, typename T, typename AccT>
+static void gemv(tv3_op *op, bool trans, const T *x, T *y, hipStream_t s, void *ws = nullptr,
+                 size_t ws_bytes = 0) {
+    gemv<V, 1, T, AccT>(op, trans, 1, x, 0, y, 0, s, ws, ws_bytes);
+}
+
+// Several vectors, each with its single product's additions in the same
+// order (same bits): a reading of A serves up to eight.  2047 x 8190 FP32, 8
+// vectors, A X 448 -> 20 us and A^T R 105 -> 18 us (26 four at a time); 64
+// vectors 3579 -> 155 and 831 -> 137 us; 4000 x 16001 BF16, 8 vectors, 571 ->
+// 34 and 342 -> 47 us (one at a time, before).
+template <typename V>
+static void gemv_multi(tv3_op *op, bool trans, int nrhs, const float *X, int64_t ldx, float *Y,
+                       int64_t ldy, hipStream_t s) {
+    for (int j = 0; j < nrhs;) {
+        const int left = nrhs - j;
+        const float *x = X + j * ldx;
+        float *y = Y + j * ldy;
+        if (left == 1) {
+            gemv<V, 1, float, float>(op, trans, 1, x, ldx, y, ldy, s);
+        } else if (left == 2) {
+            gemv<V, 2, float, float>(op, trans, 2, x, ldx, y, ldy, s);
+        } else if (left <= 4) {
+            gemv<V, 4, float, float>(op, trans, left, x, ldx, y, ldy, s);
+        } else {
+            gemv<V, 8, float, float>(op, trans, std::min(left, 8), x, ldx, y, ldy, s);
+        }
+        j += std::min(left, 8);
+    }
+}
+
+void dense_gemv_multi(tv3_op *op, bool trans, int nrhs, const float *X, int64_t ldx, float *Y,
+                      int64_t ldy, hipStream_t s) {
+    switch (op->dtype) {
+    case TV3_F32: gemv_multi<float>(op, trans, nrhs, X, ldx, Y, ldy, s); break;
+    case TV3_F16: gemv_multi<__half>(op, trans, nrhs, X, ldx, Y, ldy, s); break;
+    case TV3_BF16: gemv_multi<__hip_bfloat16>(op, trans, nrhs, X, ldx, Y, ldy, s); break;
+    default: throw tv3_error(TV3_E_FORMAT, "FP32 dense products need F32, F16 or BF16 values");
+    }
 }
 
 void dense_gemv(tv3_op *op, bool trans, const float *x, float *y, hipStream_t s, bool acc64) {

@@ -576,6 +576,11 @@ tv3_status tv3_matvec_multi(tv3_op *op, tv3_trans trans, int32_t nrhs, const flo
             op->multi_ws.release(s);
             return;
         }
+        if (!mfma && op->kind == OpKind::DENSE) {
+            dense_gemv_multi(op, T, nrhs, X, ldx, Y, ldy, s);
+            TV3_HIP(hipGetLastError());
+            return;
+        }
         if (!mfma) {
             for (int32_t j = 0; j < nrhs; ++j) op_apply(op, T, X + j * ldx, Y + j * ldy, s);
             TV3_HIP(hipGetLastError());

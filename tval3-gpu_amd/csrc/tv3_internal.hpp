@@ -432,6 +432,9 @@ void dense_gemv(tv3_op *op, bool trans, const float *x, float *y, hipStream_t s,
                 bool acc64 = false);
 void dense_gemv(tv3_op *op, bool trans, const double *x, double *y, hipStream_t s,
                 bool acc64 = true);
+// Y[:, j] = A X[:, j] or A^T X[:, j] for j < nrhs, each column as dense_gemv
+void dense_gemv_multi(tv3_op *op, bool trans, int nrhs, const float *X, int64_t ldx, float *Y,
+                      int64_t ldy, hipStream_t s);
 // y = A x as dense_gemv (FP32 accumulation) with the split-K partials in the
 // caller's workspace ws of ws_bytes; a larger need is rejected
 void dense_gemv_ws(tv3_op *op, const float *x, float *y, hipStream_t s, void *ws,
