@@ -1,5 +1,5 @@
-// solver_plain.hip -- the reference-shaped TVAL3 loop on the device: one
-// kernel per vector operation and host-side scalars, in the order of
+// solver_plain.hip -- the reference-shaped TVAL3 loop on the device, with
+// host-side scalars, in the order of
 // 3d/tval3_gpu_3d.cpp:1088-1345 (get_g :366-572, get_tau :577-666, descend
 // :671-701, update_g :706-818, min_u :823-891, get_gradient :896-919,
 // shrinkage :924-960, update_W :965-1029, update_mlp :1034-1083).
@@ -14,6 +14,12 @@
 //    the oracle's rounding instead of the accumulation order of a library;
 //  * vector kernels are compiled without FP contraction (a*x+y rounds
 //    twice, as written);
+//  * vector operations between two host decisions share kernels (descend + D;
+//    the gradient parts with lam2, lam4; shrinkage; the update of W's
+//    consequences with every sum the next decision needs), each element
+//    computed and rounded as by one kernel per operation; an iteration
+//    without backtracking waits for the device twice, and the previous
+//    iterate is kept by exchanging buffers;
 //  * every work vector is allocated once per solve (the reference allocates
 //    and frees 3 n-vectors inside get_g/update_g/update_W/update_mlp);
 //  * the A^T-skip heuristic (:398-468) leaves a skipped g as A^T(last Au)
@@ -40,27 +46,40 @@ struct PlainState {
     int64_t n, m;
     double mu, beta, muDbeta, f, lam1, lam2, lam3, lam4, lam5;
     DevBuf<T> pool;
-    T *delta, *sx, *sy, *sz, *Up, *dU, *uup, *Ux, *Uxp, *dUx, *Uy, *Uyp, *dUy, *Uz, *Uzp, *dUz,
-        *Wx, *Wy, *Wz, *Atb, *Au, *Aup, *dAu, *d, *g, *gp, *dg, *g2, *g2p, *dg2, *Vx, *Vy, *Vz,
-        *dx, *dy, *dz, *Ad, *DtsAtd, *rcdU, *bs, *lastAu, *dlast;
+    T *delta, *sx, *sy, *sz, *dU, *dUx, *dUy, *dUz, *Wx, *Wy, *Wz, *Atb, *dAu, *d, *dg, *dg2, *Ad,
+        *DtsAtd, *rcdU, *bs, *lastAu, *dlast;
+    // the iterate and what follows from it (0), and the previous one's (1)
+    T *U[2], *Ux[2], *Uy[2], *Uz[2], *g[2], *g2[2], *Au[2];
+    double dd = 0, uu = 0, upup = 0, ug = 0;   // |d|^2, |U - Up|^2, |Up|^2, <U - Up, dgrad>
     int64_t nN = 0, nT = 0;
     int cur_init = 0;        // A^T-skip state (:155-157)
     double cur_skip = 0.0;
     bool last_mul = true;    // the last get_g multiplied by A^T
 
     void alloc() {
-        T **nv[] = {&sx, &sy, &sz, &Up, &dU, &uup, &Ux, &Uxp, &dUx, &Uy, &Uyp, &dUy, &Uz, &Uzp,
-                    &dUz, &Wx, &Wy, &Wz, &Atb, &d, &g, &gp, &dg, &g2, &g2p, &dg2, &Vx, &Vy, &Vz,
-                    &dx, &dy, &dz, &DtsAtd, &rcdU};
-        T **mv[] = {&delta, &Au, &Aup, &dAu, &Ad, &bs, &lastAu, &dlast};
+        // DtsAtd, sigma and delta start at zero (:1128-1139)
+        T **nv[] = {&DtsAtd, &sx, &sy, &sz, &dU, &dUx, &dUy, &dUz, &Wx, &Wy, &Wz, &Atb, &d, &dg,
+                    &dg2, &rcdU, &U[0], &U[1], &Ux[0], &Ux[1], &Uy[0], &Uy[1], &Uz[0], &Uz[1],
+                    &g[0], &g[1], &g2[0], &g2[1]};
+        T **mv[] = {&delta, &dAu, &Ad, &bs, &lastAu, &dlast, &Au[0], &Au[1]};
         const size_t cn = sizeof(nv) / sizeof(nv[0]), cm = sizeof(mv) / sizeof(mv[0]);
         // pad each vector to 256 bytes
         auto pad = [](int64_t k) { return (k + 63) / 64 * 64; };
         pool.alloc(cn * pad(n) + cm * pad(m));
-        TV3_HIP(hipMemsetAsync(pool.p, 0, pool.bytes(), s));
         T *p = pool.p;
         for (size_t k = 0; k < cn; ++k) { *nv[k] = p; p += pad(n); }
         for (size_t k = 0; k < cm; ++k) { *mv[k] = p; p += pad(m); }
+        TV3_HIP(hipMemsetAsync(DtsAtd, 0, sizeof(T) * 4 * pad(n), s));
+        TV3_HIP(hipMemsetAsync(delta, 0, sizeof(T) * m, s));
+        // the skip rule compares with lastAu before the first product fills it
+        TV3_HIP(hipMemsetAsync(lastAu, 0, sizeof(T) * m, s));
+    }
+    PlainFields<T> fields() {
+        return {dims, n, Ux[0], Uy[0], Uz[0], Wx, Wy, Wz, sx, sy, sz, g2[0]};
+    }
+    // the iterate becomes the previous one
+    void turn() {
+        for (auto *v : {U, Ux, Uy, Uz, g, g2, Au}) std::swap(v[0], v[1]);
     }
     void copy(T *dst, const T *src, int64_t k) {
         TV3_HIP(hipMemcpyAsync(dst, src, sizeof(T) * k, hipMemcpyDeviceToDevice, s));
@@ -71,21 +90,22 @@ struct PlainState {
     }
     double fval() const { return lam1 + beta / 2 * lam2 + mu / 2 * lam3 - lam4 - lam5; }
 
-    void get_lams() {
-        auto a = lam24<T>(ctx, n, Ux, Uy, Uz, Wx, Wy, Wz, sx, sy, sz, Vx, Vy, Vz, s);
-        lam2 = a[0]; lam4 = a[1];
-        auto c = lam35<T>(ctx, m, Au, bs, delta, s);
-        lam3 = c[0]; lam5 = c[1];
+    void set_f(const double *v) {      // lam2, lam4, lam3, lam5
+        lam2 = v[0]; lam4 = v[1]; lam3 = v[2]; lam5 = v[3];
+        f = fval();
     }
     // :366-572; force: the initial and the fallback call (:1148, :880)
-    void get_g(const T *U, bool force) {
-        A(false, U, Au);
+    void get_g(bool force) {
+        A(false, U[0], Au[0]);
         bool mul = true;
         if (o->skipMulRatio != 0.0) {
             // relative change of Au since the last A^T product (:398-412)
-            axpy3<T>(m, dlast, -1.0, lastAu, Au, s);
-            const double dn = dot<T>(ctx, m, dlast, dlast, s), an = dot<T>(ctx, m, Au, Au, s);
-            const double rel = std::sqrt(dn) / std::sqrt(an);
+            axpy3<T>(m, dlast, -1.0, lastAu, Au[0], s);
+            Sums S{ctx, s};
+            queue_dot<T>(S, m, dlast, dlast);
+            queue_dot<T>(S, m, Au[0], Au[0]);
+            const double *v = S.fetch();
+            const double rel = std::sqrt(v[0]) / std::sqrt(v[1]);
             if (force) {
                 cur_skip = 0.0;
             } else if ((uint32_t)cur_init < o->numInitIterations) {
@@ -99,62 +119,70 @@ struct PlainState {
                 cur_skip -= 1.0;
                 mul = false;
             }
-            if (mul) copy(lastAu, Au, m);
+            if (mul) copy(lastAu, Au[0], m);
         }
-        if (mul) A(true, Au, g);
-        get_lams();
-        launch_Dt<T>(dims, Vx, Vy, Vz, g2, s);
-        if (mul) axpy3<T>(n, g, -1.0, Atb, g, s);
+        if (mul) A(true, Au[0], g[0]);
+        else copy(g[0], g[1], n);          // g stays as it was
+        Sums S{ctx, s};
+        queue_gradient<T>(S, fields(), mul ? g[0] : nullptr, Atb);
+        queue_lam35<T>(S, m, Au[0], bs, delta);
         last_mul = mul;
-        f = fval();
+        set_f(S.fetch());
     }
-    double get_tau(bool fst) {
-        if (fst) {
-            launch_D<T>(dims, d, dx, dy, dz, s);
-            double dDd = dot<T>(ctx, n, dx, dx, s) + dot<T>(ctx, n, dy, dy, s) +
-                         dot<T>(ctx, n, dz, dz, s);
-            double dd = dot<T>(ctx, n, d, d, s);
-            A(false, d, Ad);
-            double Add = dot<T>(ctx, m, Ad, Ad, s);
-            return std::fabs(dd / (dDd + muDbeta * Add));
-        }
-        auto r = tau_bb<T>(ctx, n, g, gp, g2, g2p, uup, muDbeta, dg, dg2, s);
-        return std::fabs(r[0] / r[1]);
+    // exact step length along d (:577-640); leaves |d|^2
+    double first_tau() {
+        A(false, d, Ad);
+        Sums S{ctx, s};
+        queue_step<T>(S, dims, d);
+        queue_dot<T>(S, m, Ad, Ad);
+        const double *v = S.fetch();
+        const double dDd = v[0] + v[1] + v[2];
+        dd = v[3];
+        return std::fabs(dd / (dDd + muDbeta * v[4]));
     }
-    void descend(T *U, double tau, bool force) {
-        axpy3<T>(n, U, -tau, d, U, s);
-        if (o->nonneg) nonneg<T>(n, U, s);
-        launch_D<T>(dims, U, Ux, Uy, Uz, s);
-        get_g(U, force);
+    void descend(double tau, bool force) {
+        descend_step<T>(dims, tau, o->nonneg != 0, U[1], d, U[0], Ux[0], Uy[0], Uz[0], s);
+        get_g(force);
     }
-    void update_g(double alpha, T *U) {
-        axpy3<T>(n, g, alpha, dg, gp, s);
-        axpy3<T>(n, g2, alpha, dg2, g2p, s);
-        axpy3<T>(n, U, alpha, dU, Up, s);
-        axpy3<T>(m, Au, alpha, dAu, Aup, s);
-        axpy3<T>(n, Ux, alpha, dUx, Uxp, s);
-        axpy3<T>(n, Uy, alpha, dUy, Uyp, s);
-        axpy3<T>(n, Uz, alpha, dUz, Uzp, s);
-        get_lams();
-        f = fval();
+    void update_g(double alpha) {
+        axpy3<T>(n, g[0], alpha, dg, g[1], s);
+        axpy3<T>(n, g2[0], alpha, dg2, g2[1], s);
+        axpy3<T>(n, U[0], alpha, dU, U[1], s);
+        axpy3<T>(m, Au[0], alpha, dAu, Au[1], s);
+        axpy3<T>(n, Ux[0], alpha, dUx, Ux[1], s);
+        axpy3<T>(n, Uy[0], alpha, dUy, Uy[1], s);
+        axpy3<T>(n, Uz[0], alpha, dUz, Uz[1], s);
+        Sums S{ctx, s};
+        queue_lam24<T>(S, fields());
+        queue_lam35<T>(S, m, Au[0], bs, delta);
+        set_f(S.fetch());
     }
-    void gradient() { grad<T>(n, d, muDbeta, g, g2, DtsAtd, s); }
-    void shrinkage() {
-        lam1 = shrink_host<T>(ctx, n, o->tv_mode == TV3_TV_ISO, Ux, Uy, Uz, sx, sy, sz, beta, Wx,
-                              Wy, Wz, s);
+    void differences() {               // trial - previous, for update_g
+        axpy3<T>(n, dU, -1.0, U[1], U[0], s);
+        axpy3<T>(n, dg, -1.0, g[1], g[0], s);
+        axpy3<T>(n, dg2, -1.0, g2[1], g2[0], s);
+        axpy3<T>(m, dAu, -1.0, Au[1], Au[0], s);
+        axpy3<T>(n, dUx, -1.0, Ux[1], Ux[0], s);
+        axpy3<T>(n, dUy, -1.0, Uy[1], Uy[0], s);
+        axpy3<T>(n, dUz, -1.0, Uz[1], Uz[0], s);
     }
+    void gradient() { grad<T>(n, d, muDbeta, g[0], g2[0], DtsAtd, s); }
+    // W, then all that follows from it: update_W (:965-1029), the direction
+    // (:896-919), and the sums of the next step length and the stopping test
     void update_W() {
         f -= (lam1 + beta / 2 * lam2 - lam4);
-        shrinkage();
-        auto a = lam24<T>(ctx, n, Ux, Uy, Uz, Wx, Wy, Wz, sx, sy, sz, Vx, Vy, Vz, s);
-        lam2 = a[0]; lam4 = a[1];
-        launch_Dt<T>(dims, Vx, Vy, Vz, g2, s);
+        Sums S{ctx, s};
+        queue_shrink<T>(S, fields(), o->tv_mode == TV3_TV_ISO, beta);
+        queue_update<T>(S, fields(), g[0], g[1], g2[1], DtsAtd, U[0], U[1], muDbeta, d);
+        const double *v = S.fetch();
+        lam1 = v[0]; lam2 = v[1]; lam4 = v[2];
+        dd = v[3]; uu = v[4]; upup = v[5]; ug = v[6];
         f += (lam1 + beta / 2 * lam2 - lam4);
     }
     void update_mlp() {
         f += (lam4 + lam5);
-        lam4 = mlp_sigma<T>(ctx, n, Ux, Uy, Uz, Wx, Wy, Wz, beta, sx, sy, sz, s);
-        lam5 = mlp_delta<T>(ctx, m, Au, bs, mu, delta, s);
+        lam4 = mlp_sigma<T>(ctx, n, Ux[0], Uy[0], Uz[0], Wx, Wy, Wz, beta, sx, sy, sz, s);
+        lam5 = mlp_delta<T>(ctx, m, Au[0], bs, mu, delta, s);
         f -= (lam4 + lam5);
     }
 };
@@ -204,15 +232,19 @@ void solve_plain(tv3_ctx *ctx, tv3_op *op, const tv3_opts &o, const int32_t dims
     scale<T>(m, S.bs, scl, b_dev, s);
 
     S.A(true, S.bs, S.Atb);
-    if (!o.warm_start) S.copy(U, S.Atb, n);
-    else scale<T>(n, U, scl, U, s);
+    if (!o.warm_start) S.copy(S.U[0], S.Atb, n);
+    else scale<T>(n, S.U[0], scl, U, s);
     S.mu = std::min(o.mu0, o.mu);
     S.beta = std::min(o.beta0, o.beta);
     S.muDbeta = S.mu / S.beta;
-    S.copy(S.rcdU, U, n);
-    launch_D<T>(dims, U, S.Ux, S.Uy, S.Uz, s);
-    S.shrinkage();
-    S.get_g(U, true);
+    S.copy(S.rcdU, S.U[0], n);
+    launch_D<T>(dims, S.U[0], S.Ux[0], S.Uy[0], S.Uz[0], s);
+    {
+        Sums L{ctx, s};
+        queue_shrink<T>(L, S.fields(), o.tv_mode == TV3_TV_ISO, S.beta);
+        S.lam1 = L.fetch()[0];
+    }
+    S.get_g(true);
     S.gradient();
 
     double Q = 1, Qp, C = S.f, gam = o.gam;
@@ -224,46 +256,35 @@ void solve_plain(tv3_ctx *ctx, tv3_op *op, const tv3_opts &o, const int32_t dims
     while (outer < o.maxcnt && total < o.maxit) {
         bool fst = true;
         while (total < o.maxit) {
-            double tau = S.get_tau(fst);
-            S.copy(S.Up, U, n); S.copy(S.gp, S.g, n); S.copy(S.g2p, S.g2, n);
-            S.copy(S.Aup, S.Au, m); S.copy(S.Uxp, S.Ux, n); S.copy(S.Uyp, S.Uy, n);
-            S.copy(S.Uzp, S.Uz, n);
-            S.descend(U, tau, false);
+            double tau = fst ? S.first_tau() : std::fabs(S.uu / S.ug);
+            S.turn();
+            S.descend(tau, false);
             double alpha = 1.0;
             const double f_trial = S.f;
-            axpy3<T>(n, S.dU, -1.0, S.Up, U, s);
-            double c_armij = dot<T>(ctx, n, S.d, S.d, s) * tau * o.c * S.beta;
+            double c_armij = S.dd * tau * o.c * S.beta;
             int cnt = 0;
             if (std::fabs(S.f) > std::fabs(C - alpha * c_armij)) {
-                axpy3<T>(n, S.dg, -1.0, S.gp, S.g, s);
-                axpy3<T>(n, S.dg2, -1.0, S.g2p, S.g2, s);
-                axpy3<T>(m, S.dAu, -1.0, S.Aup, S.Au, s);
-                axpy3<T>(n, S.dUx, -1.0, S.Uxp, S.Ux, s);
-                axpy3<T>(n, S.dUy, -1.0, S.Uyp, S.Uy, s);
-                axpy3<T>(n, S.dUz, -1.0, S.Uzp, S.Uz, s);
+                S.differences();
                 while (std::fabs(S.f) > std::fabs(C - alpha * c_armij)) {
                     if (cnt == 5) {
                         gam *= o.rate_gam;
-                        tau = S.get_tau(true);
-                        S.copy(U, S.Up, n);
-                        S.descend(U, tau, true);
+                        tau = S.first_tau();
+                        S.descend(tau, true);
                         cnt = 6;
                         ++fallbacks;
                         break;
                     }
                     alpha *= o.gamma;
-                    S.update_g(alpha, U);
+                    S.update_g(alpha);
                     ++cnt;
                 }
                 backtracks += cnt > 5 ? 5 : cnt;
             }
             S.update_W();
             Qp = Q; Q = gam * Qp + 1; C = (gam * Qp * C + S.f) / Q;
-            axpy3<T>(n, S.uup, -1.0, S.Up, U, s);
-            S.gradient();
             ++total;
-            nrmup = std::sqrt(dot<T>(ctx, n, S.Up, S.Up, s));
-            RelChg = std::sqrt(dot<T>(ctx, n, S.uup, S.uup, s)) / nrmup;
+            nrmup = std::sqrt(S.upup);
+            RelChg = std::sqrt(S.uu) / nrmup;
             if (hist && hist->count < hist->cap) {
                 int k = hist->count++;
                 hist->f[k] = S.f; hist->lam1[k] = S.lam1; hist->lam2[k] = S.lam2;
@@ -280,9 +301,9 @@ void solve_plain(tv3_ctx *ctx, tv3_op *op, const tv3_opts &o, const int32_t dims
         }
         if (nonfinite) break;
         ++outer;
-        auto dn = diff_norm<T>(ctx, n, U, S.rcdU, s);
+        auto dn = diff_norm<T>(ctx, n, S.U[0], S.rcdU, s);
         RelChgOut = std::sqrt(dn[0]) / nrmup;
-        S.copy(S.rcdU, U, n);
+        S.copy(S.rcdU, S.U[0], n);
         if (RelChgOut < o.tol) break;
         S.update_mlp();
         double beta0 = S.beta;
@@ -296,7 +317,7 @@ void solve_plain(tv3_ctx *ctx, tv3_op *op, const tv3_opts &o, const int32_t dims
         gam = o.gam; Q = 1; C = S.f;
     }
     TV3_HIP(hipEventRecord(evl1, s));
-    divide<T>(n, U, scl, U, s);    // :1275-1277
+    divide<T>(n, U, scl, S.U[0], s);    // :1275-1277
     TV3_HIP(hipEventRecord(ev1, s));
     TV3_HIP(hipStreamSynchronize(s));
     float ms = 0, msl = 0;

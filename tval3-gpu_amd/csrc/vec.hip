@@ -28,15 +28,6 @@ __global__ void k_grad(int64_t n, T *d, T a, const T *g, const T *g2, const T *d
 }
 
 template <typename T>
-__global__ void k_nonneg(int64_t n, T *u) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        T v = u[i];
-        u[i] = v < 0 ? (T)0 : v;
-    }
-}
-
-template <typename T>
 __global__ void k_scale(int64_t n, T *y, T a, const T *x) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
          i += (int64_t)gridDim.x * blockDim.x)
@@ -64,10 +55,6 @@ void axpy3(int64_t n, T *z, double a, const T *x, const T *y, hipStream_t s) {
 template <typename T>
 void grad(int64_t n, T *d, double a, const T *g, const T *g2, const T *dts, hipStream_t s) {
     hipLaunchKernelGGL(k_grad<T>, dim3(ew_blocks(n)), dim3(256), 0, s, n, d, (T)a, g, g2, dts);
-}
-template <typename T>
-void nonneg(int64_t n, T *u, hipStream_t s) {
-    hipLaunchKernelGGL(k_nonneg<T>, dim3(ew_blocks(n)), dim3(256), 0, s, n, u);
 }
 template <typename T>
 void divide(int64_t n, T *y, double a, const T *x, hipStream_t s) {
@@ -133,10 +120,8 @@ template <typename T> struct FDot {
 
 template <typename T> struct FLam24 {
     const T *Ux, *Uy, *Uz, *Wx, *Wy, *Wz, *sx, *sy, *sz;
-    T *Vx, *Vy, *Vz;
     __device__ void operator()(int64_t i, double *acc) const {
         T vx = Ux[i] - Wx[i], vy = Uy[i] - Wy[i], vz = Uz[i] - Wz[i];
-        Vx[i] = vx; Vy[i] = vy; Vz[i] = vz;
         acc[0] += (double)vx * vx + (double)vy * vy + (double)vz * vz;
         acc[1] += (double)vx * sx[i] + (double)vy * sy[i] + (double)vz * sz[i];
     }
@@ -148,18 +133,6 @@ template <typename T> struct FLam35 {
         T r = Au[i] - b[i];
         acc[0] += (double)r * r;
         acc[1] += (double)delta[i] * r;
-    }
-};
-
-template <typename T> struct FTau {
-    const T *g, *gp, *g2, *g2p, *uup;
-    T mdb;
-    T *dg, *dg2;
-    __device__ void operator()(int64_t i, double *acc) const {
-        T a = g[i] - gp[i], b = g2[i] - g2p[i], u = uup[i];
-        acc[0] += (double)u * u;
-        acc[1] += (double)u * (double)(b + mdb * a);
-        dg[i] = a; dg2[i] = b;
     }
 };
 
@@ -225,6 +198,94 @@ template <typename T> struct FDiffNorm {
     }
 };
 
+// Position of voxel i and its neighbours on the periodic grid; I: 32 bits
+// where the volume allows (two 64-bit divisions a voxel would outweigh the
+// memory traffic).
+template <typename I> struct Grid3 {
+    I p, q, r, pq;
+    struct At {
+        I i, y, x, z;
+    };
+    __device__ __forceinline__ At at(int64_t k) const {
+        const I i = (I)k, c = i / p;
+        return At{i, i - c * p, c % q, c / q};
+    }
+    __device__ __forceinline__ I up_y(const At &a) const { return a.y < p - 1 ? a.i + 1 : a.i - a.y; }
+    __device__ __forceinline__ I up_x(const At &a) const { return a.x < q - 1 ? a.i + p : a.i - a.x * p; }
+    __device__ __forceinline__ I up_z(const At &a) const { return a.z < r - 1 ? a.i + pq : a.i - a.z * pq; }
+    __device__ __forceinline__ I dn_y(const At &a) const { return a.y == 0 ? a.i + (p - 1) : a.i - 1; }
+    __device__ __forceinline__ I dn_x(const At &a) const { return a.x == 0 ? a.i + (q - 1) * p : a.i - p; }
+    __device__ __forceinline__ I dn_z(const At &a) const { return a.z == 0 ? a.i + (r - 1) * pq : a.i - pq; }
+};
+
+// D^T (DU - W) at a voxel; v: DU - W there
+template <typename T, typename I>
+__device__ __forceinline__ T dt_of(const Grid3<I> &G, const typename Grid3<I>::At &a,
+                                   const T *Ux, const T *Uy, const T *Uz, const T *Wx, const T *Wy,
+                                   const T *Wz, T vx, T vy, T vz) {
+    const I jy = G.dn_y(a), jx = G.dn_x(a), jz = G.dn_z(a);
+    const T yp = Uy[jy] - Wy[jy], xp = Ux[jx] - Wx[jx], zp = Uz[jz] - Wz[jz];
+    return yp - vy + xp - vx + zp - vz;
+}
+
+// the four sums of the exact step length: |D d|^2 per component, |d|^2
+template <typename T, typename I> struct FStep {
+    Grid3<I> G;
+    const T *d;
+    __device__ void operator()(int64_t k, double *acc) const {
+        const auto a = G.at(k);
+        const T t = d[a.i];
+        const T dy = d[G.up_y(a)] - t, dx = d[G.up_x(a)] - t, dz = d[G.up_z(a)] - t;
+        acc[0] += (double)dx * (double)dx;
+        acc[1] += (double)dy * (double)dy;
+        acc[2] += (double)dz * (double)dz;
+        acc[3] += (double)t * (double)t;
+    }
+};
+
+// after the products: lam2, lam4, g2 = D^T (DU - W), g = (A^T Au) - Atb
+template <typename T, typename I> struct FGradient {
+    Grid3<I> G;
+    const T *Ux, *Uy, *Uz, *Wx, *Wy, *Wz, *sx, *sy, *sz, *Atb;
+    T *g2, *g;     // g NULL: the A^T product was skipped
+    __device__ void operator()(int64_t k, double *acc) const {
+        const auto a = G.at(k);
+        const I i = a.i;
+        const T vx = Ux[i] - Wx[i], vy = Uy[i] - Wy[i], vz = Uz[i] - Wz[i];
+        acc[0] += (double)vx * vx + (double)vy * vy + (double)vz * vz;
+        acc[1] += (double)vx * sx[i] + (double)vy * sy[i] + (double)vz * sz[i];
+        g2[i] = dt_of<T, I>(G, a, Ux, Uy, Uz, Wx, Wy, Wz, vx, vy, vz);
+        if (g) g[i] = (T)-1 * Atb[i] + g[i];
+    }
+};
+
+// the end of an iteration, W new: lam2, lam4, g2, the direction d, and the
+// sums the next step length and the stopping test take: |d|^2, |U - Up|^2,
+// |Up|^2, <U - Up, change of the gradient>
+template <typename T, typename I> struct FUpdate {
+    Grid3<I> G;
+    const T *Ux, *Uy, *Uz, *Wx, *Wy, *Wz, *sx, *sy, *sz, *g, *gp, *g2p, *dts, *U, *Up;
+    T mdb;
+    T *g2, *d;
+    __device__ void operator()(int64_t k, double *acc) const {
+        const auto a = G.at(k);
+        const I i = a.i;
+        const T vx = Ux[i] - Wx[i], vy = Uy[i] - Wy[i], vz = Uz[i] - Wz[i];
+        acc[0] += (double)vx * vx + (double)vy * vy + (double)vz * vz;
+        acc[1] += (double)vx * sx[i] + (double)vy * sy[i] + (double)vz * sz[i];
+        const T h = dt_of<T, I>(G, a, Ux, Uy, Uz, Wx, Wy, Wz, vx, vy, vz);
+        g2[i] = h;
+        const T gi = g[i], v = mdb * gi + h, di = v + dts[i];
+        d[i] = di;
+        acc[2] += (double)di * (double)di;
+        const T up = Up[i], u = (T)-1 * up + U[i];
+        const T dg = gi - gp[i], dg2 = h - g2p[i];
+        acc[3] += (double)u * u;
+        acc[4] += (double)up * (double)up;
+        acc[5] += (double)u * (double)(dg2 + mdb * dg);
+    }
+};
+
 template <int K, typename F>
 __global__ __launch_bounds__(256) void k_reduce(int64_t n, F f, double *partials) {
     double acc[K];
@@ -235,49 +296,143 @@ __global__ __launch_bounds__(256) void k_reduce(int64_t n, F f, double *partials
     block_sum_store<K>(acc, partials, gridDim.x);
 }
 
+// launches the block partials of K sums over n items into slot s of the
+// context's buffer
 template <int K, typename F>
-std::array<double, K> reduce_now(tv3_ctx *ctx, int64_t n, const F &f, hipStream_t s) {
+static void queue_sums(Sums &S, int64_t n, const F &f) {
     int64_t nb = (n + 255) / 256;
-    if (nb > 1024) nb = 1024;
+    if (nb > kSumBlocks) nb = kSumBlocks;
     if (nb < 1) nb = 1;
-    size_t need = (size_t)K * nb;
-    if (ctx->red_partials.n < need) ctx->red_partials.alloc(need < 8192 ? 8192 : need);
-    ctx->red_host.alloc(ctx->red_partials.n);
-    hipLaunchKernelGGL((k_reduce<K, F>), dim3((unsigned)nb), dim3(256), 0, s, n, f,
-                       ctx->red_partials.p);
+    tv3_ctx *ctx = S.ctx;
+    const size_t cap = (size_t)kSumMax * kSumBlocks;
+    if (ctx->red_partials.n < cap) ctx->red_partials.alloc(cap);
+    ctx->red_host.alloc(cap);
+    TV3_REQUIRE(S.count + K <= kSumMax, TV3_E_INTERNAL, "too many sums at once");
+    hipLaunchKernelGGL((k_reduce<K, F>), dim3((unsigned)nb), dim3(256), 0, S.s, n, f,
+                       ctx->red_partials.p + S.used);
+    for (int k = 0; k < K; ++k) S.blocks[S.count++] = (int)nb;
+    S.used += (size_t)K * nb;
+}
+
+const double *Sums::fetch() {
     TV3_HIP(hipGetLastError());
-    TV3_HIP(hipMemcpyAsync(ctx->red_host.p, ctx->red_partials.p, need * sizeof(double),
+    TV3_HIP(hipMemcpyAsync(ctx->red_host.p, ctx->red_partials.p, used * sizeof(double),
                            hipMemcpyDeviceToHost, s));
     TV3_HIP(hipStreamSynchronize(s));
-    std::array<double, K> out{};
-    for (int k = 0; k < K; ++k) {
+    const double *h = ctx->red_host.p;
+    for (int k = 0; k < count; ++k) {
         double t = 0.0;
-        for (int64_t b = 0; b < nb; ++b) t += ctx->red_host.p[k * nb + b];
-        out[k] = t;
+        for (int b = 0; b < blocks[k]; ++b) t += h[b];
+        h += blocks[k];
+        value[k] = t;
     }
+    used = 0;
+    count = 0;
+    return value;
+}
+
+template <int K, typename F>
+std::array<double, K> reduce_now(tv3_ctx *ctx, int64_t n, const F &f, hipStream_t s) {
+    Sums S{ctx, s};
+    queue_sums<K>(S, n, f);
+    const double *v = S.fetch();
+    std::array<double, K> out{};
+    for (int k = 0; k < K; ++k) out[k] = v[k];
     return out;
+}
+
+// a volume's grid with 32- or 64-bit indices
+template <typename F>
+static void with_grid(const int32_t d[3], F f) {
+    const int64_t pq = (int64_t)d[0] * d[1];
+    if (pq * d[2] < (int64_t(1) << 31))
+        f(Grid3<int32_t>{d[0], d[1], d[2], (int32_t)pq});
+    else
+        f(Grid3<int64_t>{d[0], d[1], d[2], pq});
+}
+
+template <typename T, typename I>
+__global__ __launch_bounds__(256) void k_descend(Grid3<I> G, int64_t n, T tau, int nonneg,
+                                                 const T *__restrict__ U, const T *__restrict__ d,
+                                                 T *__restrict__ V, T *__restrict__ Vx,
+                                                 T *__restrict__ Vy, T *__restrict__ Vz) {
+    const T a = -tau;
+    auto moved = [&](I i) {
+        const T v = a * d[i] + U[i];
+        return nonneg && v < 0 ? (T)0 : v;
+    };
+    for (int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x; k < n; k += (int64_t)gridDim.x * 256) {
+        const auto at = G.at(k);
+        const T t = moved(at.i);
+        V[at.i] = t;
+        Vy[at.i] = moved(G.up_y(at)) - t;
+        Vx[at.i] = moved(G.up_x(at)) - t;
+        Vz[at.i] = moved(G.up_z(at)) - t;
+    }
+}
+
+template <typename T>
+void descend_step(const int32_t dims[3], double tau, bool nonneg, const T *U, const T *d, T *V,
+                  T *Vx, T *Vy, T *Vz, hipStream_t s) {
+    const int64_t n = (int64_t)dims[0] * dims[1] * dims[2];
+    with_grid(dims, [&](auto G) {
+        using I = decltype(G.p);
+        hipLaunchKernelGGL((k_descend<T, I>), dim3(ew_blocks(n)), dim3(256), 0, s, G, n, (T)tau,
+                           (int)nonneg, U, d, V, Vx, Vy, Vz);
+    });
+}
+
+template <typename T>
+void queue_step(Sums &S, const int32_t dims[3], const T *d) {
+    with_grid(dims, [&](auto G) {
+        using I = decltype(G.p);
+        queue_sums<4>(S, (int64_t)dims[0] * dims[1] * dims[2], FStep<T, I>{G, d});
+    });
+}
+
+template <typename T>
+void queue_dot(Sums &S, int64_t n, const T *a, const T *b) {
+    queue_sums<1>(S, n, FDot<T>{a, b});
+}
+
+template <typename T>
+void queue_gradient(Sums &S, const PlainFields<T> &f, T *g, const T *Atb) {
+    with_grid(f.dims, [&](auto G) {
+        using I = decltype(G.p);
+        queue_sums<2>(S, f.n, FGradient<T, I>{G, f.Ux, f.Uy, f.Uz, f.Wx, f.Wy, f.Wz, f.sx, f.sy,
+                                              f.sz, Atb, f.g2, g});
+    });
+}
+
+template <typename T>
+void queue_lam24(Sums &S, const PlainFields<T> &f) {
+    queue_sums<2>(S, f.n, FLam24<T>{f.Ux, f.Uy, f.Uz, f.Wx, f.Wy, f.Wz, f.sx, f.sy, f.sz});
+}
+
+template <typename T>
+void queue_lam35(Sums &S, int64_t m, const T *Au, const T *b, const T *delta) {
+    queue_sums<2>(S, m, FLam35<T>{Au, b, delta});
+}
+
+template <typename T>
+void queue_shrink(Sums &S, const PlainFields<T> &f, int iso, double beta) {
+    queue_sums<1>(S, f.n, FShrink<T>{f.Ux, f.Uy, f.Uz, f.sx, f.sy, f.sz, (T)beta, iso, f.Wx, f.Wy,
+                                     f.Wz});
+}
+
+template <typename T>
+void queue_update(Sums &S, const PlainFields<T> &f, const T *g, const T *gp, const T *g2p,
+                  const T *dts, const T *U, const T *Up, double mdb, T *d) {
+    with_grid(f.dims, [&](auto G) {
+        using I = decltype(G.p);
+        queue_sums<6>(S, f.n, FUpdate<T, I>{G, f.Ux, f.Uy, f.Uz, f.Wx, f.Wy, f.Wz, f.sx, f.sy,
+                                            f.sz, g, gp, g2p, dts, U, Up, (T)mdb, f.g2, d});
+    });
 }
 
 template <typename T>
 double dot(tv3_ctx *ctx, int64_t n, const T *a, const T *b, hipStream_t s) {
     return reduce_now<1>(ctx, n, FDot<T>{a, b}, s)[0];
-}
-template <typename T>
-std::array<double, 2> lam24(tv3_ctx *ctx, int64_t n, const T *Ux, const T *Uy, const T *Uz,
-                            const T *Wx, const T *Wy, const T *Wz, const T *sx, const T *sy,
-                            const T *sz, T *Vx, T *Vy, T *Vz, hipStream_t s) {
-    return reduce_now<2>(ctx, n, FLam24<T>{Ux, Uy, Uz, Wx, Wy, Wz, sx, sy, sz, Vx, Vy, Vz}, s);
-}
-template <typename T>
-std::array<double, 2> lam35(tv3_ctx *ctx, int64_t m, const T *Au, const T *b, const T *delta,
-                            hipStream_t s) {
-    return reduce_now<2>(ctx, m, FLam35<T>{Au, b, delta}, s);
-}
-template <typename T>
-std::array<double, 2> tau_bb(tv3_ctx *ctx, int64_t n, const T *g, const T *gp, const T *g2,
-                             const T *g2p, const T *uup, double mdb, T *dg, T *dg2,
-                             hipStream_t s) {
-    return reduce_now<2>(ctx, n, FTau<T>{g, gp, g2, g2p, uup, (T)mdb, dg, dg2}, s);
 }
 template <typename T>
 double shrink_host(tv3_ctx *ctx, int64_t n, int iso, const T *Ux, const T *Uy, const T *Uz,
@@ -304,22 +459,12 @@ std::array<double, 2> diff_norm(tv3_ctx *ctx, int64_t n, const T *a, const T *b,
 #define TV3_INST(T)                                                                              \
     template void axpy3<T>(int64_t, T *, double, const T *, const T *, hipStream_t);            \
     template void grad<T>(int64_t, T *, double, const T *, const T *, const T *, hipStream_t);  \
-    template void nonneg<T>(int64_t, T *, hipStream_t);                                         \
     template void scale<T>(int64_t, T *, double, const T *, hipStream_t);                       \
     template void divide<T>(int64_t, T *, double, const T *, hipStream_t);                      \
     template void launch_D<T>(const int32_t *, const T *, T *, T *, T *, hipStream_t);          \
     template void launch_Dt<T>(const int32_t *, const T *, const T *, const T *, T *,           \
                                hipStream_t);                                                    \
     template double dot<T>(tv3_ctx *, int64_t, const T *, const T *, hipStream_t);              \
-    template std::array<double, 2> lam24<T>(tv3_ctx *, int64_t, const T *, const T *,           \
-                                            const T *, const T *, const T *, const T *,         \
-                                            const T *, const T *, const T *, T *, T *, T *,     \
-                                            hipStream_t);                                       \
-    template std::array<double, 2> lam35<T>(tv3_ctx *, int64_t, const T *, const T *,           \
-                                            const T *, hipStream_t);                            \
-    template std::array<double, 2> tau_bb<T>(tv3_ctx *, int64_t, const T *, const T *,          \
-                                             const T *, const T *, const T *, double, T *, T *, \
-                                             hipStream_t);                                      \
     template double shrink_host<T>(tv3_ctx *, int64_t, int, const T *, const T *, const T *,    \
                                    const T *, const T *, const T *, double, T *, T *, T *,      \
                                    hipStream_t);                                                \
@@ -329,7 +474,17 @@ std::array<double, 2> diff_norm(tv3_ctx *ctx, int64_t n, const T *a, const T *b,
     template double mlp_delta<T>(tv3_ctx *, int64_t, const T *, const T *, double, T *,         \
                                  hipStream_t);                                                  \
     template std::array<double, 2> diff_norm<T>(tv3_ctx *, int64_t, const T *, const T *,       \
-                                                hipStream_t);
+                                                hipStream_t);                                   \
+    template void descend_step<T>(const int32_t *, double, bool, const T *, const T *, T *, T *, \
+                                  T *, T *, hipStream_t);                                       \
+    template void queue_step<T>(Sums &, const int32_t *, const T *);                            \
+    template void queue_dot<T>(Sums &, int64_t, const T *, const T *);                          \
+    template void queue_gradient<T>(Sums &, const PlainFields<T> &, T *, const T *);            \
+    template void queue_lam24<T>(Sums &, const PlainFields<T> &);                               \
+    template void queue_lam35<T>(Sums &, int64_t, const T *, const T *, const T *);             \
+    template void queue_shrink<T>(Sums &, const PlainFields<T> &, int, double);                 \
+    template void queue_update<T>(Sums &, const PlainFields<T> &, const T *, const T *,         \
+                                  const T *, const T *, const T *, const T *, double, T *);
 
 TV3_INST(float)
 TV3_INST(double)

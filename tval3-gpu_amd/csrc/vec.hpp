@@ -40,23 +40,58 @@ __device__ __forceinline__ void block_sum_store(double (&acc)[K], double *partia
     block_sum_store_at<K, NW>(acc, partials, nblk, (int)blockIdx.x);
 }
 
+// Sums over items, queued as kernels that leave FP64 block partials (at most
+// kSumBlocks per sum) and fetched together: one copy and one wait for all of
+// them; the partials are added in block order on the host.
+constexpr int kSumBlocks = 1024, kSumMax = 16;
+struct Sums {
+    tv3_ctx *ctx;
+    hipStream_t s;
+    size_t used = 0;
+    int count = 0;
+    int blocks[kSumMax] = {};
+    double value[kSumMax] = {};
+    const double *fetch();       // the sums in the order queued; waits for the stream
+};
+
+// the volume-sized fields the plain loop's fused steps share
+template <typename T> struct PlainFields {
+    const int32_t *dims;
+    int64_t n;
+    const T *Ux, *Uy, *Uz;       // D U
+    T *Wx, *Wy, *Wz;
+    const T *sx, *sy, *sz;       // sigma
+    T *g2;                       // D^T (D U - W)
+};
+
+// V = U - tau d (clamped at 0 with nonneg) and its differences D V
+template <typename T>
+void descend_step(const int32_t dims[3], double tau, bool nonneg, const T *U, const T *d, T *V,
+                  T *Vx, T *Vy, T *Vz, hipStream_t s);
+// |D d|^2 along x, y, z and |d|^2
+template <typename T> void queue_step(Sums &S, const int32_t dims[3], const T *d);
+template <typename T> void queue_dot(Sums &S, int64_t n, const T *a, const T *b);
+// lam2, lam4; g2; g -= Atb unless g is NULL
+template <typename T>
+void queue_gradient(Sums &S, const PlainFields<T> &f, T *g, const T *Atb);
+// lam2, lam4
+template <typename T> void queue_lam24(Sums &S, const PlainFields<T> &f);
+// lam3, lam5
+template <typename T>
+void queue_lam35(Sums &S, int64_t m, const T *Au, const T *b, const T *delta);
+// W; lam1
+template <typename T> void queue_shrink(Sums &S, const PlainFields<T> &f, int iso, double beta);
+// g2, d; lam2, lam4, |d|^2, |U - Up|^2, |Up|^2, <U - Up, change of the gradient>
+template <typename T>
+void queue_update(Sums &S, const PlainFields<T> &f, const T *g, const T *gp, const T *g2p,
+                  const T *dts, const T *U, const T *Up, double mdb, T *d);
+
 template <typename T> void axpy3(int64_t n, T *z, double a, const T *x, const T *y, hipStream_t s);
 template <typename T>
 void grad(int64_t n, T *d, double a, const T *g, const T *g2, const T *dts, hipStream_t s);
-template <typename T> void nonneg(int64_t n, T *u, hipStream_t s);
 template <typename T> void scale(int64_t n, T *y, double a, const T *x, hipStream_t s);
 template <typename T> void divide(int64_t n, T *y, double a, const T *x, hipStream_t s);
 template <typename T> double dot(tv3_ctx *ctx, int64_t n, const T *a, const T *b, hipStream_t s);
-template <typename T>
-std::array<double, 2> lam24(tv3_ctx *ctx, int64_t n, const T *Ux, const T *Uy, const T *Uz,
-                            const T *Wx, const T *Wy, const T *Wz, const T *sx, const T *sy,
-                            const T *sz, T *Vx, T *Vy, T *Vz, hipStream_t s);
-template <typename T>
-std::array<double, 2> lam35(tv3_ctx *ctx, int64_t m, const T *Au, const T *b, const T *delta,
-                            hipStream_t s);
-template <typename T>
-std::array<double, 2> tau_bb(tv3_ctx *ctx, int64_t n, const T *g, const T *gp, const T *g2,
-                             const T *g2p, const T *uup, double mdb, T *dg, T *dg2, hipStream_t s);
 template <typename T>
 double mlp_sigma(tv3_ctx *ctx, int64_t n, const T *Ux, const T *Uy, const T *Uz, const T *Wx,
                  const T *Wy, const T *Wz, double beta, T *sx, T *sy, T *sz, hipStream_t s);
