@@ -20,8 +20,8 @@
 //    computed and rounded as by one kernel per operation; an iteration
 //    without backtracking waits for the device twice, and the previous
 //    iterate is kept by exchanging buffers;
-//  * every work vector is allocated once per solve (the reference allocates
-//    and frees 3 n-vectors inside get_g/update_g/update_W/update_mlp);
+//  * the work vectors stay with the context (the reference allocates and
+//    frees 3 n-vectors inside get_g/update_g/update_W/update_mlp);
 //  * the A^T-skip heuristic (:398-468) leaves a skipped g as A^T(last Au)
 //    - Atb; the reference subtracts Atb a second time from the stale g
 //    (:463-467 then :565-567).
@@ -45,7 +45,6 @@ struct PlainState {
     int32_t dims[3];
     int64_t n, m;
     double mu, beta, muDbeta, f, lam1, lam2, lam3, lam4, lam5;
-    DevBuf<T> pool;
     T *delta, *sx, *sy, *sz, *dU, *dUx, *dUy, *dUz, *Wx, *Wy, *Wz, *Atb, *dAu, *d, *dg, *dg2, *Ad,
         *DtsAtd, *rcdU, *bs, *lastAu, *dlast;
     // the iterate and what follows from it (0), and the previous one's (1)
@@ -65,8 +64,9 @@ struct PlainState {
         const size_t cn = sizeof(nv) / sizeof(nv[0]), cm = sizeof(mv) / sizeof(mv[0]);
         // pad each vector to 256 bytes
         auto pad = [](int64_t k) { return (k + 63) / 64 * 64; };
-        pool.alloc(cn * pad(n) + cm * pad(m));
-        T *p = pool.p;
+        const size_t need = sizeof(T) * (cn * pad(n) + cm * pad(m));
+        if (ctx->plain_ws.bytes() < need) ctx->plain_ws.alloc(need);
+        T *p = reinterpret_cast<T *>(ctx->plain_ws.p);
         for (size_t k = 0; k < cn; ++k) { *nv[k] = p; p += pad(n); }
         for (size_t k = 0; k < cm; ++k) { *mv[k] = p; p += pad(m); }
         TV3_HIP(hipMemsetAsync(DtsAtd, 0, sizeof(T) * 4 * pad(n), s));

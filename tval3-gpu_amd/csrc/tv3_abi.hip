@@ -160,27 +160,26 @@ static tv3_status solve_host(tv3_ctx *ctx, tv3_op *op, const tv3_opts *opts,
         TV3_REQUIRE(n == op->n, TV3_E_SHAPE, "length of U must equal the columns of A");
         set_device(ctx);
         hipStream_t s = ctx->stream;
-        DevBuf<T> bd(op->m), Ud(n), Utd;
-        TV3_HIP(hipMemcpyAsync(bd.p, b, sizeof(T) * op->m, hipMemcpyHostToDevice, s));
+        auto pad = [](int64_t k) { return (k + 63) / 64 * 64; };
+        const size_t need = sizeof(T) * (pad(op->m) + pad(n) + (Ut ? n : 0));
+        if (ctx->host_ws.bytes() < need) ctx->host_ws.alloc(need);
+        T *bd = reinterpret_cast<T *>(ctx->host_ws.p), *Ud = bd + pad(op->m),
+          *Utd = Ut ? Ud + pad(n) : nullptr;
+        TV3_HIP(hipMemcpyAsync(bd, b, sizeof(T) * op->m, hipMemcpyHostToDevice, s));
         if (opts->warm_start)
-            TV3_HIP(hipMemcpyAsync(Ud.p, U, sizeof(T) * n, hipMemcpyHostToDevice, s));
-        if (Ut) {
-            Utd.alloc(n);
-            TV3_HIP(hipMemcpyAsync(Utd.p, Ut, sizeof(T) * n, hipMemcpyHostToDevice, s));
-        }
+            TV3_HIP(hipMemcpyAsync(Ud, U, sizeof(T) * n, hipMemcpyHostToDevice, s));
+        if (Ut) TV3_HIP(hipMemcpyAsync(Utd, Ut, sizeof(T) * n, hipMemcpyHostToDevice, s));
         std::memset(info, 0, sizeof(*info));
         if (hist) hist->count = 0;
         if constexpr (std::is_same<T, float>::value) {
             if (opts->solver == TV3_SOLVER_FUSED)
-                solve_fused(ctx, op, *opts, dims, bd.p, Ud.p, Ut ? Utd.p : nullptr, info, hist);
+                solve_fused(ctx, op, *opts, dims, bd, Ud, Utd, info, hist);
             else
-                solve_plain<float>(ctx, op, *opts, dims, bd.p, Ud.p, Ut ? Utd.p : nullptr, info,
-                                   hist);
+                solve_plain<float>(ctx, op, *opts, dims, bd, Ud, Utd, info, hist);
         } else {
-            solve_plain<double>(ctx, op, *opts, dims, bd.p, Ud.p, Ut ? Utd.p : nullptr, info,
-                                hist);
+            solve_plain<double>(ctx, op, *opts, dims, bd, Ud, Utd, info, hist);
         }
-        TV3_HIP(hipMemcpyAsync(U, Ud.p, sizeof(T) * n, hipMemcpyDeviceToHost, s));
+        TV3_HIP(hipMemcpyAsync(U, Ud, sizeof(T) * n, hipMemcpyDeviceToHost, s));
         TV3_HIP(hipStreamSynchronize(s));
     });
     if (info) {
@@ -241,7 +240,8 @@ void tv3_ctx_destroy(tv3_ctx *ctx) {
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
     ctx->batch_session.reset();
-    ctx->red_partials.release();
+    ctx->plain_ws.release();
+    ctx->host_ws.release();
     ctx->scratch.release();
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;

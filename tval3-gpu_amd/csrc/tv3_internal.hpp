@@ -376,9 +376,11 @@ struct tv3_ctx {
     std::string err;
     int num_cus = 256;
     size_t lds_per_block = 65536;   // largest LDS allocation of one workgroup
-    // reduction scratch
-    tv3::DevBuf<double> red_partials;
-    tv3::PinnedBuf<double> red_host;
+    tv3::PinnedBuf<double> red_host;   // block partials of the sums (vec.hpp)
+    // The vectors of a plain solve and the device copies of a host solve's b, U
+    // and U_true, grown to the largest solve so far (a solve waits for its
+    // stream before it returns, and a context serves one host thread)
+    tv3::DevBuf<uint8_t> plain_ws, host_ws;
     tv3::DevBuf<uint8_t> scratch;   // general workspace (grown on demand)
     std::unique_ptr<tv3::CtxSession> batch_session;   // the last batched solve, for reuse
 };

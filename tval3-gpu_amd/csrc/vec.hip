@@ -286,48 +286,60 @@ template <typename T, typename I> struct FUpdate {
     }
 };
 
+// Block partials of K sums, a block's K values side by side: they go straight
+// to pinned host memory (one line a block, so a fetch waits for the kernel
+// only: no copy behind it).
 template <int K, typename F>
 __global__ __launch_bounds__(256) void k_reduce(int64_t n, F f, double *partials) {
+    __shared__ double sh[K][4];
     double acc[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) acc[k] = 0.0;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
         f(i, acc);
-    block_sum_store<K>(acc, partials, gridDim.x);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const double v = wave_sum(acc[k]);
+        if (lane == 0) sh[k][wave] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x < K) {
+        const double *w = sh[threadIdx.x];
+        partials[(int64_t)blockIdx.x * K + threadIdx.x] = (w[0] + w[1]) + (w[2] + w[3]);
+    }
 }
 
-// launches the block partials of K sums over n items into slot s of the
-// context's buffer
+// queues the block partials of K sums over n items
 template <int K, typename F>
 static void queue_sums(Sums &S, int64_t n, const F &f) {
     int64_t nb = (n + 255) / 256;
     if (nb > kSumBlocks) nb = kSumBlocks;
     if (nb < 1) nb = 1;
     tv3_ctx *ctx = S.ctx;
-    const size_t cap = (size_t)kSumMax * kSumBlocks;
-    if (ctx->red_partials.n < cap) ctx->red_partials.alloc(cap);
-    ctx->red_host.alloc(cap);
+    ctx->red_host.alloc((size_t)kSumMax * kSumBlocks);
     TV3_REQUIRE(S.count + K <= kSumMax, TV3_E_INTERNAL, "too many sums at once");
     hipLaunchKernelGGL((k_reduce<K, F>), dim3((unsigned)nb), dim3(256), 0, S.s, n, f,
-                       ctx->red_partials.p + S.used);
-    for (int k = 0; k < K; ++k) S.blocks[S.count++] = (int)nb;
+                       ctx->red_host.p + S.used);
+    S.group[S.groups++] = {K, (int)nb};
+    S.count += K;
     S.used += (size_t)K * nb;
 }
 
 const double *Sums::fetch() {
     TV3_HIP(hipGetLastError());
-    TV3_HIP(hipMemcpyAsync(ctx->red_host.p, ctx->red_partials.p, used * sizeof(double),
-                           hipMemcpyDeviceToHost, s));
     TV3_HIP(hipStreamSynchronize(s));
     const double *h = ctx->red_host.p;
-    for (int k = 0; k < count; ++k) {
-        double t = 0.0;
-        for (int b = 0; b < blocks[k]; ++b) t += h[b];
-        h += blocks[k];
-        value[k] = t;
+    double *out = value;
+    for (int g = 0; g < groups; ++g) {
+        const int K = group[g].sums;
+        for (int k = 0; k < K; ++k) out[k] = 0.0;
+        for (int b = 0; b < group[g].blocks; ++b, h += K)
+            for (int k = 0; k < K; ++k) out[k] += h[k];
+        out += K;
     }
     used = 0;
-    count = 0;
+    count = groups = 0;
     return value;
 }
 

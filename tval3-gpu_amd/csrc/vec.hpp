@@ -41,15 +41,17 @@ __device__ __forceinline__ void block_sum_store(double (&acc)[K], double *partia
 }
 
 // Sums over items, queued as kernels that leave FP64 block partials (at most
-// kSumBlocks per sum) and fetched together: one copy and one wait for all of
-// them; the partials are added in block order on the host.
+// kSumBlocks per sum) in pinned host memory, and fetched with one wait for
+// all of them; the partials are added in block order on the host.
 constexpr int kSumBlocks = 1024, kSumMax = 16;
 struct Sums {
     tv3_ctx *ctx;
     hipStream_t s;
     size_t used = 0;
-    int count = 0;
-    int blocks[kSumMax] = {};
+    int count = 0, groups = 0;
+    struct Group {
+        int sums, blocks;
+    } group[kSumMax] = {};
     double value[kSumMax] = {};
     const double *fetch();       // the sums in the order queued; waits for the stream
 };
