@@ -18,8 +18,10 @@
 //    the gradient parts with lam2, lam4; shrinkage; the update of W's
 //    consequences with every sum the next decision needs), each element
 //    computed and rounded as by one kernel per operation; an iteration
-//    without backtracking waits for the device twice, and the previous
-//    iterate is kept by exchanging buffers;
+//    without backtracking waits for the device once, and the previous iterate
+//    is kept by exchanging buffers (64^3 voxels, 65,536 rays: FIGURES an
+//    iteration against 270 us with one kernel per operation and a wait per
+//    inner product);
 //  * the work vectors stay with the context (the reference allocates and
 //    frees 3 n-vectors inside get_g/update_g/update_W/update_mlp);
 //  * the A^T-skip heuristic (:398-468) leaves a skipped g as A^T(last Au)
@@ -27,8 +29,10 @@
 //    (:463-467 then :565-567).
 // This path is the parity anchor and the baseline the fused path is
 // measured against.
-#include <chrono>
 #include <cmath>
+#include <cstring>
+#include <limits>
+#include <utility>
 
 #include "vec.hpp"
 
@@ -45,10 +49,12 @@ struct PlainState {
     int32_t dims[3];
     int64_t n, m;
     double mu, beta, muDbeta, f, lam1, lam2, lam3, lam4, lam5;
-    T *delta, *sx, *sy, *sz, *dU, *dUx, *dUy, *dUz, *Wx, *Wy, *Wz, *Atb, *dAu, *d, *dg, *dg2, *Ad,
-        *DtsAtd, *rcdU, *bs, *lastAu, *dlast;
+    T *delta, *sx, *sy, *sz, *dU, *dUx, *dUy, *dUz, *Atb, *dAu, *dg, *dg2, *Ad, *DtsAtd, *rcdU,
+        *bs, *lastAu, *dlast;
     // the iterate and what follows from it (0), and the previous one's (1)
     T *U[2], *Ux[2], *Uy[2], *Uz[2], *g[2], *g2[2], *Au[2];
+    // W, D^T (DU - W) for it and the direction: in use (0; g2[0]) and next
+    T *Wx[2], *Wy[2], *Wz[2], *d[2], *g2_next;
     double dd = 0, uu = 0, upup = 0, ug = 0;   // |d|^2, |U - Up|^2, |Up|^2, <U - Up, dgrad>
     int64_t nN = 0, nT = 0;
     int cur_init = 0;        // A^T-skip state (:155-157)
@@ -57,8 +63,8 @@ struct PlainState {
 
     void alloc() {
         // DtsAtd, sigma and delta start at zero (:1128-1139)
-        T **nv[] = {&DtsAtd, &sx, &sy, &sz, &dU, &dUx, &dUy, &dUz, &Wx, &Wy, &Wz, &Atb, &d, &dg,
-                    &dg2, &rcdU, &U[0], &U[1], &Ux[0], &Ux[1], &Uy[0], &Uy[1], &Uz[0], &Uz[1],
+        T **nv[] = {&DtsAtd, &sx, &sy, &sz, &dU, &dUx, &dUy, &dUz, &Wx[0], &Wx[1], &Wy[0],
+                    &Wy[1], &Wz[0], &Wz[1], &Atb, &d[0], &d[1], &dg, &dg2, &g2_next, &rcdU, &U[0], &U[1], &Ux[0], &Ux[1], &Uy[0], &Uy[1], &Uz[0], &Uz[1],
                     &g[0], &g[1], &g2[0], &g2[1]};
         T **mv[] = {&delta, &dAu, &Ad, &bs, &lastAu, &dlast, &Au[0], &Au[1]};
         const size_t cn = sizeof(nv) / sizeof(nv[0]), cm = sizeof(mv) / sizeof(mv[0]);
@@ -75,7 +81,7 @@ struct PlainState {
         TV3_HIP(hipMemsetAsync(lastAu, 0, sizeof(T) * m, s));
     }
     PlainFields<T> fields() {
-        return {dims, n, Ux[0], Uy[0], Uz[0], Wx, Wy, Wz, sx, sy, sz, g2[0]};
+        return {dims, n, Ux[0], Uy[0], Uz[0], Wx[0], Wy[0], Wz[0], sx, sy, sz, g2[0]};
     }
     // the iterate becomes the previous one
     void turn() {
@@ -94,17 +100,18 @@ struct PlainState {
         lam2 = v[0]; lam4 = v[1]; lam3 = v[2]; lam5 = v[3];
         f = fval();
     }
-    // :366-572; force: the initial and the fallback call (:1148, :880)
-    void get_g(bool force) {
+    // :366-572; force: the initial and the fallback call (:1148, :880).  With
+    // ahead the sums of update_W are queued behind and returned too.
+    const double *get_g(Sums &S, bool force, bool ahead) {
         A(false, U[0], Au[0]);
         bool mul = true;
         if (o->skipMulRatio != 0.0) {
             // relative change of Au since the last A^T product (:398-412)
             axpy3<T>(m, dlast, -1.0, lastAu, Au[0], s);
-            Sums S{ctx, s};
-            queue_dot<T>(S, m, dlast, dlast);
-            queue_dot<T>(S, m, Au[0], Au[0]);
-            const double *v = S.fetch();
+            Sums R{ctx, s};
+            queue_dot<T>(R, m, dlast, dlast);
+            queue_dot<T>(R, m, Au[0], Au[0]);
+            const double *v = R.fetch();
             const double rel = std::sqrt(v[0]) / std::sqrt(v[1]);
             if (force) {
                 cur_skip = 0.0;
@@ -123,26 +130,28 @@ struct PlainState {
         }
         if (mul) A(true, Au[0], g[0]);
         else copy(g[0], g[1], n);          // g stays as it was
-        Sums S{ctx, s};
         queue_gradient<T>(S, fields(), mul ? g[0] : nullptr, Atb);
         queue_lam35<T>(S, m, Au[0], bs, delta);
         last_mul = mul;
-        set_f(S.fetch());
+        if (ahead) queue_W(S);
+        const double *v = S.fetch();
+        set_f(v);
+        return v + 4;
     }
     // exact step length along d (:577-640); leaves |d|^2
     double first_tau() {
-        A(false, d, Ad);
+        A(false, d[0], Ad);
         Sums S{ctx, s};
-        queue_step<T>(S, dims, d);
+        queue_step<T>(S, dims, d[0]);
         queue_dot<T>(S, m, Ad, Ad);
         const double *v = S.fetch();
         const double dDd = v[0] + v[1] + v[2];
         dd = v[3];
         return std::fabs(dd / (dDd + muDbeta * v[4]));
     }
-    void descend(double tau, bool force) {
-        descend_step<T>(dims, tau, o->nonneg != 0, U[1], d, U[0], Ux[0], Uy[0], Uz[0], s);
-        get_g(force);
+    const double *descend(Sums &S, double tau, bool force, bool ahead) {
+        descend_step<T>(dims, tau, o->nonneg != 0, U[1], d[0], U[0], Ux[0], Uy[0], Uz[0], s);
+        return get_g(S, force, ahead);
     }
     void update_g(double alpha) {
         axpy3<T>(n, g[0], alpha, dg, g[1], s);
@@ -166,38 +175,63 @@ struct PlainState {
         axpy3<T>(n, dUy, -1.0, Uy[1], Uy[0], s);
         axpy3<T>(n, dUz, -1.0, Uz[1], Uz[0], s);
     }
-    void gradient() { grad<T>(n, d, muDbeta, g[0], g2[0], DtsAtd, s); }
+    void gradient() { grad<T>(n, d[0], muDbeta, g[0], g2[0], DtsAtd, s); }
     // W, then all that follows from it: update_W (:965-1029), the direction
-    // (:896-919), and the sums of the next step length and the stopping test
-    void update_W() {
+    // (:896-919), and the sums of the next step length and the stopping test.
+    // They go to the next buffers, so they can be queued before the line
+    // search of the trial is decided (nearly every trial is accepted; an
+    // iteration then waits for the device once).
+    void queue_W(Sums &S) {
+        PlainFields<T> F = fields();
+        F.Wx = Wx[1]; F.Wy = Wy[1]; F.Wz = Wz[1];
+        F.g2 = g2_next;
+        queue_shrink<T>(S, F, o->tv_mode == TV3_TV_ISO, beta);
+        queue_update<T>(S, F, g[0], g[1], g2[1], DtsAtd, U[0], U[1], muDbeta, d[1]);
+    }
+    void take_W(const double *v) {
         f -= (lam1 + beta / 2 * lam2 - lam4);
-        Sums S{ctx, s};
-        queue_shrink<T>(S, fields(), o->tv_mode == TV3_TV_ISO, beta);
-        queue_update<T>(S, fields(), g[0], g[1], g2[1], DtsAtd, U[0], U[1], muDbeta, d);
-        const double *v = S.fetch();
         lam1 = v[0]; lam2 = v[1]; lam4 = v[2];
         dd = v[3]; uu = v[4]; upup = v[5]; ug = v[6];
         f += (lam1 + beta / 2 * lam2 - lam4);
+        for (auto *w : {Wx, Wy, Wz, d}) std::swap(w[0], w[1]);
+        std::swap(g2[0], g2_next);
     }
     void update_mlp() {
         f += (lam4 + lam5);
-        lam4 = mlp_sigma<T>(ctx, n, Ux[0], Uy[0], Uz[0], Wx, Wy, Wz, beta, sx, sy, sz, s);
+        lam4 = mlp_sigma<T>(ctx, n, Ux[0], Uy[0], Uz[0], Wx[0], Wy[0], Wz[0], beta, sx, sy, sz, s);
         lam5 = mlp_delta<T>(ctx, m, Au[0], bs, mu, delta, s);
         f -= (lam4 + lam5);
     }
 };
 
-// scaleb (3d/tval3_gpu_3d.cpp:225-266) on the host copy of b
+// scaleb (3d/tval3_gpu_3d.cpp:225-266) on a host copy of b: the entries of
+// least and largest magnitude, the first on ties.  Magnitudes are compared as
+// the integers of their bits, which order alike (a loop the compiler can
+// vectorise); the largest tells whether any entry is NaN or Inf.
 template <typename T>
-double scale_factor_of(const std::vector<T> &b) {
-    if (b.empty()) return 1.0;
-    T bmin = b[0], bmax = bmin, amin = std::fabs(bmin), amax = amin;
-    for (T v : b) {
-        T a = std::fabs(v);
-        if (a < amin) { bmin = v; amin = a; }
-        if (a > amax) { bmax = v; amax = a; }
+double scale_factor_of(const T *b, int64_t m) {
+    using I = std::conditional_t<sizeof(T) == 4, int32_t, int64_t>;
+    const I mask = std::numeric_limits<I>::max();
+    auto bits = [mask](T v) {
+        I i;
+        std::memcpy(&i, &v, sizeof(T));
+        return (I)(i & mask);
+    };
+    if (m == 0) return 1.0;
+    I lo = mask, hi = 0;
+    for (int64_t k = 0; k < m; ++k) {
+        const I i = bits(b[k]);
+        lo = i < lo ? i : lo;
+        hi = i > hi ? i : hi;
     }
-    T dif = std::fabs(bmax - bmin);
+    TV3_REQUIRE(hi < bits(std::numeric_limits<T>::infinity()), TV3_E_NONFINITE,
+                "b holds NaN or Inf");
+    auto first = [&](I want) {
+        int64_t k = 0;
+        while (bits(b[k]) != want) ++k;
+        return b[k];
+    };
+    const T dif = std::fabs(first(hi) - first(lo));
     T s = 1;
     if (dif < (T)0.5) s = (T)0.5 / dif;
     else if (dif > (T)1.5) s = (T)1.5 / dif;
@@ -208,7 +242,8 @@ double scale_factor_of(const std::vector<T> &b) {
 
 template <typename T>
 void solve_plain(tv3_ctx *ctx, tv3_op *op, const tv3_opts &o, const int32_t dims[3],
-                 const T *b_dev, T *U, const T *Ut_dev, tv3_info *info, tv3_history *hist) {
+                 const T *b_dev, T *U, const T *Ut_dev, tv3_info *info, tv3_history *hist,
+                 const T *b_host) {
     hipStream_t s = ctx->stream;
     PlainState<T> S;
     S.ctx = ctx; S.op = op; S.o = &o; S.s = s;
@@ -223,12 +258,15 @@ void solve_plain(tv3_ctx *ctx, tv3_op *op, const tv3_opts &o, const int32_t dims
     TV3_HIP(hipEventCreate(&evl0)); TV3_HIP(hipEventCreate(&evl1));
     TV3_HIP(hipEventRecord(ev0, s));
 
-    // b: scale on the device by the factor found on a host copy (:1122-1124)
-    std::vector<T> bh(m);
-    TV3_HIP(hipMemcpyAsync(bh.data(), b_dev, sizeof(T) * m, hipMemcpyDeviceToHost, s));
-    TV3_HIP(hipStreamSynchronize(s));
-    for (T v : bh) TV3_REQUIRE(std::isfinite((double)v), TV3_E_NONFINITE, "b holds NaN or Inf");
-    double scl = scale_factor_of<T>(bh);
+    // b: scale on the device by the factor found on the host (:1122-1124)
+    std::vector<T> bh;
+    if (!b_host) {
+        bh.resize(m);
+        TV3_HIP(hipMemcpyAsync(bh.data(), b_dev, sizeof(T) * m, hipMemcpyDeviceToHost, s));
+        TV3_HIP(hipStreamSynchronize(s));
+        b_host = bh.data();
+    }
+    const double scl = scale_factor_of<T>(b_host, m);
     scale<T>(m, S.bs, scl, b_dev, s);
 
     S.A(true, S.bs, S.Atb);
@@ -243,8 +281,8 @@ void solve_plain(tv3_ctx *ctx, tv3_op *op, const tv3_opts &o, const int32_t dims
         Sums L{ctx, s};
         queue_shrink<T>(L, S.fields(), o.tv_mode == TV3_TV_ISO, S.beta);
         S.lam1 = L.fetch()[0];
+        S.get_g(L, true, false);
     }
-    S.get_g(true);
     S.gradient();
 
     double Q = 1, Qp, C = S.f, gam = o.gam;
@@ -258,7 +296,8 @@ void solve_plain(tv3_ctx *ctx, tv3_op *op, const tv3_opts &o, const int32_t dims
         while (total < o.maxit) {
             double tau = fst ? S.first_tau() : std::fabs(S.uu / S.ug);
             S.turn();
-            S.descend(tau, false);
+            Sums sums{ctx, s};
+            const double *next_W = S.descend(sums, tau, false, true);
             double alpha = 1.0;
             const double f_trial = S.f;
             double c_armij = S.dd * tau * o.c * S.beta;
@@ -269,7 +308,7 @@ void solve_plain(tv3_ctx *ctx, tv3_op *op, const tv3_opts &o, const int32_t dims
                     if (cnt == 5) {
                         gam *= o.rate_gam;
                         tau = S.first_tau();
-                        S.descend(tau, true);
+                        S.descend(sums, tau, true, false);
                         cnt = 6;
                         ++fallbacks;
                         break;
@@ -279,8 +318,10 @@ void solve_plain(tv3_ctx *ctx, tv3_op *op, const tv3_opts &o, const int32_t dims
                     ++cnt;
                 }
                 backtracks += cnt > 5 ? 5 : cnt;
+                S.queue_W(sums);           // the queued one was the trial's
+                next_W = sums.fetch();
             }
-            S.update_W();
+            S.take_W(next_W);
             Qp = Q; Q = gam * Qp + 1; C = (gam * Qp * C + S.f) / Q;
             ++total;
             nrmup = std::sqrt(S.upup);
@@ -312,7 +353,7 @@ void solve_plain(tv3_ctx *ctx, tv3_op *op, const tv3_opts &o, const int32_t dims
         if (S.mu > o.mu) S.mu = o.mu;
         S.muDbeta = S.mu / S.beta;
         S.f = S.fval();
-        scale<T>(n, S.DtsAtd, beta0 / S.beta, S.d, s);
+        scale<T>(n, S.DtsAtd, beta0 / S.beta, S.d[0], s);
         S.gradient();
         gam = o.gam; Q = 1; C = S.f;
     }
@@ -343,9 +384,10 @@ void solve_plain(tv3_ctx *ctx, tv3_op *op, const tv3_opts &o, const int32_t dims
 }
 
 template void solve_plain<float>(tv3_ctx *, tv3_op *, const tv3_opts &, const int32_t *,
-                                 const float *, float *, const float *, tv3_info *, tv3_history *);
+                                 const float *, float *, const float *, tv3_info *, tv3_history *,
+                                 const float *);
 template void solve_plain<double>(tv3_ctx *, tv3_op *, const tv3_opts &, const int32_t *,
                                   const double *, double *, const double *, tv3_info *,
-                                  tv3_history *);
+                                  tv3_history *, const double *);
 
 }  // namespace tv3

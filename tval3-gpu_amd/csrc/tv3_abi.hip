@@ -175,9 +175,9 @@ static tv3_status solve_host(tv3_ctx *ctx, tv3_op *op, const tv3_opts *opts,
             if (opts->solver == TV3_SOLVER_FUSED)
                 solve_fused(ctx, op, *opts, dims, bd, Ud, Utd, info, hist);
             else
-                solve_plain<float>(ctx, op, *opts, dims, bd, Ud, Utd, info, hist);
+                solve_plain<float>(ctx, op, *opts, dims, bd, Ud, Utd, info, hist, b);
         } else {
-            solve_plain<double>(ctx, op, *opts, dims, bd, Ud, Utd, info, hist);
+            solve_plain<double>(ctx, op, *opts, dims, bd, Ud, Utd, info, hist, b);
         }
         TV3_HIP(hipMemcpyAsync(U, Ud, sizeof(T) * n, hipMemcpyDeviceToHost, s));
         TV3_HIP(hipStreamSynchronize(s));
@@ -614,7 +614,7 @@ static void solve_device_impl(tv3_ctx *ctx, tv3_op *op, const tv3_opts *opts,
     if (opts->solver == TV3_SOLVER_FUSED)
         solve_fused(ctx, op, *opts, dims, b, U, Ut, info, hist);
     else
-        solve_plain<float>(ctx, op, *opts, dims, b, U, Ut, info, hist);
+        solve_plain<float>(ctx, op, *opts, dims, b, U, Ut, info, hist, nullptr);
 }
 
 tv3_status tv3_solve_device(tv3_ctx *ctx, tv3_op *op, const tv3_opts *opts, const int32_t dims[3],

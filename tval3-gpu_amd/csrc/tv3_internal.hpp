@@ -531,9 +531,11 @@ void permute_gather(const float *in, const int32_t *map, float *out, int64_t n, 
 void permute_scatter(const float *in, const int32_t *map, float *out, int64_t n, hipStream_t s);
 
 // solvers
+// b_host: b in host memory where the caller has it there (else NULL)
 template <typename T>
 void solve_plain(tv3_ctx *ctx, tv3_op *op, const tv3_opts &o, const int32_t dims[3],
-                 const T *b_dev, T *U_dev, const T *Ut_dev, tv3_info *info, tv3_history *hist);
+                 const T *b_dev, T *U_dev, const T *Ut_dev, tv3_info *info, tv3_history *hist,
+                 const T *b_host);
 void solve_fused(tv3_ctx *ctx, tv3_op *op, const tv3_opts &o, const int32_t dims[3],
                  const float *b_dev, float *U_dev, const float *Ut_dev, tv3_info *info,
                  tv3_history *hist);
