@@ -31,6 +31,13 @@
 // one chunk ahead.  The S partial tiles
 // go to a row-major scratch; a second kernel sums them in a fixed order,
 // subtracts, and writes Y column-major through an LDS transpose.
+// Bound by reading M (and R x 64 partial sums per slice, written and read):
+// 4096 x 16384, 64 columns, 132 -> 83 us for A X and A^T R together (M twice,
+// 268 MB: 3.2 TB/s; the products alone 31-34 us each, 4.2 TB/s).  Converting X
+// once per product into operand order (no conversion and one barrier here, a
+// launch more) took 81 us, but 2-4 us more at 2048 x 8192 and below; M two
+// chunks ahead at one workgroup a CU, workgroups of one XCD on the same slices
+// of K: no change.
 //
 // MFMA operand layout (v_mfma_f32_32x32x16_bf16, checked on the device):
 // lane l supplies A[l % 32][8 (l / 32) + e] and B[8 (l / 32) + e][l % 32],
@@ -55,7 +62,7 @@ __device__ __forceinline__ uint16_t bf16_rne(float x) {
     return (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
 }
 
-__global__ __launch_bounds__(512) void k_gemm_rhs(const uint16_t *__restrict__ M,
+__global__ __launch_bounds__(512, 4) void k_gemm_rhs(const uint16_t *__restrict__ M,
                                                   int64_t R, int64_t K, int S,
                                                   const float *__restrict__ X, int64_t ldx,
                                                   int G, float *__restrict__ part,
@@ -77,126 +84,140 @@ __global__ __launch_bounds__(512) void k_gemm_rhs(const uint16_t *__restrict__ M
     const int xc = t >> 3, xk = (t & 7) * 8;
     const float *xcol = X + (int64_t)(xc < G ? xc : G - 1) * ldx + xk;
     const float xon = xc < G ? 1.f : 0.f;
-    f32x16 acc0 = {}, acc1 = {};
-    // Chunk c's operands are requested one chunk ahead: while chunk c is
-    // converted and multiplied, chunk c + 1's M and X loads are in flight.
-    // Two register sets, unrolled by two, so no copy ties the wait for the
-    // next chunk's loads to the current chunk's work.
+    f32x16 tot0 = {}, tot1 = {};
+    // The next chunk's operands are requested while the current one is
+    // multiplied: X's before the products, an operand of M as soon as its last
+    // product is issued (into the same registers: two sets, and the totals,
+    // would leave one workgroup a CU).
     const int64_t nchunk = (k_end - k_beg) / kChunk;
-    auto load_a = [&](bf16x8 *a, int64_t c) {
+    auto load_a = [&](int64_t c, int st) {
         const int64_t kc = k_beg + min(c, nchunk - 1) * kChunk;   // clamped: in range
-#pragma unroll
-        for (int st = 0; st < 4; ++st)
-            a[st] = *reinterpret_cast<const bf16x8 *>(mrow + (kc / 16 + st) * 512);
+        return *reinterpret_cast<const bf16x8 *>(mrow + (kc / 16 + st) * 512);
     };
-    auto load_x = [&](float4 *x, int64_t c) {
-        const int64_t kc = k_beg + min(c, nchunk - 1) * kChunk;
-#pragma unroll
-        for (int q = 0; q < 2; ++q) x[q] = *reinterpret_cast<const float4 *>(xcol + kc + 4 * q);
+    float4 x0, x1;
+    auto load_x = [&](int64_t c) {
+        const float *p = xcol + k_beg + min(c, nchunk - 1) * kChunk;
+        x0 = *reinterpret_cast<const float4 *>(p);
+        x1 = *reinterpret_cast<const float4 *>(p + 4);
     };
-    auto chunk = [&](const float4 *x, const bf16x8 *a) {
+    bf16x8 a[4];
+    load_x(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int st = 0; st < 4; ++st) a[st] = load_a(0, st);
+    for (int64_t c = 0; c < nchunk; ++c) {
         __syncthreads();   // the previous chunk's LDS operands have been read
         // the three BF16 terms of 8 values, packed two per word: 16-byte LDS stores
-        uint32_t ph[4], pm[4], pl[4];
+        {
+            const float v[8] = {x0.x * xon, x0.y * xon, x0.z * xon, x0.w * xon,
+                                x1.x * xon, x1.y * xon, x1.z * xon, x1.w * xon};
+            uint32_t ph[4], pm[4], pl[4];
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const float v[4] = {x[q].x * xon, x[q].y * xon, x[q].z * xon, x[q].w * xon};
-#pragma unroll
-            for (int e = 0; e < 4; e += 2) {
-                uint32_t h2 = 0, m2 = 0, l2 = 0;
+            for (int e = 0; e < 4; ++e) {
+                ph[e] = pm[e] = pl[e] = 0;
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
-                    const float w = v[e + u];
+                    const float w = v[2 * e + u];
                     const uint32_t h = bf16_rne(w);
                     const float r1 = w - __uint_as_float(h << 16);
                     const uint32_t md = bf16_rne(r1);
                     const float r2 = r1 - __uint_as_float(md << 16);
-                    const uint32_t lo = bf16_rne(r2);
-                    h2 |= h << (16 * u); m2 |= md << (16 * u); l2 |= lo << (16 * u);
+                    ph[e] |= h << (16 * u);
+                    pm[e] |= md << (16 * u);
+                    pl[e] |= (uint32_t)bf16_rne(r2) << (16 * u);
                 }
-                ph[2 * q + e / 2] = h2; pm[2 * q + e / 2] = m2; pl[2 * q + e / 2] = l2;
             }
+            *reinterpret_cast<uint4 *>(&xh[xc][xk]) = make_uint4(ph[0], ph[1], ph[2], ph[3]);
+            *reinterpret_cast<uint4 *>(&xm[xc][xk]) = make_uint4(pm[0], pm[1], pm[2], pm[3]);
+            *reinterpret_cast<uint4 *>(&xl[xc][xk]) = make_uint4(pl[0], pl[1], pl[2], pl[3]);
         }
-        *reinterpret_cast<uint4 *>(&xh[xc][xk]) = make_uint4(ph[0], ph[1], ph[2], ph[3]);
-        *reinterpret_cast<uint4 *>(&xm[xc][xk]) = make_uint4(pm[0], pm[1], pm[2], pm[3]);
-        *reinterpret_cast<uint4 *>(&xl[xc][xk]) = make_uint4(pl[0], pl[1], pl[2], pl[3]);
+        __builtin_amdgcn_sched_barrier(0);
+        load_x(c + 1);
+        __builtin_amdgcn_sched_barrier(0);
         __syncthreads();
+        // a chunk's sums (64 products a term) start at zero and are added to
+        // the totals: a chain as long as a whole slice of K loses bits
+        f32x16 acc0 = {}, acc1 = {};
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
             const int kk = 16 * st + 8 * (lane >> 5);
             const int c0 = lane & 31, c1 = 32 + (lane & 31);
-            // smallest terms first: the accumulator adds the large ones last
-            const bf16x8 b0l = *reinterpret_cast<const bf16x8 *>(&xl[c0][kk]);
-            const bf16x8 b1l = *reinterpret_cast<const bf16x8 *>(&xl[c1][kk]);
-            acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[st], b0l, acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[st], b1l, acc1, 0, 0, 0);
-            const bf16x8 b0m = *reinterpret_cast<const bf16x8 *>(&xm[c0][kk]);
-            const bf16x8 b1m = *reinterpret_cast<const bf16x8 *>(&xm[c1][kk]);
-            acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[st], b0m, acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[st], b1m, acc1, 0, 0, 0);
-            const bf16x8 b0h = *reinterpret_cast<const bf16x8 *>(&xh[c0][kk]);
-            const bf16x8 b1h = *reinterpret_cast<const bf16x8 *>(&xh[c1][kk]);
-            acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[st], b0h, acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[st], b1h, acc1, 0, 0, 0);
+            auto term = [&](const uint16_t (*xt)[kPadK]) {
+                const bf16x8 b0 = *reinterpret_cast<const bf16x8 *>(&xt[c0][kk]);
+                const bf16x8 b1 = *reinterpret_cast<const bf16x8 *>(&xt[c1][kk]);
+                acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[st], b0, acc0, 0, 0, 0);
+                acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[st], b1, acc1, 0, 0, 0);
+            };
+            term(xl);          // smallest terms first: the large ones are added last
+            term(xm);
+            term(xh);
+            a[st] = load_a(c + 1, st);
         }
-    };
-    bf16x8 a0[4], a1[4];
-    float4 x0[2], x1[2];
-    load_x(x0, 0);
-    load_a(a0, 0);
-    // (no exit between the two halves, so the compiler does not sink the
-    // next chunk's loads below the current chunk's work; an odd last chunk
-    // runs after the loop)
-    int64_t c = 0;
-    for (; c + 1 < nchunk; c += 2) {
-        load_x(x1, c + 1);
-        load_a(a1, c + 1);
-        chunk(x0, a0);
-        load_x(x0, c + 2);
-        load_a(a0, c + 2);
-        chunk(x1, a1);
+        tot0 += acc0;
+        tot1 += acc1;
+        // issue order: kAhead operand reads lead the matrix instructions, each
+        // of which is followed by one more read; a step's load of M goes out
+        // as soon as its operand is free.  Left alone the compiler reads an
+        // operand, waits, multiplies, and sinks the loads to the loop's end.
+        constexpr int kAhead = 4;
+        __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);
+#pragma unroll
+        for (int k = 0; k < 24; ++k) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if (k < 24 - kAhead) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            if (k % 6 == 5) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+        }
     }
-    if (c < nchunk) chunk(x0, a0);
     // partial tile, row-major [s][row][64]
     float *out = part + ((int64_t)s * R + tile * kRows + wave * 32) * kCols;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const int i = 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        out[(int64_t)i * kCols + (lane & 31)] = acc0[r];
-        out[(int64_t)i * kCols + 32 + (lane & 31)] = acc1[r];
+        out[(int64_t)i * kCols + (lane & 31)] = tot0[r];
+        out[(int64_t)i * kCols + 32 + (lane & 31)] = tot1[r];
     }
 }
 
-// Y[j ldy + row] = sum_s part[s][row][j] (- sub[j ldy + row]), j < G, the
-// S partials added in order s = 0, 1, ...; one workgroup per 32 rows (a
-// thread sums 8 rows of one column: eight independent load chains), LDS
-// transpose for column-major stores of 32 consecutive rows
+// Y[j ldy + row] = sum_s part[s][row][j] (- sub[j ldy + row]), j < G: one
+// workgroup per 8 rows, a thread sums every other partial of four columns of
+// a row (fixed order), eight loads in flight; the halves meet in LDS, read
+// back with rows consecutive.  (32 rows a workgroup and one chain of S loads
+// a thread took 11 us at S = 16, and 25 us of a whole 35 us product at 1024 x
+// 4096 and S = 64.)
 __global__ __launch_bounds__(256) void k_gemm_reduce(const float *__restrict__ part, int64_t R,
                                                      int S, int G, float *__restrict__ Y,
                                                      int64_t ldy, const float *__restrict__ sub,
                                                      const int32_t *gate) {
     if (gate && !*gate) return;
-    __shared__ float tile[kCols][33];
+    __shared__ float tile[2][8][kCols + 1];
     const int t = threadIdx.x;
-    const int64_t r0 = (int64_t)blockIdx.x * 32;
-    const int c = t & 63, rg = (t >> 6) * 8;
-    float v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int s = 0; s < S; ++s) {
-        const float *p = part + ((int64_t)s * R + r0 + rg) * kCols + c;
+    const int64_t r0 = (int64_t)blockIdx.x * 8;
+    const int c = (t & 15) * 4, row = (t >> 4) & 7, half = t >> 7;
+    const float *p = part + (r0 + row) * kCols + c;
+    float4 v = make_float4(0, 0, 0, 0);
+    auto add = [&v](const float4 &w) {
+        v.x += w.x; v.y += w.y; v.z += w.z; v.w += w.w;
+    };
+    int s = half;
+    for (; s + 14 < S; s += 16) {
+        float4 w[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] += p[(int64_t)i * kCols];
+        for (int i = 0; i < 8; ++i)
+            w[i] = *reinterpret_cast<const float4 *>(p + (int64_t)(s + 2 * i) * R * kCols);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) add(w[i]);
     }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) tile[c][rg + i] = v[i];
+    for (; s < S; s += 2) add(*reinterpret_cast<const float4 *>(p + (int64_t)s * R * kCols));
+    float *o = &tile[half][row][c];
+    o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
     __syncthreads();
-    const int rr = t & 31, cg = (t >> 5) * 8;
+    const int rr = t & 7;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int cc = cg + i;
+    for (int cc = t >> 3; cc < kCols; cc += 32) {
         if (cc >= G) break;
-        const int64_t o = (int64_t)cc * ldy + r0 + rr;
-        const float w = tile[cc][rr];
-        Y[o] = sub ? w - sub[o] : w;
+        const int64_t q = (int64_t)cc * ldy + r0 + rr;
+        const float w = tile[0][rr][cc] + tile[1][rr][cc];
+        Y[q] = sub ? w - sub[q] : w;
     }
 }
 
@@ -247,7 +268,7 @@ void gemm_rhs(const uint16_t *M, int64_t R, int64_t K, const float *X, int64_t l
     const unsigned grid = (unsigned)((R / kRows) * splits);
     hipLaunchKernelGGL(k_gemm_rhs, dim3(grid), dim3(kThreads), 0, s, M, R, K, splits, X, ldx, G,
                        part, gate);
-    hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)(R / 32)), dim3(256), 0, s, part, R, splits,
+    hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)(R / 8)), dim3(256), 0, s, part, R, splits,
                        G, Y, ldy, sub, gate);
 }
 

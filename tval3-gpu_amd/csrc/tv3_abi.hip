@@ -586,9 +586,15 @@ tv3_status tv3_matvec_multi(tv3_op *op, tv3_trans trans, int32_t nrhs, const flo
             TV3_HIP(hipGetLastError());
             return;
         }
-        // K splits: enough workgroups to fill the device, K a multiple of 64 splits
+        // K splits (K a multiple of 64 splits): a workgroup a CU, and a second
+        // one where 2,048 values of K are left to each: every split writes and
+        // reads back R x 64 partial sums.  64 columns, A X, us, with 256, 512,
+        // 1024 workgroups: 4096 x 16384 45, 44, 57; 8192 x 32768 155, 150, 160;
+        // 2048 x 8192 20, 23, 32
+        const int64_t tiles = R / gemm_rhs_rows(), cus = op->ctx->num_cus;
         int splits = 1;
-        while ((R / gemm_rhs_rows()) * splits < 1024 && gemm_rhs_shape_ok(R, K, splits * 2))
+        while (gemm_rhs_shape_ok(R, K, splits * 2) &&
+               (tiles * splits < cus || (tiles * splits < 2 * cus && K / (2 * splits) >= 2048)))
             splits *= 2;
         const size_t need = gemm_rhs_scratch(R, splits) * sizeof(float);
         if (op->ctx->scratch.bytes() < need) op->ctx->scratch.alloc(need);
