@@ -441,9 +441,7 @@ std::unique_ptr<FusedLayout> build_dyn_layout(tv3_op *op) {
         TV3_HIP(hipGetLastError());
         TV3_HIP(hipStreamSynchronize(ctx->stream));
     }
-    const int64_t big = n > m ? n : m;
-    D->xin.alloc(big > 0 ? big : 1);
-    D->yout.alloc(big > 0 ? big : 1);
+    D->rin.alloc(m > 0 ? m : 1);
     TV3_HIP(hipStreamSynchronize(ctx->stream));
     // the matrices themselves are not kept: sizes only
     for (SparseRows *S : {&L->A, &L->AT}) {
@@ -460,17 +458,15 @@ std::unique_ptr<FusedLayout> build_dyn_layout(tv3_op *op) {
 bool dyn_tile_apply(tv3_op *op, bool trans, const float *x, float *y, hipStream_t s) {
     FusedLayout *F = op->fused.get();
     if (!F || !F->dyn) return false;
+    // natural order in and out without passes of its own, except r: A x stages
+    // its boxes from x as it is, and the sums are stored through the maps
     DynTiles &D = *F->dyn;
-    const int64_t n = op->n, m = op->m;
     if (!trans) {
-        permute_gather(x, F->v_int2nat.p, D.xin.p, n, s);
-        launch_dyn_N<float>(D, D.xin.p, F->RS.part.p, nullptr, s);
-        launch_seg_sum(F->RS, EpiStoreIf{D.yout.p, nullptr}, s);
-        permute_scatter(D.yout.p, F->r_int2nat.p, y, m, s);
+        launch_dyn_N<true, float>(D, x, F->RS.part.p, nullptr, s);
+        launch_seg_sum(F->RS, EpiScatter{y, F->r_int2nat.p}, s);
     } else {
-        permute_gather(x, F->r_int2nat.p, D.xin.p, m, s);
-        launch_dyn_T<float>(D, D.xin.p, EpiStoreIf{D.yout.p, nullptr}, s);
-        permute_scatter(D.yout.p, F->v_int2nat.p, y, n, s);
+        permute_gather(x, F->r_int2nat.p, D.rin.p, op->m, s);
+        launch_dyn_T<float>(D, D.rin.p, EpiScatter{y, F->v_int2nat.p}, s);
     }
     TV3_HIP(hipGetLastError());
     return true;

@@ -85,6 +85,19 @@ struct EpiStoreIf {
     __device__ __forceinline__ void finish() const {}
 };
 
+// Epilogue that stores y[map[row]] = sum.
+struct EpiScatter {
+    float *y;
+    const int32_t *map;
+    struct Pre { int32_t at; };
+    __device__ bool skip() const { return false; }
+    __device__ __forceinline__ Pre load(int r) const { return {map[r]}; }
+    __device__ __forceinline__ void row(int, float s, bool on, const Pre &p) const {
+        if (on) y[p.at] = s;
+    }
+    __device__ __forceinline__ void finish() const {}
+};
+
 // Extra workgroups an epilogue asks of a panel launch (Epi::kExtra, default
 // 0): blocks 0 .. kExtra - 1 run epi.extra() instead of a panel.
 template <typename E, typename = void> struct ExtraBlocks { static constexpr int value = 0; };
@@ -539,6 +552,7 @@ struct DynView {
     const uint16_t *pos;
     int emax_cap;
     int tile_dx, tile_dz;   // internal offset of the next tile along x, z
+    int nx, ny;             // voxels along x, y
 };
 
 inline DynView dyn_view(const DynTiles &D, const DynBoxes &X) {
@@ -549,6 +563,8 @@ inline DynView dyn_view(const DynTiles &D, const DynBoxes &X) {
     v.emax_cap = D.emax_cap;
     v.tile_dx = D.tile_dx;
     v.tile_dz = D.tile_dz;
+    v.nx = D.N[0];
+    v.ny = D.N[1];
     return v;
 }
 
@@ -654,8 +670,9 @@ __host__ __device__ __forceinline__ void dyn_seg_walk(const DynView &g, const Dy
 
 // A x, first pass: per box its voxels staged in LDS, each thread walks
 // segments and stores their partial sums (walk order) in part[segment].
+// NAT: x in natural order (y, x, z), else in the internal order.
 // `active` (may be NULL) predicates the launch like an epilogue's skip().
-template <typename T>
+template <bool NAT, typename T>
 __global__ __launch_bounds__(256) void k_dyn_tile_N(DynView g, const T *__restrict__ x,
                                                     T *__restrict__ part,
                                                     const int32_t *active) {
@@ -663,16 +680,22 @@ __global__ __launch_bounds__(256) void k_dyn_tile_N(DynView g, const T *__restri
     __shared__ T xs[4096];
     const DynPan P = g.pan[g.order[blockIdx.x]];
     const int t = threadIdx.x, bs = P.bs, ey = P.ey, nv = ey * bs * bs;
+    const int sy = 31 - __clz(ey), sx = 31 - __clz(bs);      // the edges are powers of two
     for (int i = t; i < nv; i += 256) {     // linear box order y + ey x + ey bs z
-        // tile sb of the box (bits: y, x, z; boxes of one tile or brick: 0)
-        const int j = i & 511, sb = i >> 9;
-        int lx, ly, lz;
-        dyn_local_xyz(j, lx, ly, lz);
-        lx += (sb & 2) << 2;
-        ly += (sb & 1) << 3;
-        lz += (sb & 4) << 1;
-        xs[ly + ey * (lx + bs * lz)] =
-            x[P.v0 + (sb & 1) * 512 + ((sb >> 1) & 1) * g.tile_dx + (sb >> 2) * g.tile_dz + j];
+        if constexpr (NAT) {
+            const int ly = i & (ey - 1), lx = (i >> sy) & (bs - 1), lz = i >> (sy + sx);
+            xs[i] = x[((int64_t)(P.bz + lz) * g.nx + P.bx + lx) * g.ny + P.by + ly];
+        } else {
+            // tile sb of the box (bits: y, x, z; boxes of one tile or brick: 0)
+            const int j = i & 511, sb = i >> 9;
+            int lx, ly, lz;
+            dyn_local_xyz(j, lx, ly, lz);
+            lx += (sb & 2) << 2;
+            ly += (sb & 1) << 3;
+            lz += (sb & 4) << 1;
+            xs[ly + ey * (lx + bs * lz)] =
+                x[P.v0 + (sb & 1) * 512 + ((sb >> 1) & 1) * g.tile_dx + (sb >> 2) * g.tile_dz + j];
+        }
     }
     __syncthreads();
     for (int sg = P.s0 + t; sg < P.s1; sg += 256) {
@@ -751,10 +774,10 @@ __global__ __launch_bounds__(NT) void k_dyn_tile_T(DynView g, const T *__restric
     epi.finish();
 }
 
-template <typename T>
+template <bool NAT, typename T>
 void launch_dyn_N(const DynTiles &D, const T *x, T *part, const int32_t *active, hipStream_t s) {
     if (D.fwd.npan == 0) return;
-    hipLaunchKernelGGL((k_dyn_tile_N<T>), dim3((unsigned)D.fwd.npan), dim3(256), 0, s,
+    hipLaunchKernelGGL((k_dyn_tile_N<NAT, T>), dim3((unsigned)D.fwd.npan), dim3(256), 0, s,
                        dyn_view(D, D.fwd), x, part, active);
 }
 
@@ -815,7 +838,7 @@ template <typename Acc, typename Epi>
 void launch_forward(const FusedLayout &F, const float *x, const Epi &epi, hipStream_t s,
                     const int32_t *active = nullptr) {
     if (F.dyn) {
-        launch_dyn_N<float>(*F.dyn, x, F.RS.part.p, active, s);
+        launch_dyn_N<false, float>(*F.dyn, x, F.RS.part.p, active, s);
         launch_seg_sum(F.RS, epi, s);
     } else if (F.panels_A) {
         launch_panel(F.PA, x, EpiStoreIf{F.RS.part.p, active}, s);

@@ -317,7 +317,7 @@ struct DynTiles {
     DevBuf<uint32_t> pptr;           // n + 1: padded starts of the voxel rows
     DevBuf<uint16_t> pos;            // per voxel row its entries' positions in its bwd
                                      // box, ray order, padded to 4 with the position ne
-    DevBuf<float> xin, yout;         // natural <-> internal order staging (max(n, m))
+    DevBuf<float> rin;               // a caller's r in internal ray order (m)
 };
 
 // The fused solver's internal layout of a sparse operator: voxels numbered by
