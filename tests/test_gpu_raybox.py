@@ -43,6 +43,8 @@ GEOMS = {
     "remainders": lambda: wl.transducer_geometry(20, 45, dims=(17, 9, 23), seed=3),
     "long_y": lambda: wl.transducer_geometry(9, 64, dims=(61, 7, 8), seed=4),
     "split_boxes": lambda: wl.transducer_geometry(96, 256, dims=(16, 13, 10), seed=9),
+    # Siddon on 8^3 tiles of about 26,000 entries: A^T boxes of half a tile
+    "half_tiles": lambda: wl.transducer_geometry(48, 256, dims=(16, 16, 16), seed=2),
     "two_positions": lambda: _two_positions(10, 30, (22, 18, 15)),
     "masked": lambda: _masked(24, 40, (19, 21, 33)),
     "outside": lambda: _outside(12, 24, (20, 14, 11)),

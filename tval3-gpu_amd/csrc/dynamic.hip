@@ -282,6 +282,7 @@ __global__ __launch_bounds__(kBoxThreads) void k_box_T(GeoView g, int nby, int n
     P.bz = it.x / nby / nbx * kRayBoxXZ;
     P.bs = kRayBoxXZ;
     P.ey = kRayBoxY;
+    P.ez = kRayBoxXZ;
     for (int i = t; i < NV; i += NT) box[i] = 0;
     __syncthreads();
     // a part needs two loads in turn, its segment and then its ray's record

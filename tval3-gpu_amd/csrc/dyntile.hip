@@ -6,9 +6,11 @@
 // Boxes: for A x, blocks of 2 x 2 x 2 of the fused solver's 8^3 tiles
 // (16^3 voxels) where every tile count is even, else pairs of tiles
 // consecutive in y (or single tiles, or 4^3 bricks when B = 4); for A^T r,
-// the 8^3 tiles, or
-// their 4^3 bricks where a tile holds more ray entries than the A^T product
-// keeps in LDS (and every brick when B = 4).  A box is convex, so a ray's
+// the 8^3 tiles, or their halves along z, or
+// their 4^3 bricks where a tile (a half) holds more ray entries than the A^T
+// product keeps in LDS (and every brick when B = 4).  Halves cut fewer rays
+// than bricks: with both products' permutations gone, A^T at 128^3 171 -> 158
+// us.  A box is convex, so a ray's
 // entries inside it are consecutive in traversal order: one segment.
 // Segments are numbered box by box, inside a box by decreasing length in
 // buckets, ascending ray in a bucket (sort_segments); an A^T box's entries
@@ -127,23 +129,28 @@ SegPlan plan_segments(const std::vector<int32_t> &ptr, const std::vector<int32_t
     return S;
 }
 
-// boxes: tile u (B = 8) whole or as its 8 bricks, or brick u (B = 4)
+// boxes: tile u (B = 8) whole (parts = 1), as its two halves along z (2) or
+// as its 8 bricks (8), or brick u (B = 4)
 void add_boxes(std::vector<DynPan> &pan, std::vector<int32_t> &box_of, int B, int64_t u, int nby,
-               int nbx, bool split) {
+               int nbx, int parts) {
     const int ty = (int)(u % nby), tx = (int)((u / nby) % nbx),
               tz = (int)(u / ((int64_t)nby * nbx));
-    if (B == 8 && !split) {
-        pan.push_back(DynPan{(int32_t)(u << 9), 8 * tx, 8 * ty, 8 * tz, 8, 8, 0, 0, 0});
-        for (int k = 0; k < 8; ++k) box_of[(u << 3) + k] = (int32_t)pan.size() - 1;
+    if (B == 8 && parts < 8) {
+        for (int h = 0; h < parts; ++h) {
+            pan.push_back(DynPan{(int32_t)((u << 9) + 256 * h), 8 * tx, 8 * ty, 8 * tz + 4 * h, 8, 8,
+                                 8 / parts, 0, 0, 0});
+            for (int k = 0; k < 8 / parts; ++k)
+                box_of[(u << 3) + 4 * h + k] = (int32_t)pan.size() - 1;
+        }
     } else if (B == 8) {
         for (int sb = 0; sb < 8; ++sb) {   // sub-brick bits: y (1), x (2), z (4)
             pan.push_back(DynPan{(int32_t)((u << 9) + (sb << 6)), 8 * tx + 4 * ((sb >> 1) & 1),
-                                 8 * ty + 4 * (sb & 1), 8 * tz + 4 * ((sb >> 2) & 1), 4, 4, 0, 0,
-                                 0});
+                                 8 * ty + 4 * (sb & 1), 8 * tz + 4 * ((sb >> 2) & 1), 4, 4, 4, 0,
+                                 0, 0});
             box_of[(u << 3) + sb] = (int32_t)pan.size() - 1;
         }
     } else {
-        pan.push_back(DynPan{(int32_t)(u << 6), 4 * tx, 4 * ty, 4 * tz, 4, 4, 0, 0, 0});
+        pan.push_back(DynPan{(int32_t)(u << 6), 4 * tx, 4 * ty, 4 * tz, 4, 4, 4, 0, 0, 0});
         box_of[u] = (int32_t)pan.size() - 1;
     }
 }
@@ -154,7 +161,7 @@ void add_pair_box(std::vector<DynPan> &pan, std::vector<int32_t> &box_of, int64_
                   int nbx) {
     const int ty = (int)(u % nby), tx = (int)((u / nby) % nbx),
               tz = (int)(u / ((int64_t)nby * nbx));
-    pan.push_back(DynPan{(int32_t)(u << 9), 8 * tx, 8 * ty, 8 * tz, 8, 16, 0, 0, 0});
+    pan.push_back(DynPan{(int32_t)(u << 9), 8 * tx, 8 * ty, 8 * tz, 8, 16, 8, 0, 0, 0});
     for (int k = 0; k < 16; ++k) box_of[(u << 3) + k] = (int32_t)pan.size() - 1;
 }
 
@@ -165,7 +172,7 @@ void add_box16(std::vector<DynPan> &pan, std::vector<int32_t> &box_of, int64_t u
                int nbx) {
     const int ty = (int)(u % nby), tx = (int)((u / nby) % nbx),
               tz = (int)(u / ((int64_t)nby * nbx));
-    pan.push_back(DynPan{(int32_t)(u << 9), 8 * tx, 8 * ty, 8 * tz, 16, 16, 0, 0, 0});
+    pan.push_back(DynPan{(int32_t)(u << 9), 8 * tx, 8 * ty, 8 * tz, 16, 16, 16, 0, 0, 0});
     for (int sb = 0; sb < 8; ++sb) {
         const int64_t t = u + (sb & 1) + ((sb >> 1) & 1) * (int64_t)nby +
                           (sb >> 2) * (int64_t)nby * nbx;
@@ -231,7 +238,7 @@ std::vector<uint16_t> segment_starts(const std::vector<int32_t> &ptr,
             const DynPan &P = pan[box_of[ind[k] >> 6]];
             int x, y, z;
             box_local(ind[k], P, B, nby, nbx, x, y, z);
-            TV3_REQUIRE(x >= 0 && y >= 0 && z >= 0 && x < P.bs && y < P.ey && z < P.bs,
+            TV3_REQUIRE(x >= 0 && y >= 0 && z >= 0 && x < P.bs && y < P.ey && z < P.ez,
                         TV3_E_INTERNAL, "a segment starts outside its box");
             c0[sg] = (uint16_t)(x | (y << 4) | (z << 8));
         }
@@ -337,8 +344,9 @@ std::unique_ptr<FusedLayout> build_dyn_layout(tv3_op *op) {
     const int B = L->B, nby = L->nby, nbx = L->nbx;   // tiles (B = 8) or bricks (B = 4)
     const int64_t nunit = n / (B == 8 ? 512 : 64);
     const int ushift = B == 8 ? 9 : 6;
-    std::vector<int32_t> unit_ent(nunit, 0);
-    for (int64_t k = 0; k < nnz; ++k) ++unit_ent[ind[k] >> ushift];
+    std::vector<int64_t> unit_ent(nunit, 0), brick_ent((size_t)(n >> 6), 0);
+    for (int64_t k = 0; k < nnz; ++k) ++brick_ent[ind[k] >> 6];
+    for (int64_t b = 0; b < n >> 6; ++b) unit_ent[b >> (ushift - 6)] += brick_ent[b];
     // forward boxes: whole units; backward: split where the LDS limits ask
     std::vector<DynPan> panF, panT;
     std::vector<int32_t> boxF((size_t)(n >> 6), -1), boxT((size_t)(n >> 6), -1);
@@ -357,11 +365,17 @@ std::unique_ptr<FusedLayout> build_dyn_layout(tv3_op *op) {
         if (box16) {
             if (ty % 2 == 0 && tx % 2 == 0 && tz % 2 == 0) add_box16(panF, boxF, u, nby, nbx);
         } else if (!pairs) {
-            add_boxes(panF, boxF, B, u, nby, nbx, false);
+            add_boxes(panF, boxF, B, u, nby, nbx, 1);
         } else if (u % 2 == 0) {
             add_pair_box(panF, boxF, u, nby, nbx);
         }
-        add_boxes(panT, boxT, B, u, nby, nbx, unit_ent[u] > D->emax_cap);
+        int parts = 1;
+        if (B == 8 && unit_ent[u] > D->emax_cap) {
+            const int64_t b0 = u << 3;
+            const int64_t lo = brick_ent[b0] + brick_ent[b0 + 1] + brick_ent[b0 + 2] + brick_ent[b0 + 3];
+            parts = std::max(lo, unit_ent[u] - lo) <= D->emax_cap ? 2 : 8;
+        }
+        add_boxes(panT, boxT, B, u, nby, nbx, parts);
     }
     if (B == 8) {
         D->tile_dx = nby * 512;
@@ -399,7 +413,7 @@ std::unique_ptr<FusedLayout> build_dyn_layout(tv3_op *op) {
         }
     }
     for (const DynPan &P : panT) {                    // padding: the box's zero slot ne
-        const int nv = P.ey * P.bs * P.bs;
+        const int nv = P.ey * P.bs * P.ez;
         for (int32_t v = P.v0; v < P.v0 + nv; ++v)
             for (uint32_t q = vfill[v]; q < pptr[v + 1]; ++q) pos[q] = (uint16_t)P.ne;
     }

@@ -620,7 +620,7 @@ __host__ __device__ __forceinline__ void dyn_seg_walk(const DynSeg &sr, const Dy
     const int lc[3] = {c0 & 15, (c0 >> 4) & 15, (c0 >> 8) & 15};
     const int b0[3] = {P.bx, P.by, P.bz};
     const int bs = P.bs, ey = P.ey;
-    const int ext[3] = {bs, ey, bs};
+    const int ext[3] = {bs, ey, P.ez};
     const int stride[3] = {ey, 1, ey * bs};
     float kf[3], tk[3], st[3];
     int dstep[3], off = 0;
@@ -642,7 +642,7 @@ __host__ __device__ __forceinline__ void dyn_seg_walk(const DynSeg &sr, const Dy
         dstep[a] = up ? stride[a] : (par ? 0 : -stride[a]);
     }
     // the offset is masked all the same, so that no index leaves the box
-    const int mask = ey * bs * bs - 1;
+    const int mask = ey * bs * P.ez - 1;
     float tcur = ts;
     for (int step = 0; step < 2 * bs + ey + 4; ++step) {
         float tnext = te;
@@ -719,7 +719,7 @@ __global__ __launch_bounds__(NT) void k_dyn_tile_T(DynView g, const T *__restric
     static_assert(NT >= 512, "one voxel row per thread (boxes of at most 8^3)");
     const DynPan P = g.pan[g.order[blockIdx.x]];
     T *pe = reinterpret_cast<T *>(dyn_smem);
-    const int t = threadIdx.x, ns = P.s1 - P.s0, nv = P.ey * P.bs * P.bs;
+    const int t = threadIdx.x, ns = P.s1 - P.s0, nv = P.ey * P.bs * P.ez;
     // phase 2's operands do not depend on phase 1: its row starts, first
     // positions and epilogue operands are requested before the walks
     const bool has_row = t < nv;

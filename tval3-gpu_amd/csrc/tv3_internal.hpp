@@ -282,9 +282,9 @@ struct SegSum {
 struct DynPan {
     int32_t v0;          // first internal voxel of the box (of its first tile)
     int32_t bx, by, bz;  // box corner in voxel coordinates (x, y, z)
-    int32_t bs;          // box edge along x and z: 16 (2 x 2 x 2 tiles), 8 (tiles) or 4
-                         // (a brick)
+    int32_t bs;          // box edge along x: 16 (2 x 2 x 2 tiles), 8 (tiles) or 4 (a brick)
     int32_t ey;          // box edge along y: bs, or 16 for two tiles consecutive in y
+    int32_t ez;          // box edge along z: bs, or 4 for half a tile
     int32_t s0, s1;      // its segments
     int32_t ne;          // entries of its segments
 };
