@@ -33,7 +33,7 @@ import ctypes as C
 import torch
 
 from . import _lib as L
-from .api import _torch_stream, _vp
+from .api import _torch_stream
 
 
 def _dtype_code(t):
@@ -68,22 +68,36 @@ def matvec(op, x, trans=False):
     return MatVec.apply(x, op, trans)
 
 
+_Dims = C.c_int32 * 3
+
+
+def _rows(t):
+    """Addresses of t[0], t[1], t[2], without the three views (1 us each)."""
+    if t.shape[0] < 3:
+        raise IndexError("a field of three rows is needed, got %d" % t.shape[0])
+    p, step = t.data_ptr(), t.stride(0) * t.element_size()
+    return p, p + step, p + 2 * step
+
+
 def _D(tctx, U, dims):
+    code = _dtype_code(U)
+    U = _c(U)
     out = torch.empty((3, U.numel()), dtype=U.dtype, device=U.device)
-    d = (C.c_int32 * 3)(*dims)
-    f = L.load().tv3_D_f64 if U.dtype == torch.float64 else L.load().tv3_D
-    _dtype_code(U)
-    tctx.check(f(tctx.h, d, _vp(_c(U)), _vp(out[0]), _vp(out[1]), _vp(out[2]), _torch_stream()))
+    f = L.load().tv3_D_f64 if code == L.F64 else L.load().tv3_D
+    st = f(tctx.h, _Dims(*dims), U.data_ptr(), *_rows(out), _torch_stream())
+    if st:
+        tctx.check(st)
     return out
 
 
 def _Dt(tctx, V, dims):
+    code = _dtype_code(V)
     V = _c(V)
     out = torch.empty(V.shape[1], dtype=V.dtype, device=V.device)
-    d = (C.c_int32 * 3)(*dims)
-    f = L.load().tv3_Dt_f64 if V.dtype == torch.float64 else L.load().tv3_Dt
-    _dtype_code(V)
-    tctx.check(f(tctx.h, d, _vp(V[0]), _vp(V[1]), _vp(V[2]), _vp(out), _torch_stream()))
+    f = L.load().tv3_Dt_f64 if code == L.F64 else L.load().tv3_Dt
+    st = f(tctx.h, _Dims(*dims), *_rows(V), out.data_ptr(), _torch_stream())
+    if st:
+        tctx.check(st)
     return out
 
 
@@ -139,10 +153,12 @@ class Shrink(torch.autograd.Function):
         if mask_in is not None:
             assert mask_in.dtype == torch.uint8 and mask_in.numel() == n
             mask_in = _c(mask_in)
-        tctx.check(L.load().tv3_shrink_apply(tctx.h, n, L.ISO if iso else L.ANISO,
-                                             _dtype_code(V), _vp(V[0]), _vp(V[1]), _vp(V[2]),
-                                             float(t), _vp(W[0]), _vp(W[1]), _vp(W[2]), _vp(s),
-                                             _vp(mask_in), _vp(active), _torch_stream()))
+        st = L.load().tv3_shrink_apply(tctx.h, n, L.ISO if iso else L.ANISO, _dtype_code(V),
+                                       *_rows(V), float(t), *_rows(W), s.data_ptr(),
+                                       None if mask_in is None else mask_in.data_ptr(),
+                                       active.data_ptr(), _torch_stream())
+        if st:
+            tctx.check(st)
         ctx.save_for_backward(V)
         ctx.t, ctx.iso, ctx.tctx = float(t), iso, tctx
         ctx.mark_non_differentiable(active)
@@ -157,10 +173,12 @@ class Shrink(torch.autograd.Function):
         gW = _c(gW)
         gs = None if gs is None else _c(gs)
         gV = torch.empty_like(V)
-        ctx.tctx.check(L.load().tv3_shrink_adjoint(
-            ctx.tctx.h, n, L.ISO if ctx.iso else L.ANISO, _dtype_code(V), _vp(V[0]), _vp(V[1]),
-            _vp(V[2]), ctx.t, _vp(gW[0]), _vp(gW[1]), _vp(gW[2]), _vp(gs), _vp(gV[0]),
-            _vp(gV[1]), _vp(gV[2]), _torch_stream()))
+        st = L.load().tv3_shrink_adjoint(ctx.tctx.h, n, L.ISO if ctx.iso else L.ANISO,
+                                         _dtype_code(V), *_rows(V), ctx.t, *_rows(gW),
+                                         None if gs is None else gs.data_ptr(), *_rows(gV),
+                                         _torch_stream())
+        if st:
+            ctx.tctx.check(st)
         return gV, None, None, None, None
 
 
