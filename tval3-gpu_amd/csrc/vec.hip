@@ -443,10 +443,6 @@ void queue_update(Sums &S, const PlainFields<T> &f, const T *g, const T *gp, con
 }
 
 template <typename T>
-double dot(tv3_ctx *ctx, int64_t n, const T *a, const T *b, hipStream_t s) {
-    return reduce_now<1>(ctx, n, FDot<T>{a, b}, s)[0];
-}
-template <typename T>
 double shrink_host(tv3_ctx *ctx, int64_t n, int iso, const T *Ux, const T *Uy, const T *Uz,
                    const T *sx, const T *sy, const T *sz, double beta, T *Wx, T *Wy, T *Wz,
                    hipStream_t s) {
@@ -476,7 +472,6 @@ std::array<double, 2> diff_norm(tv3_ctx *ctx, int64_t n, const T *a, const T *b,
     template void launch_D<T>(const int32_t *, const T *, T *, T *, T *, hipStream_t);          \
     template void launch_Dt<T>(const int32_t *, const T *, const T *, const T *, T *,           \
                                hipStream_t);                                                    \
-    template double dot<T>(tv3_ctx *, int64_t, const T *, const T *, hipStream_t);              \
     template double shrink_host<T>(tv3_ctx *, int64_t, int, const T *, const T *, const T *,    \
                                    const T *, const T *, const T *, double, T *, T *, T *,      \
                                    hipStream_t);                                                \

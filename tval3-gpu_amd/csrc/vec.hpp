@@ -93,7 +93,6 @@ template <typename T>
 void grad(int64_t n, T *d, double a, const T *g, const T *g2, const T *dts, hipStream_t s);
 template <typename T> void scale(int64_t n, T *y, double a, const T *x, hipStream_t s);
 template <typename T> void divide(int64_t n, T *y, double a, const T *x, hipStream_t s);
-template <typename T> double dot(tv3_ctx *ctx, int64_t n, const T *a, const T *b, hipStream_t s);
 template <typename T>
 double mlp_sigma(tv3_ctx *ctx, int64_t n, const T *Ux, const T *Uy, const T *Uz, const T *Wx,
                  const T *Wy, const T *Wz, double beta, T *sx, T *sy, T *sz, hipStream_t s);
