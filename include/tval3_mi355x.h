@@ -412,9 +412,10 @@ tv3_status tv3_bandwidth_probe(tv3_ctx *ctx, int64_t bytes, int32_t reps, double
 
 /* ---- tuning ------------------------------------------------------------- */
 /* Time the sparse kernels of op over their launch shapes and keep the
- * fastest: the row-blocked kernel with 1024/2048/4096-entry blocks (returned
- * as -1024/-2048/-4096) or the row-group kernel with L lanes per row
- * (returned as L).  tv3_op_set_lanes accepts the same codes (0 = keep). */
+ * fastest: the row blocks a new operator has (returned as 0), the row-blocked
+ * kernel with 1024/2048/4096-entry blocks (returned as -1024/-2048/-4096) or
+ * the row-group kernel with L lanes per row (returned as L).
+ * tv3_op_set_lanes accepts the same codes (0 = keep). */
 tv3_status tv3_op_autotune(tv3_op *op, int32_t *lanes_N, int32_t *lanes_T);
 tv3_status tv3_op_set_lanes(tv3_op *op, int32_t lanes_N, int32_t lanes_T);
 

@@ -19,7 +19,7 @@
 //    consequences with every sum the next decision needs), each element
 //    computed and rounded as by one kernel per operation; an iteration
 //    without backtracking waits for the device once, and the previous iterate
-//    is kept by exchanging buffers (64^3 voxels, 65,536 rays: FIGURES an
+//    is kept by exchanging buffers (64^3 voxels, 65,536 rays: 95 us an
 //    iteration against 270 us with one kernel per operation and a wait per
 //    inner product);
 //  * the work vectors stay with the context (the reference allocates and

@@ -10,7 +10,9 @@
 // (col, val) pairs per step and a 64-wide wavefront reads 64/L rows' worth of
 // consecutive memory: the col/val streams are fully coalesced whatever L is.
 // x is gathered (it stays in L2 / MALL); the group sum is a butterfly over L
-// lanes.  L is chosen from the mean row length or by the autotuner.
+// lanes.  L is chosen from the mean row length or by the autotuner.  That
+// form serves FP64 vectors on matrices with long rows and what set_lanes or
+// the autotuner picks; a new operator's products run over row blocks.
 #include <algorithm>
 
 #include "spmv_stream.hpp"
@@ -118,14 +120,114 @@ static void launch_f64(const SparseRows &S, const double *x, double *y, hipStrea
     TV3_HIP(hipGetLastError());
 }
 
-void build_row_blocks(tv3_ctx *ctx, SparseRows &S, int blk_nnz,
-                      const std::vector<int64_t> *starts) {
+// Wavefront blocks: at most kWave rows and kWaveBlk entries, or one longer row.
+constexpr int kWave = 64, kWaveBlk = 256;
+static bool wave_blocks(const SparseRows &S) { return S.blk_nnz == kWaveBlk; }
+
+// Row blocks for one wavefront each: the block's (col, val) pairs are read
+// with unit stride, its products go to the wavefront's part of LDS, and
+// 1 << lg lanes sum each row.  Nothing waits for another wavefront, so the
+// phases of neighbouring blocks overlap; eight times smaller blocks than
+// k_csr_stream's also fill the chip more evenly when few are left.  A longer
+// row (a voxel next to a transducer) is summed lane by lane, J gathers in
+// flight.
+//
+// Bound by the line fills of the gathers (L2 -> L1, 128 B each, ~30 TB/s)
+// and, where x outgrows an L2 slice, by its misses.  us, against 2048-entry
+// blocks of a 256-thread workgroup: 64^3 voxels x 65,536 rays FP32 weights
+// A^T 27.0 -> 18.0, A 17.2 -> 17.0; 128^3 x 262,144 FP16 A^T 130 -> 107,
+// A 149 -> 148, FP64 A^T 298 -> 186, A 300 -> 260 (k_csr_f64).
+//
+// Acc = double also serves FP32 vectors whose row sums are rounded once.
+template <typename V, typename X, typename Acc>
+__global__ __launch_bounds__(256) void k_csr_wave(const BlkDesc *__restrict__ desc,
+                                                  const int32_t *__restrict__ ptr,
+                                                  const int32_t *__restrict__ ind,
+                                                  const V *__restrict__ val,
+                                                  const X *__restrict__ x, X *__restrict__ y,
+                                                  int nblk) {
+    constexpr int J = kWaveBlk / kWave;
+    __shared__ Acc products[256 / kWave][kWaveBlk];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int b = xcd_remap(blockIdx.x, gridDim.x) * (256 / kWave) + wave;
+    if (b >= nblk) return;
+    Acc *prod = products[wave];
+    const int t = threadIdx.x & (kWave - 1);
+    const BlkDesc d = desc[b];
+    const int L = 1 << d.lg, rr = t >> d.lg, lane = t & (L - 1);
+    const bool has = rr < d.nr;
+    const int row = d.r0 + (has ? rr : d.nr - 1);
+    const int end = d.p0 + d.len;
+    const int a = ptr[row], e = ptr[row + 1];
+    V w[J];
+    // J entries of this lane from entry k0 on, clamped to the block's last.
+    // Loads return in order, so with the weights requested first a gather
+    // starts when its entry's streams are in; earlier gathers crowd out the
+    // streams of other wavefronts.  A and A^T in turn, the matrices from HBM,
+    // 128^3, us (columns first -> weights first): FP16 310 -> 277, FP32 301 ->
+    // 296.
+    Acc p[J];
+    auto entries = [&](int k0) {
+#pragma unroll
+        for (int j = 0; j < J; ++j) w[j] = val[min(k0 + j * kWave + t, end - 1)];
+        __builtin_amdgcn_sched_barrier(0);
+        int c[J];
+#pragma unroll
+        for (int j = 0; j < J; ++j) c[j] = ind[min(k0 + j * kWave + t, end - 1)];
+#pragma unroll
+        for (int j = 0; j < J; ++j) p[j] = (Acc)x[c[j]];
+    };
+    if (d.len > 0) entries(d.p0);
+    auto weight = [](V v) {
+        if constexpr (std::is_same_v<V, double>) return v;
+        else return (Acc)to_f32(v);
+    };
+    Acc s = 0;
+    if (d.len <= kWaveBlk) {
+        if (d.len > 0) {
+#pragma unroll
+            for (int j = 0; j < J; ++j) prod[j * kWave + t] = weight(w[j]) * p[j];
+        }
+        // the wavefront's own LDS operations complete in order
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (has) s = row_sum<kWaveBlk>(prod, a - d.p0, e - d.p0, lane, L);
+    } else {
+        for (int k0 = d.p0;;) {
+#pragma unroll
+            for (int j = 0; j < J; ++j)
+                if (k0 + j * kWave + t < end) s = fma(weight(w[j]), p[j], s);
+            k0 += kWaveBlk;
+            if (k0 >= end) break;
+            entries(k0);
+        }
+    }
+    s = lane_sum(s, L);
+    if (has && lane == 0) y[row] = (X)s;
+}
+
+template <typename V, typename X, typename Acc>
+static void launch_wave(const SparseRows &S, const X *x, X *y, hipStream_t s) {
+    if (S.nblk == 0) return;
+    hipLaunchKernelGGL((k_csr_wave<V, X, Acc>), dim3((unsigned)((S.nblk + 3) / 4)), dim3(256), 0, s,
+                       S.desc.p, S.ptr.p, S.ind.p, reinterpret_cast<const V *>(S.val.p), x, y,
+                       (int)S.nblk);
+    TV3_HIP(hipGetLastError());
+}
+
+static std::vector<int32_t> row_pointers(tv3_ctx *ctx, const SparseRows &S) {
     std::vector<int32_t> ptr(S.rows + 1);
     TV3_HIP(hipMemcpyAsync(ptr.data(), S.ptr.p, sizeof(int32_t) * (S.rows + 1),
                            hipMemcpyDeviceToHost, ctx->stream));
     TV3_HIP(hipStreamSynchronize(ctx->stream));
+    return ptr;
+}
+
+static void row_blocks(tv3_ctx *ctx, SparseRows &S, int blk_nnz, const std::vector<int32_t> &ptr,
+                       const std::vector<int64_t> *starts) {
+    const int threads = blk_nnz == kWaveBlk ? kWave : 256;
     std::vector<int32_t> blk;
-    blk.reserve(S.nnz / (blk_nnz / 2) + S.rows / 256 + 2);
+    blk.reserve(S.nnz / (blk_nnz / 2) + S.rows / threads + 2);
     int64_t start = 0;
     size_t si = 0;   // next forced block start
     blk.push_back(0);
@@ -134,14 +236,14 @@ void build_row_blocks(tv3_ctx *ctx, SparseRows &S, int blk_nnz,
         const bool forced = starts && si < starts->size() && (*starts)[si] == r;
         // close the current block before row r if adding it would overflow
         if (r > start &&
-            (forced || (int64_t)ptr[r + 1] - ptr[start] > blk_nnz || r - start >= 256)) {
+            (forced || (int64_t)ptr[r + 1] - ptr[start] > blk_nnz || r - start >= threads)) {
             blk.push_back((int32_t)r);
             start = r;
         }
     }
     blk.push_back((int32_t)S.rows);
     S.nblk = (int64_t)blk.size() - 1;
-    const std::vector<BlkDesc> d = make_blk_desc(blk, ptr.data(), nullptr);
+    const std::vector<BlkDesc> d = make_blk_desc(blk, ptr.data(), nullptr, threads);
     S.desc.alloc(d.size());
     TV3_HIP(hipMemcpyAsync(S.desc.p, d.data(), sizeof(BlkDesc) * d.size(), hipMemcpyHostToDevice,
                            ctx->stream));
@@ -149,8 +251,25 @@ void build_row_blocks(tv3_ctx *ctx, SparseRows &S, int blk_nnz,
     S.blk_nnz = blk_nnz;
 }
 
+void build_row_blocks(tv3_ctx *ctx, SparseRows &S, int blk_nnz,
+                      const std::vector<int64_t> *starts) {
+    row_blocks(ctx, S, blk_nnz, row_pointers(ctx, S), starts);
+}
+
+// Wavefront blocks, unless a row is so long that one wavefront would still
+// sum it when the others are done (16 rounds of gathers): then 2048-entry
+// workgroup blocks.  Voxels next to a transducer are crossed by about 1,000
+// rays of 262,144.  A^T, us, 256 / 512 entries a wavefront: 64^3 voxels
+// 18.0 / 20.7, 96^3 49 / 49, 128^3 107 / 112.
+void build_default_blocks(tv3_ctx *ctx, SparseRows &S) {
+    const std::vector<int32_t> ptr = row_pointers(ctx, S);
+    int32_t longest = 0;
+    for (int64_t r = 0; r < S.rows; ++r) longest = std::max(longest, ptr[r + 1] - ptr[r]);
+    row_blocks(ctx, S, longest <= 16 * kWaveBlk ? kWaveBlk : 2048, ptr, nullptr);
+}
+
 std::vector<BlkDesc> make_blk_desc(const std::vector<int32_t> &blk, const int32_t *ptr,
-                                   const std::vector<int32_t> *pad_start) {
+                                   const std::vector<int32_t> *pad_start, int threads) {
     const size_t nb = blk.empty() ? 0 : blk.size() - 1;
     std::vector<BlkDesc> d(nb + 1);
     for (size_t b = 0; b < nb; ++b) {
@@ -163,7 +282,7 @@ std::vector<BlkDesc> make_blk_desc(const std::vector<int32_t> &blk, const int32_
         e.len = ptr[blk[b + 1]] - e.p0;
         e.q0 = pad_start ? (*pad_start)[b] : e.p0;
         int lg = 6;
-        while (lg > 0 && (1 << lg) * e.nr > 256) --lg;
+        while (lg > 0 && (1 << lg) * e.nr > threads) --lg;
         e.lg = lg;
         e.pad0 = e.pad1 = 0;
     }
@@ -177,6 +296,23 @@ std::vector<BlkDesc> make_blk_desc(const std::vector<int32_t> &blk, const int32_
 
 void spmv_csr(const SparseRows &S, const float *x, float *y, hipStream_t s, int lanes,
               bool acc64) {
+    if (!lanes && wave_blocks(S)) {
+        switch (S.vtype) {
+        case TV3_F32:
+            acc64 ? launch_wave<float, float, double>(S, x, y, s)
+                  : launch_wave<float, float, float>(S, x, y, s);
+            return;
+        case TV3_F16:
+            acc64 ? launch_wave<__half, float, double>(S, x, y, s)
+                  : launch_wave<__half, float, float>(S, x, y, s);
+            return;
+        case TV3_BF16:
+            acc64 ? launch_wave<__hip_bfloat16, float, double>(S, x, y, s)
+                  : launch_wave<__hip_bfloat16, float, float>(S, x, y, s);
+            return;
+        default: throw tv3_error(TV3_E_FORMAT, "FP32 products need F32, F16 or BF16 values");
+        }
+    }
     if (!lanes && S.blk_nnz) {
         if (acc64) launch_stream_any<double>(S, x, EpiStore<double>{y}, s);
         else launch_stream_any<float>(S, x, EpiStore<float>{y}, s);
@@ -201,6 +337,13 @@ void spmv_csr(const SparseRows &S, const float *x, float *y, hipStream_t s, int 
 
 void spmv_csr(const SparseRows &S, const double *x, double *y, hipStream_t s, int lanes,
               bool) {
+    if (!lanes && wave_blocks(S)) {
+        switch (S.vtype) {
+        case TV3_F64: launch_wave<double, double, double>(S, x, y, s); return;
+        case TV3_F32: launch_wave<float, double, double>(S, x, y, s); return;
+        default: throw tv3_error(TV3_E_FORMAT, "FP64 products need F64 or F32 values");
+        }
+    }
     int L = lanes ? lanes : (S.lanes ? S.lanes : default_lanes(S.rows, S.nnz));
     switch (S.vtype) {
     case TV3_F64: launch_f64<double>(S, x, y, s, L); break;
@@ -249,15 +392,16 @@ __device__ __forceinline__ float4 row_sum4(const float4 *prod, int a, int e, int
     return make_float4(s0.x + s1.x, s0.y + s1.y, s0.z + s1.z, s0.w + s1.w);
 }
 
-// k_csr_stream for KT columns: a row block's entries are read once, KT / 4
-// neighbouring lanes gather one entry's KT values (one line look-up serves
-// them), the products go to LDS, and 256 threads per four columns sum the
-// rows.  Every column is summed as k_csr_stream sums it (same bits).  Bound
+// k_csr_stream (W = 256) or k_csr_wave (W = 64) for KT columns: a row block's
+// entries are read once, KT / 4 neighbouring lanes gather one entry's KT
+// values (one line look-up serves them), the products go to LDS, and W
+// threads per four columns sum the rows.  Every column is summed as the
+// kernel for one vector sums it (same bits).  Bound
 // by the gathers of Xt: at 64^3 voxels and 65,536 rays, 8 columns, FP32
-// weights, A 30 us and A^T 59 us, Xt 3-7 us, against eight launches of 17 and
-// 27 us (43 and 81 us when a lane gathered an entry's values in turn).
-template <int NB, int KT, typename V>
-__global__ __launch_bounds__(64 * KT) void k_csr_multi(const BlkDesc *__restrict__ desc,
+// weights, Xt included, A 41 us and A^T 39 us (2048-entry blocks 43 and 68),
+// against eight launches of 17 and 18 us.
+template <int NB, int KT, int W, typename V>
+__global__ __launch_bounds__(W * KT / 4) void k_csr_multi(const BlkDesc *__restrict__ desc,
                                                        const int32_t *__restrict__ ptr,
                                                        const int32_t *__restrict__ ind,
                                                        const V *__restrict__ val,
@@ -266,27 +410,26 @@ __global__ __launch_bounds__(64 * KT) void k_csr_multi(const BlkDesc *__restrict
     constexpr int Q = KT / 4;                // quads of columns
     __shared__ float4 prod[Q][NB];
     const BlkDesc d = desc[xcd_remap(blockIdx.x, gridDim.x)];
-    const int t = threadIdx.x & 255, q2 = threadIdx.x >> 8;      // phase 2: thread, quad
+    const int t = threadIdx.x % W, q2 = threadIdx.x / W;         // phase 2: thread, quad
     const int L = 1 << d.lg, rr = t >> d.lg, lane = t & (L - 1);
     const bool has = rr < d.nr;
     const int row = d.r0 + (has ? rr : d.nr - 1);
     if (d.len <= NB) {
-        constexpr int J = NB / 256;
+        constexpr int J = NB / W;
         const int a = ptr[row] - d.p0, e = ptr[row + 1] - d.p0;
         if (d.len > 0) {
             const int q = threadIdx.x % Q, slot = threadIdx.x / Q, last = d.p0 + d.len - 1;
             int c[J];
-            float w[J];
+            V w[J];                          // weights first: see k_csr_wave
 #pragma unroll
-            for (int j = 0; j < J; ++j) {
-                const int k = min(d.p0 + j * 256 + slot, last);
-                c[j] = ind[k];
-                w[j] = ld_weight<V>(val, k);
-            }
+            for (int j = 0; j < J; ++j) w[j] = val[min(d.p0 + j * W + slot, last)];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < J; ++j) c[j] = ind[min(d.p0 + j * W + slot, last)];
 #pragma unroll
             for (int j = 0; j < J; ++j)
-                prod[q][j * 256 + slot] =
-                    w[j] * *reinterpret_cast<const float4 *>(Xt + (int64_t)c[j] * KT + 4 * q);
+                prod[q][j * W + slot] =
+                    to_f32(w[j]) * *reinterpret_cast<const float4 *>(Xt + (int64_t)c[j] * KT + 4 * q);
         }
         __syncthreads();
         float4 s = make_float4(0, 0, 0, 0);
@@ -295,6 +438,20 @@ __global__ __launch_bounds__(64 * KT) void k_csr_multi(const BlkDesc *__restrict
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             if (has && lane == 0 && 4 * q2 + j < G) Y[row + (4 * q2 + j) * ldy] = o[j];
+    } else if constexpr (W == kWave) {
+        // one row longer than NB, summed as k_csr_wave does
+        float s[4] = {};
+        for (int k = d.p0 + t; k < d.p0 + d.len; k += kWave) {
+            const float w = ld_weight<V>(val, k);
+            const float *x = Xt + (int64_t)ind[k] * KT + 4 * q2;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s[j] = fma(w, x[j], s[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            s[j] = lane_sum<kWave>(s[j]);
+            if (t == 0 && 4 * q2 + j < G) Y[row + (4 * q2 + j) * ldy] = s[j];
+        }
     } else {
         // one row longer than NB
         float s[4] = {};
@@ -322,27 +479,28 @@ bool spmv_multi_ok(const SparseRows &S) {
 
 size_t spmv_multi_scratch(const SparseRows &S) { return (size_t)S.cols * 8; }
 
+template <int NB, int KT, int W, typename V>
+static void launch_blocks(const SparseRows &S, int G, const float *xt, float *Y, int64_t ldy,
+                          hipStream_t s) {
+    hipLaunchKernelGGL((k_csr_multi<NB, KT, W, V>), dim3((unsigned)S.nblk), dim3(W * KT / 4), 0, s,
+                       S.desc.p, S.ptr.p, S.ind.p, reinterpret_cast<const V *>(S.val.p), xt, Y, ldy,
+                       G);
+}
+
 template <int KT, typename V>
 static void launch_multi(const SparseRows &S, int G, const float *xt, float *Y, int64_t ldy,
                          hipStream_t s) {
-    const dim3 g((unsigned)S.nblk);
-    const V *val = reinterpret_cast<const V *>(S.val.p);
-#define TV3_MCASE(NBV)                                                                        \
-    case NBV:                                                                                 \
-        hipLaunchKernelGGL((k_csr_multi<NBV, KT, V>), g, dim3(64 * KT), 0, s, S.desc.p,        \
-                           S.ptr.p, S.ind.p, val, xt, Y, ldy, G);                             \
-        return;
     switch (S.blk_nnz) {
-        TV3_MCASE(1024) TV3_MCASE(2048)
+    case kWaveBlk: launch_blocks<kWaveBlk, KT, kWave, V>(S, G, xt, Y, ldy, s); return;
+    case 1024: launch_blocks<1024, KT, 256, V>(S, G, xt, Y, ldy, s); return;
+    case 2048: launch_blocks<2048, KT, 256, V>(S, G, xt, Y, ldy, s); return;
     case 4096:           // 64 KB of products for four columns
         if constexpr (KT == 4) {
-            hipLaunchKernelGGL((k_csr_multi<4096, KT, V>), g, dim3(64 * KT), 0, s, S.desc.p, S.ptr.p,
-                               S.ind.p, val, xt, Y, ldy, G);
+            launch_blocks<4096, KT, 256, V>(S, G, xt, Y, ldy, s);
             return;
         }
     default: throw tv3_error(TV3_E_ARG, "stream block size must be 1024, 2048 or 4096");
     }
-#undef TV3_MCASE
 }
 
 template <int KT>
@@ -629,7 +787,7 @@ void build_transpose(tv3_ctx *ctx, const SparseRows &A, SparseRows &AT) {
     TV3_HIP(hipGetLastError());
     TV3_HIP(hipStreamSynchronize(s));
     AT.lanes = default_lanes(AT.rows, AT.nnz);
-    build_row_blocks(ctx, AT, 2048);
+    build_default_blocks(ctx, AT);
 }
 
 }  // namespace tv3

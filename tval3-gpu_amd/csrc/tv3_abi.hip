@@ -254,7 +254,7 @@ const char *tv3_last_error(const tv3_ctx *ctx) {
 void *tv3_ctx_stream(tv3_ctx *ctx) { return ctx ? (void *)ctx->stream : nullptr; }
 
 // host rows (CSR of A, or its CSC as the CSR of A^T) to the device, with the
-// default launch shape and 2048-entry row blocks
+// default launch shape and row blocks
 static void upload_rows(tv3_ctx *ctx, SparseRows &R, int64_t rows, int64_t cols, int64_t nnz,
                         const int32_t *ptr, const int32_t *ind, const void *val, tv3_dtype vt) {
     hipStream_t s = ctx->stream;
@@ -263,7 +263,7 @@ static void upload_rows(tv3_ctx *ctx, SparseRows &R, int64_t rows, int64_t cols,
     upload(R.ind, ind, nnz, s);
     upload_bytes(R.val, val, nnz * dtype_size(vt), s);
     R.lanes = default_lanes(rows, nnz);
-    build_row_blocks(ctx, R, 2048);
+    build_default_blocks(ctx, R);
 }
 
 tv3_status tv3_op_csr_create(tv3_ctx *ctx, int64_t m, int64_t n, int64_t nnz,
@@ -818,11 +818,13 @@ tv3_status tv3_op_autotune(tv3_op *op, int32_t *lanes_N, int32_t *lanes_T) {
         TV3_HIP(hipMemsetAsync(x.p, 0, x.bytes(), op->ctx->stream));
         DevBuf<float> xm(op->m);
         TV3_HIP(hipMemsetAsync(xm.p, 0, xm.bytes(), op->ctx->stream));
-        // candidates: row-blocked stream kernel with 1024/2048/4096-entry
-        // blocks (reported as -NB) and the row-group kernel with L lanes
+        // candidates: a new operator's row blocks (reported as 0), the
+        // row-blocked stream kernel with 1024/2048/4096-entry blocks
+        // (reported as -NB) and the row-group kernel with L lanes
         auto best = [&](SparseRows &S, const float *xx) {
             int choice = 0;
-            float bt = 1e30f;
+            build_default_blocks(op->ctx, S);
+            float bt = time_spmv(op->ctx, S, 0, xx, y.p);
             for (int nb : {1024, 2048, 4096}) {
                 build_row_blocks(op->ctx, S, nb);
                 float t = time_spmv(op->ctx, S, 0, xx, y.p);
@@ -832,7 +834,9 @@ tv3_status tv3_op_autotune(tv3_op *op, int32_t *lanes_N, int32_t *lanes_T) {
                 float t = time_spmv(op->ctx, S, L, xx, y.p);
                 if (t < bt) { bt = t; choice = L; }
             }
-            if (choice < 0) {
+            if (choice == 0) {
+                build_default_blocks(op->ctx, S);
+            } else if (choice < 0) {
                 build_row_blocks(op->ctx, S, -choice);
             } else {
                 S.lanes = choice;

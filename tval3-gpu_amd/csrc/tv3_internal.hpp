@@ -141,7 +141,7 @@ enum class OpKind { CSR, DENSE, DYNAMIC, HYBRID };
 // scalar load: rows [r0, r0 + nr), entries [p0, p0 + len) of the CSR arrays
 // (q0: the block's first entry in a padded entry array, = p0 when none), lg =
 // log2 of the lanes per row in phase 2 (the largest power of two <= 64 with
-// (1 << lg) * nr <= 256).
+// (1 << lg) * nr <= the threads of a block: 256, or 64 in wavefront blocks).
 struct BlkDesc {
     int32_t r0, nr, p0, len, q0, lg, pad0, pad1;
 };
@@ -149,7 +149,7 @@ struct BlkDesc {
 // Descriptors of the row blocks whose first rows are blk[0 .. nb) (blk[nb] =
 // end), plus one empty sentinel so that block b + 1 can always be read.
 std::vector<BlkDesc> make_blk_desc(const std::vector<int32_t> &blk, const int32_t *ptr,
-                                   const std::vector<int32_t> *pad_start);
+                                   const std::vector<int32_t> *pad_start, int threads = 256);
 
 // Compressed sparse rows of a matrix (also used for the CSC = CSR of A^T).
 struct SparseRows {
@@ -159,7 +159,8 @@ struct SparseRows {
     DevBuf<uint8_t> val;   // nnz * dtype_size(vtype)
     int lanes = 0;         // row-group kernel: lanes per row (power of two <= 64)
     // row-blocked ("stream") kernel: blocks of consecutive rows holding at most
-    // blk_nnz entries (or one longer row); blk[b] = first row of block b
+    // blk_nnz entries (or one longer row); blk[b] = first row of block b.
+    // 256: wavefront blocks (at most 64 rows).
     int blk_nnz = 0;       // 0: use the row-group kernel
     int64_t nblk = 0;
     DevBuf<BlkDesc> desc;  // nblk + 1 (sentinel)
@@ -169,6 +170,8 @@ struct SparseRows {
 // starts (sorted, optional): rows where a block must begin.
 void build_row_blocks(tv3_ctx *ctx, SparseRows &S, int blk_nnz,
                       const std::vector<int64_t> *starts = nullptr);
+// The blocks a new operator's products run with.
+void build_default_blocks(tv3_ctx *ctx, SparseRows &S);
 
 // The parts of a geometry's rays inside boxes of kRayBox{Y,X,Z} voxels, for
 // the A^T products of dynamic.hip: built on the device when a matrix-free
