@@ -9,7 +9,7 @@
 //    update_W read V on a stream that did not wait for its producer);
 //  * lam2/lam4 use all three components with sigma in X,Y,Z order;
 //  * inner products accumulate in FP64 (block partials summed in a fixed
-//    order on the host), scalars are FP64, and every entry of a product
+//    order), scalars are FP64, and every entry of a product
 //    A x is summed in FP64 and rounded once, so the FP32 iterates restate
 //    the oracle's rounding instead of the accumulation order of a library;
 //  * vector kernels are compiled without FP contraction (a*x+y rounds
@@ -19,7 +19,7 @@
 //    consequences with every sum the next decision needs), each element
 //    computed and rounded as by one kernel per operation; an iteration
 //    without backtracking waits for the device once, and the previous iterate
-//    is kept by exchanging buffers (64^3 voxels, 65,536 rays: 95 us an
+//    is kept by exchanging buffers (64^3 voxels, 65,536 rays: 70 us an
 //    iteration against 270 us with one kernel per operation and a wait per
 //    inner product);
 //  * the work vectors stay with the context (the reference allocates and
@@ -130,10 +130,14 @@ struct PlainState {
         }
         if (mul) A(true, Au[0], g[0]);
         else copy(g[0], g[1], n);          // g stays as it was
-        queue_gradient<T>(S, fields(), mul ? g[0] : nullptr, Atb);
-        queue_lam35<T>(S, m, Au[0], bs, delta);
+        T *gm = mul ? g[0] : nullptr;
+        if (ahead) {
+            queue_trial<T>(S, fields(), gm, Atb, m, Au[0], bs, delta, next_fields(), iso(), beta);
+            queue_next(S);
+        } else {
+            queue_gradient<T>(S, fields(), gm, Atb, m, Au[0], bs, delta);
+        }
         last_mul = mul;
-        if (ahead) queue_W(S);
         const double *v = S.fetch();
         set_f(v);
         return v + 4;
@@ -182,12 +186,19 @@ struct PlainState {
     // search of the trial is decided (nearly every trial is accepted; an
     // iteration then waits for the device once).
     void queue_W(Sums &S) {
+        queue_shrink<T>(S, next_fields(), iso(), beta);
+        queue_next(S);
+    }
+    void queue_next(Sums &S) {
+        queue_update<T>(S, next_fields(), g[0], g[1], g2[1], DtsAtd, U[0], U[1], muDbeta, d[1]);
+    }
+    PlainFields<T> next_fields() {
         PlainFields<T> F = fields();
         F.Wx = Wx[1]; F.Wy = Wy[1]; F.Wz = Wz[1];
         F.g2 = g2_next;
-        queue_shrink<T>(S, F, o->tv_mode == TV3_TV_ISO, beta);
-        queue_update<T>(S, F, g[0], g[1], g2[1], DtsAtd, U[0], U[1], muDbeta, d[1]);
+        return F;
     }
+    int iso() const { return o->tv_mode == TV3_TV_ISO; }
     void take_W(const double *v) {
         f -= (lam1 + beta / 2 * lam2 - lam4);
         lam1 = v[0]; lam2 = v[1]; lam4 = v[2];

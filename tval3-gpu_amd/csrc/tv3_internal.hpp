@@ -371,6 +371,12 @@ inline uint64_t next_op_uid() {
     static std::atomic<uint64_t> counter{0};
     return ++counter;
 }
+
+// a sum left for the host, and the number of the fetch it belongs to
+struct SumResult {
+    double value;
+    uint64_t ticket;
+};
 }  // namespace tv3
 
 struct tv3_ctx {
@@ -379,7 +385,9 @@ struct tv3_ctx {
     std::string err;
     int num_cus = 256;
     size_t lds_per_block = 65536;   // largest LDS allocation of one workgroup
-    tv3::PinnedBuf<double> red_host;   // block partials of the sums (vec.hpp)
+    tv3::DevBuf<double> red_part;      // block partials of the sums (vec.hpp)
+    tv3::PinnedBuf<tv3::SumResult> red_host;   // their totals
+    uint64_t red_ticket = 0;           // number of the last fetch
     // The vectors of a plain solve and the device copies of a host solve's b, U
     // and U_true, grown to the largest solve so far (a solve waits for its
     // stream before it returns, and a context serves one host thread)

@@ -6,6 +6,8 @@
 // D :170-215, D^T :479-510, lam2/lam4 :724-771 (all three components, sigma
 // in X,Y,Z order), lam3/lam5 :876-919, BB step :1017-1067, nonneg
 // :1176-1188, shrinkage :1249-1300 (plus the isotropic variant).
+#include <chrono>
+
 #include "vec.hpp"
 
 namespace tv3 {
@@ -286,17 +288,16 @@ template <typename T, typename I> struct FUpdate {
     }
 };
 
-// Block partials of K sums, a block's K values side by side: they go straight
-// to pinned host memory (one line a block, so a fetch waits for the kernel
-// only: no copy behind it).
+// Block partials of K sums over n items by workgroup b of nb, a workgroup's K
+// values side by side.
 template <int K, typename F>
-__global__ __launch_bounds__(256) void k_reduce(int64_t n, F f, double *partials) {
+__device__ __forceinline__ void reduce_items(int64_t n, const F &f, int b, int nb,
+                                             double *partials) {
     __shared__ double sh[K][4];
     double acc[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) acc[k] = 0.0;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
-        f(i, acc);
+    for (int64_t i = (int64_t)b * 256 + threadIdx.x; i < n; i += (int64_t)nb * 256) f(i, acc);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -306,40 +307,116 @@ __global__ __launch_bounds__(256) void k_reduce(int64_t n, F f, double *partials
     __syncthreads();
     if (threadIdx.x < K) {
         const double *w = sh[threadIdx.x];
-        partials[(int64_t)blockIdx.x * K + threadIdx.x] = (w[0] + w[1]) + (w[2] + w[3]);
+        partials[(int64_t)b * K + threadIdx.x] = (w[0] + w[1]) + (w[2] + w[3]);
     }
+}
+
+template <int K, typename F>
+__global__ __launch_bounds__(256) void k_reduce(int64_t n, F f, double *partials) {
+    reduce_items<K>(n, f, blockIdx.x, gridDim.x, partials);
+}
+
+// Three reductions that do not depend on each other, one behind the other in
+// the grid: a launch of its own for each costs 4 us of a 64^3 iteration's 70.
+template <int K1, typename F1, int K2, typename F2, int K3, typename F3>
+__global__ __launch_bounds__(256) void k_reduce3(int64_t n1, F1 f1, int nb1, int64_t n2, F2 f2,
+                                                 int nb2, int64_t n3, F3 f3, int nb3,
+                                                 double *partials) {
+    const int b = blockIdx.x;
+    if (b < nb1)
+        reduce_items<K1>(n1, f1, b, nb1, partials);
+    else if (b < nb1 + nb2)
+        reduce_items<K2>(n2, f2, b - nb1, nb2, partials + (int64_t)K1 * nb1);
+    else
+        reduce_items<K3>(n3, f3, b - nb1 - nb2, nb3,
+                         partials + (int64_t)K1 * nb1 + (int64_t)K2 * nb2);
+}
+
+// One workgroup a sum: adds its block partials in a fixed order and leaves
+// the value in pinned host memory, then the ticket that says so.  (With the
+// partials themselves in pinned memory the host read and added up to 9,700 of
+// them an iteration while the device idled; see Sums.)
+struct SumList {
+    int first[kSumMax], stride[kSumMax], blocks[kSumMax];
+};
+__global__ __launch_bounds__(256) void k_sum_blocks(SumList L, const double *partials,
+                                                    SumResult *out, uint64_t ticket) {
+    __shared__ double sh[4];
+    const int j = blockIdx.x, blocks = L.blocks[j], stride = L.stride[j];
+    const double *p = partials + L.first[j];
+    double v = 0.0;
+    for (int b = threadIdx.x; b < blocks; b += 256) v += p[(int64_t)b * stride];
+    v = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        out[j].value = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+        __hip_atomic_store(&out[j].ticket, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+static int sum_blocks(int64_t n) {
+    return (int)std::min<int64_t>(std::max<int64_t>((n + 255) / 256, 1), kSumBlocks);
+}
+
+// room for the block partials of K more sums over n items
+template <int K>
+static double *place_sums(Sums &S, int64_t n) {
+    tv3_ctx *ctx = S.ctx;
+    if (!ctx->red_part.p) {
+        ctx->red_part.alloc((size_t)kSumMax * kSumBlocks);
+        ctx->red_host.alloc(kSumMax);
+        for (int j = 0; j < kSumMax; ++j) ctx->red_host.p[j].ticket = 0;
+    }
+    TV3_REQUIRE(S.count + K <= kSumMax, TV3_E_INTERNAL, "too many sums at once");
+    const int nb = sum_blocks(n);
+    double *p = ctx->red_part.p + S.used;
+    for (int k = 0; k < K; ++k) S.sum[S.count++] = {(int)S.used + k, K, nb};
+    S.used += (size_t)K * nb;
+    return p;
 }
 
 // queues the block partials of K sums over n items
 template <int K, typename F>
 static void queue_sums(Sums &S, int64_t n, const F &f) {
-    int64_t nb = (n + 255) / 256;
-    if (nb > kSumBlocks) nb = kSumBlocks;
-    if (nb < 1) nb = 1;
-    tv3_ctx *ctx = S.ctx;
-    ctx->red_host.alloc((size_t)kSumMax * kSumBlocks);
-    TV3_REQUIRE(S.count + K <= kSumMax, TV3_E_INTERNAL, "too many sums at once");
-    hipLaunchKernelGGL((k_reduce<K, F>), dim3((unsigned)nb), dim3(256), 0, S.s, n, f,
-                       ctx->red_host.p + S.used);
-    S.group[S.groups++] = {K, (int)nb};
-    S.count += K;
-    S.used += (size_t)K * nb;
+    double *p = place_sums<K>(S, n);
+    hipLaunchKernelGGL((k_reduce<K, F>), dim3((unsigned)sum_blocks(n)), dim3(256), 0, S.s, n, f, p);
 }
 
-const double *Sums::fetch() {
-    TV3_HIP(hipGetLastError());
-    TV3_HIP(hipStreamSynchronize(s));
-    const double *h = ctx->red_host.p;
-    double *out = value;
-    for (int g = 0; g < groups; ++g) {
-        const int K = group[g].sums;
-        for (int k = 0; k < K; ++k) out[k] = 0.0;
-        for (int b = 0; b < group[g].blocks; ++b, h += K)
-            for (int k = 0; k < K; ++k) out[k] += h[k];
-        out += K;
+static inline void cpu_pause() {
+#if defined(__x86_64__)
+    __builtin_ia32_pause();
+#endif
+}
+
+const double *Sums::fetch(bool drain) {
+    SumList L{};
+    for (int j = 0; j < count; ++j) {
+        L.first[j] = sum[j].first;
+        L.stride[j] = sum[j].stride;
+        L.blocks[j] = sum[j].blocks;
     }
+    const uint64_t ticket = ++ctx->red_ticket;
+    SumResult *out = ctx->red_host.p;
+    hipLaunchKernelGGL(k_sum_blocks, dim3((unsigned)count), dim3(256), 0, s, L, ctx->red_part.p, out,
+                       ticket);
+    TV3_HIP(hipGetLastError());
+    auto landed = [&] {
+        for (int j = 0; j < count; ++j)
+            if (__atomic_load_n(&out[j].ticket, __ATOMIC_ACQUIRE) != ticket) return false;
+        return true;
+    };
+    // a bounded watch of the tickets, then the stream's own wait (which also
+    // reports a failed launch)
+    bool there = false;
+    if (!drain) {
+        const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+        while (!(there = landed()) && std::chrono::steady_clock::now() < until) cpu_pause();
+    }
+    if (!there) TV3_HIP(hipStreamSynchronize(s));
+    for (int j = 0; j < count; ++j) value[j] = out[j].value;
     used = 0;
-    count = groups = 0;
+    count = 0;
     return value;
 }
 
@@ -347,7 +424,7 @@ template <int K, typename F>
 std::array<double, K> reduce_now(tv3_ctx *ctx, int64_t n, const F &f, hipStream_t s) {
     Sums S{ctx, s};
     queue_sums<K>(S, n, f);
-    const double *v = S.fetch();
+    const double *v = S.fetch(/*drain=*/true);
     std::array<double, K> out{};
     for (int k = 0; k < K; ++k) out[k] = v[k];
     return out;
@@ -408,11 +485,33 @@ void queue_dot(Sums &S, int64_t n, const T *a, const T *b) {
 }
 
 template <typename T>
-void queue_gradient(Sums &S, const PlainFields<T> &f, T *g, const T *Atb) {
+void queue_gradient(Sums &S, const PlainFields<T> &f, T *g, const T *Atb, int64_t m, const T *Au,
+                    const T *b, const T *delta) {
     with_grid(f.dims, [&](auto G) {
         using I = decltype(G.p);
         queue_sums<2>(S, f.n, FGradient<T, I>{G, f.Ux, f.Uy, f.Uz, f.Wx, f.Wy, f.Wz, f.sx, f.sy,
                                               f.sz, Atb, f.g2, g});
+    });
+    queue_lam35<T>(S, m, Au, b, delta);
+}
+
+template <typename T>
+void queue_trial(Sums &S, const PlainFields<T> &f, T *g, const T *Atb, int64_t m, const T *Au,
+                 const T *b, const T *delta, const PlainFields<T> &next, int iso, double beta) {
+    const FLam35<T> f2{Au, b, delta};
+    const FShrink<T> f3{next.Ux, next.Uy, next.Uz, next.sx, next.sy, next.sz, (T)beta, iso,
+                        next.Wx, next.Wy, next.Wz};
+    with_grid(f.dims, [&](auto G) {
+        using I = decltype(G.p);
+        using F1 = FGradient<T, I>;
+        const F1 f1{G, f.Ux, f.Uy, f.Uz, f.Wx, f.Wy, f.Wz, f.sx, f.sy, f.sz, Atb, f.g2, g};
+        double *p = place_sums<2>(S, f.n);
+        place_sums<2>(S, m);
+        place_sums<1>(S, f.n);
+        const int nb1 = sum_blocks(f.n), nb2 = sum_blocks(m);
+        hipLaunchKernelGGL((k_reduce3<2, F1, 2, FLam35<T>, 1, FShrink<T>>),
+                           dim3((unsigned)(2 * nb1 + nb2)), dim3(256), 0, S.s, f.n, f1, nb1, m, f2,
+                           nb2, f.n, f3, nb1, p);
     });
 }
 
@@ -486,7 +585,11 @@ std::array<double, 2> diff_norm(tv3_ctx *ctx, int64_t n, const T *a, const T *b,
                                   T *, T *, hipStream_t);                                       \
     template void queue_step<T>(Sums &, const int32_t *, const T *);                            \
     template void queue_dot<T>(Sums &, int64_t, const T *, const T *);                          \
-    template void queue_gradient<T>(Sums &, const PlainFields<T> &, T *, const T *);            \
+    template void queue_gradient<T>(Sums &, const PlainFields<T> &, T *, const T *, int64_t,    \
+                                    const T *, const T *, const T *);                          \
+    template void queue_trial<T>(Sums &, const PlainFields<T> &, T *, const T *, int64_t,       \
+                                 const T *, const T *, const T *, const PlainFields<T> &, int,  \
+                                 double);                                                       \
     template void queue_lam24<T>(Sums &, const PlainFields<T> &);                               \
     template void queue_lam35<T>(Sums &, int64_t, const T *, const T *, const T *);             \
     template void queue_shrink<T>(Sums &, const PlainFields<T> &, int, double);                 \
