@@ -319,7 +319,9 @@ __global__ __launch_bounds__(kBoxThreads) void k_box_T(GeoView g, int nby, int n
             if (cur.xr != 0) {
                 if constexpr (SID) {
                     dyn_seg_walk(DynSeg{cur.ra, cur.rb, cur.amax, (int)cur.sg.y}, P,
-                                 [&](int i, float w) { atomicAdd(&box[i], (double)((T)w * cur.xr)); });
+                                 [&](int i, float w, bool on) {
+                                     if (on) atomicAdd(&box[i], (double)((T)w * cur.xr));
+                                 });
                 } else {
                     const double v = (double)(cur.xr * (T)g.scale);
                     BresWalk w(cur.w, cur.sg.y & 0xffff, kRayBoxY, 1, kRayBoxY * kRayBoxXZ);

@@ -19,23 +19,11 @@
 #include <algorithm>
 #include <numeric>
 
-// build-time tuning of the A^T boxes: workgroup size, and the entries one
-// box keeps in LDS where a workgroup may hold 160 KiB (15360 otherwise).
-// 512 threads and 19456 entries (76 KiB) let two workgroups share a CU, one
-// walking while the other sums: measured at 128^3 with 262144 rays, 238 us
-// against 302 us for one 1024-thread workgroup holding 32768 entries.
-#ifndef TV3_DYN_T_THREADS
-#define TV3_DYN_T_THREADS 512
-#endif
+// The entries one A^T box keeps in LDS where a workgroup may hold 160 KiB
+// (15360 otherwise): 19456 entries (76 KiB) let two workgroups share a CU,
+// one walking while the other sums.
 #ifndef TV3_DYN_EMAX_BIG
 #define TV3_DYN_EMAX_BIG 19456
-#endif
-// work items of the A x boxes of 16^3 voxels: this many times the segments
-// and entries of a two-tile box's item (each item stages its box's 4,096
-// voxels).  Measured at 128^3: A 85-87 us with 1, 77 with 2, 73 with 4, 77
-// with 6, 83 with 8 (two-tile boxes: 81-83 us).
-#ifndef TV3_DYN_CHUNK16
-#define TV3_DYN_CHUNK16 4
 #endif
 
 #include "panels.hpp"
@@ -269,19 +257,25 @@ void finish_boxes(tv3_ctx *ctx, std::vector<DynPan> &pan, const SegPlan &S,
     }
     if (!offsets) {
         // A x: a box's segments in chunks of at most 512 segments and about
-        // 6,144 entries (TV3_DYN_CHUNK16 times that in boxes of 16^3 voxels),
-        // one workgroup each (it stages the box's voxels, and each segment's
-        // partial sum is its own), so that the heaviest boxes do not run long
-        // chains after the others have ended
+        // 6,144 entries, one workgroup each (it stages the box's voxels, and
+        // each segment's partial sum is its own), so that the heaviest boxes
+        // do not run long chains after the others have ended.
+        // Boxes of 16^3 voxels: up to four times that (each item stages the
+        // box's 4,096 voxels), but about five items a CU.  A x, us, with 1, 2,
+        // 4 times, 64^3 / 96^3 / 128^3: 21, 27, 36 / 40, 38, 44 / 77, 68, 64.
+        int64_t entries = 0;
+        for (const DynPan &P : pan) entries += P.ne;
+        const float scale16 =
+            std::min(4.f, std::max(1.f, (float)entries / (6144.f * 5 * ctx->num_cus)));
         std::vector<DynPan> items;
         for (const DynPan &P : pan) {
-            const int scale = P.bs == 16 ? TV3_DYN_CHUNK16 : 1;
+            const float scale = P.bs == 16 ? scale16 : 1;
             int32_t sg = P.s0;
             while (sg < P.s1) {
                 DynPan c = P;
                 c.s0 = sg;
                 int32_t e = 0;
-                while (sg < P.s1 && sg - c.s0 < 512 * scale && e < 6144 * scale)
+                while (sg < P.s1 && sg - c.s0 < (int)(512 * scale) && e < (int)(6144 * scale))
                     e += S.seg_len[sg++];
                 c.s1 = sg;
                 c.ne = e;
@@ -340,7 +334,6 @@ std::unique_ptr<FusedLayout> build_dyn_layout(tv3_op *op) {
     // devices that allow 160 KiB per workgroup hold whole tiles
     const size_t lds = std::min<size_t>(ctx->lds_per_block, size_t(160) << 10);
     D->emax_cap = lds >= (size_t(150) << 10) ? TV3_DYN_EMAX_BIG : 15360;
-    D->threads_T = TV3_DYN_T_THREADS;
     const int B = L->B, nby = L->nby, nbx = L->nbx;   // tiles (B = 8) or bricks (B = 4)
     const int64_t nunit = n / (B == 8 ? 512 : 64);
     const int ushift = B == 8 ? 9 : 6;

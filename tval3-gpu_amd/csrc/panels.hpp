@@ -580,8 +580,8 @@ __host__ __device__ __forceinline__ void dyn_local_xyz(int i, int &x, int &y, in
 
 // The traversal of one segment (the part of an internal ray inside box P,
 // starting in the voxel of box-local coordinates c0 = x | y << 4 | z << 8):
-// emit(offset of the voxel in the box, length) in traversal order, the
-// offset in linear box order y + ey x + ey bs z (edges bs, ey, bs along x,
+// emit(offset of the voxel in the box, length, whether the length is
+// positive: only then it is an entry) in traversal order, the offset in linear box order y + ey x + ey bs z (edges bs, ey, bs along x,
 // y, z).  These are the entries the
 // walk of the whole ray (sid_walk, siddon.hpp) emits inside the box:
 //   * the ray record holds sid_setup's A, B, L, amin, amax (12 words:
@@ -592,7 +592,7 @@ __host__ __device__ __forceinline__ void dyn_local_xyz(int i, int &x, int &y, in
 //     parameter not above it, as in sid_box;
 //   * it ends at min(amax, t of the box's exit plane per axis);
 //   * each step is sid_walk's: the nearest next plane, the length
-//     (t_next - t_cur) L emitted when positive, every axis whose next plane
+//     (t_next - t_cur) L an entry when positive, every axis whose next plane
 //     is crossed at t_next advanced; the plane parameters are the same fused
 //     operation on the same values.  A parallel axis has A = 0, B = +inf, so
 //     its next plane never comes; no plane beyond the box's exit is ever
@@ -632,25 +632,21 @@ __host__ __device__ __forceinline__ void dyn_seg_walk(const DynSeg &sr, const Dy
         st[a] = up ? 1.f : (par ? 0.f : -1.f);
         kf[a] = (float)(up ? c + 1 : c);
         tk[a] = sid_fma(kf[a], A[a], B[a]);
-        if (!par) {
-            const float tin = sid_fma((float)(up ? c : c + 1), A[a], B[a]);
-            const float tout = sid_fma((float)(up ? b0[a] + ext[a] : b0[a]), A[a], B[a]);
-            ts = tin > ts ? tin : ts;
-            te = tout < te ? tout : te;
-        }
+        const float tin = sid_fma((float)(up ? c : c + 1), A[a], B[a]);
+        const float tout = sid_fma((float)(up ? b0[a] + ext[a] : b0[a]), A[a], B[a]);
+        ts = !par && tin > ts ? tin : ts;
+        te = !par && tout < te ? tout : te;
         off += lc[a] * stride[a];
         dstep[a] = up ? stride[a] : (par ? 0 : -stride[a]);
     }
     // the offset is masked all the same, so that no index leaves the box
     const int mask = ey * bs * P.ez - 1;
     float tcur = ts;
-    for (int step = 0; step < 2 * bs + ey + 4; ++step) {
-        float tnext = te;
-#pragma unroll
-        for (int a = 0; a < 3; ++a) tnext = tk[a] < tnext ? tk[a] : tnext;
+    for (int left = 2 * bs + ey + 4;;) {
+        const float tnext = __builtin_fminf(__builtin_fminf(te, tk[0]), __builtin_fminf(tk[1], tk[2]));
         const float seg = (tnext - tcur) * ra.w;
-        if (seg > 0) emit(off & mask, seg);
-        if (!(tnext < te)) break;
+        emit(off & mask, seg, seg > 0);
+        const bool more = tnext < te;
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
             const bool m = tk[a] == tnext;
@@ -659,6 +655,7 @@ __host__ __device__ __forceinline__ void dyn_seg_walk(const DynSeg &sr, const Dy
             tk[a] = sid_fma(kf[a], A[a], B[a]);
         }
         tcur = tnext;
+        if (!(more && --left > 0)) break;
     }
 }
 
@@ -701,39 +698,63 @@ __global__ __launch_bounds__(256) void k_dyn_tile_N(DynView g, const T *__restri
     for (int sg = P.s0 + t; sg < P.s1; sg += 256) {
         T acc = 0;
         dyn_seg_walk(g, P, g.seg_ray[sg], g.seg_c0[sg],
-                     [&](int li, float w) { acc += (T)w * xs[li]; });
+                     [&](int li, float w, bool on) {
+                         const T sum = acc + (T)w * xs[li];
+                         acc = on ? sum : acc;
+                     });
         part[sg] = acc;
     }
 }
 
 // A^T r: per box each thread walks segments and writes w r_ray at the
-// entry's position in the box's entry array in LDS (ray-major, emax_cap + 1
-// slots); then each voxel row sums its entries in ray order through the
-// stored positions (padding points at the zero slot ne) and the epilogue
-// takes the sum.
+// entry's position in the box's entry array in LDS (ray-major, emax_cap + 2
+// slots); then NT / (voxels of the box) lanes share a voxel, sum its entries
+// through the stored positions (each lane every LR-th group of four, in ray
+// order; padding points at the zero slot ne) and the epilogue takes the sum.
+//
+// The walks are bound by their vector instructions (25 a step), the sums by
+// the latency of positions (memory) and entries (LDS): both want many
+// wavefronts, so a workgroup has 1024 threads of at most 64 registers and two
+// share a CU (and its LDS), and each lane has kDynPosBatch groups of
+// positions, the first batch before the walks, and their LDS reads in
+// flight.  Siddon, A^T, us, 96^3 voxels x 147,456 rays / 128^3 x 262,144 /
+// 64^3 x 65,536: 49 / 96 / 24; with 512 threads 60 / 114 / 31; with 4 or 8
+// groups 50 / 99 / 25; one group at a time 86 / 157 / 43 (512 threads).
+constexpr int kDynPosBatch = 6, kDynThreadsT = 1024;
 template <typename T, int NT, typename Epi>
-__global__ __launch_bounds__(NT) void k_dyn_tile_T(DynView g, const T *__restrict__ x, Epi epi) {
+__global__ __launch_bounds__(NT, NT / 128) void k_dyn_tile_T(DynView g, const T *__restrict__ x,
+                                                             Epi epi) {
     static_assert(ExtraBlocks<Epi>::value == 0, "no extra workgroups in the tile product");
     extern __shared__ __align__(16) unsigned char dyn_smem[];
     if (epi.skip()) return;
-    static_assert(NT >= 512, "one voxel row per thread (boxes of at most 8^3)");
+    static_assert(NT >= 512, "a lane for every voxel row (boxes of at most 8^3)");
     const DynPan P = g.pan[g.order[blockIdx.x]];
     T *pe = reinterpret_cast<T *>(dyn_smem);
     const int t = threadIdx.x, ns = P.s1 - P.s0, nv = P.ey * P.bs * P.ez;
     // phase 2's operands do not depend on phase 1: its row starts, first
     // positions and epilogue operands are requested before the walks
-    const bool has_row = t < nv;
-    const int row = P.v0 + (has_row ? t : 0);
+    const int lg = min(6, 31 - __clz(NT / nv));        // nv is 512, 256 or 64
+    const int LR = 1 << lg, lane = t & (LR - 1);
+    const bool has_row = t >> lg < nv;
+    const int row = P.v0 + (has_row ? t >> lg : 0);
     uint32_t q0 = 0, q1 = 0;
     if (has_row) {
-        q0 = g.pptr[row];
+        q0 = g.pptr[row] + 4 * lane;
         q1 = g.pptr[row + 1];
     }
-    uint2 u0 = make_uint2(0, 0);
-    if (q0 < q1) u0 = *reinterpret_cast<const uint2 *>(g.pos + q0);
+    constexpr int PB = kDynPosBatch;
+    uint2 u[PB];
+    // groups q, q + 4 LR, ... of this lane, clamped to the row's last
+    auto positions = [&](uint32_t q) {
+#pragma unroll
+        for (int i = 0; i < PB; ++i)
+            u[i] = *reinterpret_cast<const uint2 *>(g.pos + min(q + (4 * i << lg), q1 - 4));
+    };
+    if (q0 < q1) positions(q0);
     const auto pre = epi.load(row);
     // phase 1: the next segment's record, slots and residual are requested
-    // while the current one is walked
+    // while the current one is walked; an entry past the segment's slots
+    // (there is none) or of no length would go to slot ne + 1
     struct Cur {
         DynSeg sr;
         int e0, e1;
@@ -750,11 +771,11 @@ __global__ __launch_bounds__(NT) void k_dyn_tile_T(DynView g, const T *__restric
             Cur nxt = cur;
             if (j + NT < ns) nxt = fetch(j + NT);
             int e = cur.e0;
-            const int e1 = cur.e1;
+            const int e1 = cur.e1, dump = P.ne + 1;
             const T xv = cur.xv;
-            dyn_seg_walk(cur.sr, P, [&](int, float w) {
-                if (e < e1) pe[e] = (T)w * xv;
-                ++e;
+            dyn_seg_walk(cur.sr, P, [&](int, float w, bool on) {
+                pe[e < e1 ? e : dump] = (T)w * xv;
+                e += on ? 1 : 0;           // else the next entry overwrites it
             });
             cur = nxt;
         }
@@ -763,13 +784,19 @@ __global__ __launch_bounds__(NT) void k_dyn_tile_T(DynView g, const T *__restric
     __syncthreads();
     if (has_row) {
         T acc = 0;
-        if (q0 < q1)
-            acc += (pe[u0.x & 0xffffu] + pe[u0.x >> 16]) + (pe[u0.y & 0xffffu] + pe[u0.y >> 16]);
-        for (uint32_t q = q0 + 4; q < q1; q += 4) {
-            const uint2 u = *reinterpret_cast<const uint2 *>(g.pos + q);
-            acc += (pe[u.x & 0xffffu] + pe[u.x >> 16]) + (pe[u.y & 0xffffu] + pe[u.y >> 16]);
+        for (uint32_t q = q0; q < q1;) {
+            T v[PB];
+#pragma unroll
+            for (int i = 0; i < PB; ++i)
+                v[i] = (pe[u[i].x & 0xffffu] + pe[u[i].x >> 16]) +
+                       (pe[u[i].y & 0xffffu] + pe[u[i].y >> 16]);
+#pragma unroll
+            for (int i = 0; i < PB; ++i) acc += q + (4 * i << lg) < q1 ? v[i] : (T)0;
+            q += 4 * PB << lg;
+            if (q < q1) positions(q);
         }
-        epi.row(row, acc, true, pre);
+        acc = lane_sum(acc, LR);
+        epi.row(row, acc, lane == 0, pre);
     }
     epi.finish();
 }
@@ -784,18 +811,9 @@ void launch_dyn_N(const DynTiles &D, const T *x, T *part, const int32_t *active,
 template <typename T, typename Epi>
 void launch_dyn_T(const DynTiles &D, const T *x, const Epi &epi, hipStream_t s) {
     if (D.bwd.npan == 0) return;
-    const size_t lds = sizeof(T) * (size_t)(D.emax_cap + 1);
-    switch (D.threads_T) {
-    case 512:
-        hipLaunchKernelGGL((k_dyn_tile_T<T, 512, Epi>), dim3((unsigned)D.bwd.npan), dim3(512), lds,
-                           s, dyn_view(D, D.bwd), x, epi);
-        break;
-    case 1024:
-        hipLaunchKernelGGL((k_dyn_tile_T<T, 1024, Epi>), dim3((unsigned)D.bwd.npan), dim3(1024),
-                           lds, s, dyn_view(D, D.bwd), x, epi);
-        break;
-    default: throw tv3_error(TV3_E_ARG, "the A^T tile product runs 512 or 1024 threads");
-    }
+    const size_t lds = sizeof(T) * (size_t)(D.emax_cap + 2);
+    hipLaunchKernelGGL((k_dyn_tile_T<T, kDynThreadsT, Epi>), dim3((unsigned)D.bwd.npan),
+                       dim3(kDynThreadsT), lds, s, dyn_view(D, D.bwd), x, epi);
 }
 
 #ifndef TV3_SEGSUM_NLB

@@ -307,7 +307,6 @@ struct DynBoxes {
 struct DynTiles {
     int64_t nnz = 0;
     int32_t emax_cap = 0;                 // A^T box limit: entries in LDS
-    int32_t threads_T = 512;              // workgroup of the A^T product
     float org[3] = {0, 0, 0}, h[3] = {1, 1, 1};
     int32_t N[3] = {0, 0, 0};        // voxels along x, y, z
     int32_t tile_dx = 0, tile_dz = 0;  // internal offset of the next 8^3 tile along x, z
