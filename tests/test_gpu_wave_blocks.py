@@ -79,3 +79,24 @@ def test_default_blocks_columns_equal_matvec(ctx, name, nrhs):
         Y = op.mat_mat_mul(X, trans=trans)
         for j in range(nrhs):
             assert torch.equal(Y[:, j], op.mat_vec_mul(X[:, j].contiguous(), trans=trans)), (trans, j)
+
+
+@pytest.mark.parametrize("n", [1 << 20, (1 << 20) + 1, 3_000_000])
+def test_block_order_exact(ctx, n):
+    # more columns than an L2 slice holds: blocks run in another order than the
+    # rows'; empty rows, and columns at both ends
+    import torch
+    rng = np.random.default_rng(n)
+    lens = np.concatenate([[0, 300, 1, 0], rng.integers(0, 90, 900), [0, 257]])
+    m = len(lens)
+    rowptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    col = rng.integers(0, n, rowptr[-1]).astype(np.int32)
+    col[[0, -1]] = n - 1, 0
+    val = rng.integers(-3, 4, len(col)).astype(np.float32)
+    op = api.SparseOperator(ctx, m, n, rowptr, col, val, dtype="f16")
+    x = rng.integers(-4, 5, (2, n)).astype(np.float32)
+    rows = np.repeat(np.arange(m), lens)
+    want = np.stack([np.bincount(rows, val * v[col], minlength=m) for v in x])
+    xd = torch.from_numpy(x).cuda()
+    assert (op.mat_vec_mul(xd[0]).cpu().numpy() == want[0]).all()
+    assert (op.mat_mat_mul(xd.t()).cpu().numpy() == want.T).all()

@@ -700,7 +700,7 @@ void dynamic_materialize(tv3_op *op, tv3_dtype vt, SparseRows &A) {
     TV3_HIP(hipGetLastError());
     TV3_HIP(hipStreamSynchronize(s));
     A.lanes = default_lanes(A.rows, A.nnz);
-    build_default_blocks(ctx, A);
+    build_default_blocks(ctx, A, true);
 }
 
 }  // namespace tv3

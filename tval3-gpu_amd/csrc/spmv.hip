@@ -136,7 +136,8 @@ static bool wave_blocks(const SparseRows &S) { return S.blk_nnz == kWaveBlk; }
 // and, where x outgrows an L2 slice, by its misses.  us, against 2048-entry
 // blocks of a 256-thread workgroup: 64^3 voxels x 65,536 rays FP32 weights
 // A^T 27.0 -> 18.0, A 17.2 -> 17.0; 128^3 x 262,144 FP16 A^T 130 -> 107,
-// A 149 -> 148, FP64 A^T 298 -> 186, A 300 -> 260 (k_csr_f64).
+// A 149 -> 148, FP64 A^T 298 -> 186, A 300 -> 260 (k_csr_f64); A in natural
+// block order (order_blocks).
 //
 // Acc = double also serves FP32 vectors whose row sums are rounded once.
 template <typename V, typename X, typename Acc>
@@ -223,8 +224,9 @@ static std::vector<int32_t> row_pointers(tv3_ctx *ctx, const SparseRows &S) {
     return ptr;
 }
 
-static void row_blocks(tv3_ctx *ctx, SparseRows &S, int blk_nnz, const std::vector<int32_t> &ptr,
-                       const std::vector<int64_t> *starts) {
+static std::vector<BlkDesc> row_blocks(tv3_ctx *ctx, SparseRows &S, int blk_nnz,
+                                       const std::vector<int32_t> &ptr,
+                                       const std::vector<int64_t> *starts) {
     const int threads = blk_nnz == kWaveBlk ? kWave : 256;
     std::vector<int32_t> blk;
     blk.reserve(S.nnz / (blk_nnz / 2) + S.rows / threads + 2);
@@ -243,12 +245,13 @@ static void row_blocks(tv3_ctx *ctx, SparseRows &S, int blk_nnz, const std::vect
     }
     blk.push_back((int32_t)S.rows);
     S.nblk = (int64_t)blk.size() - 1;
-    const std::vector<BlkDesc> d = make_blk_desc(blk, ptr.data(), nullptr, threads);
+    std::vector<BlkDesc> d = make_blk_desc(blk, ptr.data(), nullptr, threads);
     S.desc.alloc(d.size());
     TV3_HIP(hipMemcpyAsync(S.desc.p, d.data(), sizeof(BlkDesc) * d.size(), hipMemcpyHostToDevice,
                            ctx->stream));
     TV3_HIP(hipStreamSynchronize(ctx->stream));
     S.blk_nnz = blk_nnz;
+    return d;
 }
 
 void build_row_blocks(tv3_ctx *ctx, SparseRows &S, int blk_nnz,
@@ -256,16 +259,73 @@ void build_row_blocks(tv3_ctx *ctx, SparseRows &S, int blk_nnz,
     row_blocks(ctx, S, blk_nnz, row_pointers(ctx, S), starts);
 }
 
+// Where a block's first row runs: the sixteenths of the columns that its ends
+// lie in, and its middle entry's 4096th (20 bits).
+constexpr int kKeyBits = 20;
+__global__ __launch_bounds__(256) void k_block_keys(int64_t nblk, int64_t cols,
+                                                    const BlkDesc *__restrict__ desc,
+                                                    const int32_t *__restrict__ ptr,
+                                                    const int32_t *__restrict__ ind,
+                                                    uint32_t *__restrict__ key) {
+    const int64_t b = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (b >= nblk) return;
+    const int r = desc[b].r0, p0 = ptr[r], p1 = ptr[r + 1];
+    uint32_t v = 0;
+    if (p0 < p1) {
+        const int64_t i = ind[p0], j = ind[p1 - 1], k = ind[p0 + (p1 - p0) / 2];
+        const uint32_t lo = (uint32_t)(16 * min(i, j) / cols), hi = (uint32_t)(16 * max(i, j) / cols);
+        v = lo << 16 | hi << 12 | (uint32_t)(4096 * k / cols);
+    }
+    key[b] = v;
+}
+
+// Blocks in the order of their keys (stable): the blocks that an XCD runs one
+// after the other then gather from the same parts of x, whatever order the
+// rays come in; the matrix and y stay as they are.  Worth it where x (FP32) is
+// larger than an XCD's L2: A x, us, natural order -> this, 128^3 voxels x
+// 262,144 rays FP16 148 -> 135, FP64 260 -> 220, 112^3 x 262,144 FP16 118 ->
+// 112, 128^3 x 65,536 FP16 40.5 -> 38; below it the scattered streams cost
+// more than the gathers gain (96^3 x 147,456 FP32 54 -> 56).
+constexpr int64_t kOrderedCols = (int64_t(4) << 20) / sizeof(float);
+static void order_blocks(tv3_ctx *ctx, SparseRows &S, const std::vector<BlkDesc> &d) {
+    const int64_t nb = S.nblk;
+    if (nb < 2) return;
+    hipStream_t s = ctx->stream;
+    DevBuf<uint32_t> key(nb);
+    hipLaunchKernelGGL(k_block_keys, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, s, nb, S.cols,
+                       S.desc.p, S.ptr.p, S.ind.p, key.p);
+    TV3_HIP(hipGetLastError());
+    std::vector<uint32_t> k(nb);
+    TV3_HIP(hipMemcpyAsync(k.data(), key.p, sizeof(uint32_t) * nb, hipMemcpyDeviceToHost, s));
+    TV3_HIP(hipStreamSynchronize(s));
+    std::vector<int32_t> from(nb), to(nb);
+    for (int64_t b = 0; b < nb; ++b) from[b] = (int32_t)b;
+    constexpr int kDigit = kKeyBits / 2, kBins = 1 << kDigit;
+    for (int shift = 0; shift < kKeyBits; shift += kDigit) {
+        std::vector<int32_t> at(kBins + 1, 0);
+        for (int64_t b = 0; b < nb; ++b) ++at[(k[b] >> shift & (kBins - 1)) + 1];
+        for (int i = 0; i < kBins; ++i) at[i + 1] += at[i];
+        for (int64_t b = 0; b < nb; ++b) to[at[k[from[b]] >> shift & (kBins - 1)]++] = from[b];
+        from.swap(to);
+    }
+    std::vector<BlkDesc> o(d);
+    for (int64_t b = 0; b < nb; ++b) o[b] = d[from[b]];
+    TV3_HIP(hipMemcpyAsync(S.desc.p, o.data(), sizeof(BlkDesc) * o.size(), hipMemcpyHostToDevice, s));
+    TV3_HIP(hipStreamSynchronize(s));
+}
+
 // Wavefront blocks, unless a row is so long that one wavefront would still
 // sum it when the others are done (16 rounds of gathers): then 2048-entry
 // workgroup blocks.  Voxels next to a transducer are crossed by about 1,000
 // rays of 262,144.  A^T, us, 256 / 512 entries a wavefront: 64^3 voxels
 // 18.0 / 20.7, 96^3 49 / 49, 128^3 107 / 112.
-void build_default_blocks(tv3_ctx *ctx, SparseRows &S) {
+void build_default_blocks(tv3_ctx *ctx, SparseRows &S, bool measurements) {
     const std::vector<int32_t> ptr = row_pointers(ctx, S);
     int32_t longest = 0;
     for (int64_t r = 0; r < S.rows; ++r) longest = std::max(longest, ptr[r + 1] - ptr[r]);
-    row_blocks(ctx, S, longest <= 16 * kWaveBlk ? kWaveBlk : 2048, ptr, nullptr);
+    const std::vector<BlkDesc> d =
+        row_blocks(ctx, S, longest <= 16 * kWaveBlk ? kWaveBlk : 2048, ptr, nullptr);
+    if (measurements && wave_blocks(S) && S.cols > kOrderedCols) order_blocks(ctx, S, d);
 }
 
 std::vector<BlkDesc> make_blk_desc(const std::vector<int32_t> &blk, const int32_t *ptr,
@@ -787,7 +847,7 @@ void build_transpose(tv3_ctx *ctx, const SparseRows &A, SparseRows &AT) {
     TV3_HIP(hipGetLastError());
     TV3_HIP(hipStreamSynchronize(s));
     AT.lanes = default_lanes(AT.rows, AT.nnz);
-    build_default_blocks(ctx, AT);
+    build_default_blocks(ctx, AT, false);
 }
 
 }  // namespace tv3

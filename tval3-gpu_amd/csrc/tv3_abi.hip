@@ -256,14 +256,15 @@ void *tv3_ctx_stream(tv3_ctx *ctx) { return ctx ? (void *)ctx->stream : nullptr;
 // host rows (CSR of A, or its CSC as the CSR of A^T) to the device, with the
 // default launch shape and row blocks
 static void upload_rows(tv3_ctx *ctx, SparseRows &R, int64_t rows, int64_t cols, int64_t nnz,
-                        const int32_t *ptr, const int32_t *ind, const void *val, tv3_dtype vt) {
+                        const int32_t *ptr, const int32_t *ind, const void *val, tv3_dtype vt,
+                        bool measurements) {
     hipStream_t s = ctx->stream;
     R.rows = rows; R.cols = cols; R.nnz = nnz; R.vtype = vt;
     upload(R.ptr, ptr, rows + 1, s);
     upload(R.ind, ind, nnz, s);
     upload_bytes(R.val, val, nnz * dtype_size(vt), s);
     R.lanes = default_lanes(rows, nnz);
-    build_default_blocks(ctx, R);
+    build_default_blocks(ctx, R, measurements);
 }
 
 tv3_status tv3_op_csr_create(tv3_ctx *ctx, int64_t m, int64_t n, int64_t nnz,
@@ -291,8 +292,8 @@ tv3_status tv3_op_csr_create(tv3_ctx *ctx, int64_t m, int64_t n, int64_t nnz,
         op->device = ctx->device;
         op->kind = OpKind::CSR;
         op->m = m; op->n = n;
-        upload_rows(ctx, op->A, m, n, nnz, rowptr, col, val, vt);
-        if (has_csc) upload_rows(ctx, op->AT, n, m, nnz, cptr, crow, cval, vt);
+        upload_rows(ctx, op->A, m, n, nnz, rowptr, col, val, vt, true);
+        if (has_csc) upload_rows(ctx, op->AT, n, m, nnz, cptr, crow, cval, vt, false);
         else build_transpose(ctx, op->A, op->AT);
         TV3_HIP(hipStreamSynchronize(ctx->stream));
         *out = op.release();
@@ -441,13 +442,13 @@ tv3_status tv3_op_hybrid_create(tv3_ctx *ctx, const tv3_geometry *geom, tv3_weig
             TV3_REQUIRE(nnz == 0 || (crow && cval), TV3_E_ARG, "partial CSC arrays");
             check_csr_host(n, m, nnz, cptr, crow, "CSC");
             TV3_REQUIRE(finite_host(cval, vt, nnz), TV3_E_NONFINITE, "A holds NaN or Inf");
-            upload_rows(ctx, op->AT, n, m, nnz, cptr, crow, cval, vt);
+            upload_rows(ctx, op->AT, n, m, nnz, cptr, crow, cval, vt, false);
         } else if (rowptr) {                 // the caller's CSR, transposed on the device
             TV3_REQUIRE(nnz >= 0 && nnz <= INT32_MAX, TV3_E_SHAPE, "bad sparse sizes");
             TV3_REQUIRE(nnz == 0 || (col && val), TV3_E_ARG, "partial CSR arrays");
             check_csr_host(m, n, nnz, rowptr, col, "CSR");
             TV3_REQUIRE(finite_host(val, vt, nnz), TV3_E_NONFINITE, "A holds NaN or Inf");
-            upload_rows(ctx, A, m, n, nnz, rowptr, col, val, vt);
+            upload_rows(ctx, A, m, n, nnz, rowptr, col, val, vt, false);
             build_transpose(ctx, A, op->AT);
         } else {                             // no matrix given: the geometry's own
             dynamic_materialize(op.get(), vt, A);
@@ -823,7 +824,7 @@ tv3_status tv3_op_autotune(tv3_op *op, int32_t *lanes_N, int32_t *lanes_T) {
         // (reported as -NB) and the row-group kernel with L lanes
         auto best = [&](SparseRows &S, const float *xx) {
             int choice = 0;
-            build_default_blocks(op->ctx, S);
+            build_default_blocks(op->ctx, S, &S == &op->A);
             float bt = time_spmv(op->ctx, S, 0, xx, y.p);
             for (int nb : {1024, 2048, 4096}) {
                 build_row_blocks(op->ctx, S, nb);
@@ -835,7 +836,7 @@ tv3_status tv3_op_autotune(tv3_op *op, int32_t *lanes_N, int32_t *lanes_T) {
                 if (t < bt) { bt = t; choice = L; }
             }
             if (choice == 0) {
-                build_default_blocks(op->ctx, S);
+                build_default_blocks(op->ctx, S, &S == &op->A);
             } else if (choice < 0) {
                 build_row_blocks(op->ctx, S, -choice);
             } else {

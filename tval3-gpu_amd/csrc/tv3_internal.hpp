@@ -170,8 +170,9 @@ struct SparseRows {
 // starts (sorted, optional): rows where a block must begin.
 void build_row_blocks(tv3_ctx *ctx, SparseRows &S, int blk_nnz,
                       const std::vector<int64_t> *starts = nullptr);
-// The blocks a new operator's products run with.
-void build_default_blocks(tv3_ctx *ctx, SparseRows &S);
+// The blocks a new operator's products run with; measurements: S's rows are
+// A's, else they are A^T's (voxels, whose neighbours share rays).
+void build_default_blocks(tv3_ctx *ctx, SparseRows &S, bool measurements);
 
 // The parts of a geometry's rays inside boxes of kRayBox{Y,X,Z} voxels, for
 // the A^T products of dynamic.hip: built on the device when a matrix-free
