@@ -72,3 +72,22 @@ def test_products_equal_materialized_matrix(ctx, name, mode, dt):
         k = np.bincount(out, minlength=size).max() + 2
         err = np.abs(y - want)
         assert (err <= k * u * bound).all(), (trans, err.max())
+
+
+@pytest.mark.parametrize("mode", ["bresenham", "siddon"])
+@pytest.mark.parametrize("E,R", [(1, 1), (256, 255), (256, 256), (512, 257), (512, 512)])
+def test_lanes_sharing_a_ray(ctx, E, R, mode):
+    # A x with 8, 4, 2 and 1 lanes a ray (by the number of rays), walks shorter
+    # than the lanes are many
+    import torch
+    op = api.DynamicOperator(ctx, wl.transducer_geometry(E, R, dims=(13, 6, 9), seed=11), mode)
+    rp, col, val = op.materialize("f32").download_csr()
+    rng = np.random.default_rng(E + R)
+    x = rng.normal(size=op.n).astype(np.float32)
+    rows = np.repeat(np.arange(op.m), np.diff(rp))
+    t = val.astype(np.float64) * x[col]
+    want = np.bincount(rows, t, minlength=op.m)
+    mass = np.bincount(rows, np.abs(t), minlength=op.m)
+    k = np.diff(rp) + 2
+    y = op.mat_vec_mul(torch.from_numpy(x).cuda()).cpu().numpy()
+    assert (np.abs(y - want) <= k * 2.0 ** -24 * mass).all()

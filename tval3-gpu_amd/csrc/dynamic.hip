@@ -163,46 +163,55 @@ __device__ __forceinline__ void ray_ends(const GeoView &g, int64_t k, R p0[3], R
     for (int a = 0; a < 3; ++a) { p0[a] = (R)g.ep[3 * e + a]; p1[a] = (R)g.rp[3 * r + a]; }
 }
 
-// N of a Bresenham operator with every transducer in the grid: a thread owns
-// a ray (in bundles of neighbours, so the lanes of a wavefront gather near
-// each other) and gathers eight voxels at a time; one at a time, each step
-// waited for its gather.  At 128^3 with 262,144 rays 206 -> 77 us, now bound
-// by the gathers' cache lines (4 to 32 at a time, bundles of 4^2 to 32^2 rays
-// and workgroups of 64 to 1024 threads all take 77-79 us).
+// N of a Bresenham operator with every transducer in the grid: 1 << lg lanes
+// share a ray's steps, one behind the other (rays in bundles of neighbours, so
+// the lanes of a wavefront gather near each other), and gather eight voxels at
+// a time; one at a time, each step waited for its gather.  At 128^3 with
+// 262,144 rays 206 -> 77 us, now bound by the gathers' line look-ups (4 to 32
+// at a time, bundles of 4^2 to 32^2 rays and workgroups of 64 to 1024 threads
+// all take 77-79 us; x in bricks of 4 x 4 x 2 voxels 70, and 6 for the copy).
 template <typename T, typename AccT>
 __global__ __launch_bounds__(64) void k_bres_N(GeoView g, const int32_t *__restrict__ bundle,
                                                const int4 *__restrict__ walk,
-                                               const T *__restrict__ x, T *__restrict__ y) {
-    const int64_t i = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * 64 + threadIdx.x;
-    if (i >= g.P) return;
+                                               const T *__restrict__ x, T *__restrict__ y, int lg) {
+    const int64_t t = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * 64 + threadIdx.x, i = t >> lg;
+    if (i >= g.P) return;             // whole groups of lanes leave together
     const int64_t k = bundle ? bundle[i] : i;
-    BresWalk w(walk[k], 0, g.rvy, 1, g.rvx * g.rvy);
+    const int4 rec = walk[k];
+    // this lane's steps of the walk: from j0, n of them
+    const int part = (int)t & ((1 << lg) - 1);
+    const int steps = max(max(abs(rec.y >> 16), abs((int)(int16_t)rec.z)), abs(rec.z >> 16)) + 1;
+    const int j0 = steps * part >> lg, n = (steps * (part + 1) >> lg) - j0;
+    BresWalk w(rec, j0, g.rvy, 1, g.rvx * g.rvy);
     w.off = (w.z * g.rvx + w.x) * g.rvy + w.y;
     const AccT wt = (AccT)(T)g.scale;
     AccT acc = 0;
-    for (int j = 0; j < w.steps; j += 8) {
+    for (int j = 0; j < n; j += 8) {
         T v[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
             v[u] = x[w.off];
-            if (j + u + 1 < w.steps) w.next();   // stays at the receiver's voxel
+            if (j + u + 1 < n) w.next();   // stays at the last voxel
         }
 #pragma unroll
         for (int u = 0; u < 8; ++u)
-            if (j + u < w.steps) acc += (AccT)v[u] * wt;
+            if (j + u < n) acc += (AccT)v[u] * wt;
     }
-    y[k] = (T)acc;
+    acc = lane_sum(acc, 1 << lg);
+    if (part == 0) y[k] = (T)acc;
 }
 
 // N of a Siddon operator likewise: sid_walk's steps with eight gathers at a
-// time (77 x 101 x 90 voxels, 90,150 rays: 73 -> 32 us).  The Siddon operator is the FP32 traversal: FP64 products accumulate
-// its weights in FP64 (the same matrix in both precisions).
+// time (77 x 101 x 90 voxels, 90,150 rays: 73 -> 32 us).  The Siddon operator
+// is the FP32 traversal: FP64 products accumulate its weights in FP64 (the
+// same matrix in both precisions).
 template <typename T, typename AccT>
 __global__ __launch_bounds__(64) void k_sid_N(GeoView g, const int32_t *__restrict__ bundle,
-                                              const T *__restrict__ x, T *__restrict__ y) {
+                                              const T *__restrict__ x, T *__restrict__ y, int lg) {
 #pragma clang fp contract(off)
-    const int64_t i = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * 64 + threadIdx.x;
-    if (i >= g.P) return;
+    const int64_t t = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * 64 + threadIdx.x, i = t >> lg;
+    if (i >= g.P) return;             // whole groups of lanes leave together
+    const int part = (int)t & ((1 << lg) - 1);
     const int64_t k = bundle ? bundle[i] : i;
     float p0[3], p1[3];
     const int N[3] = {g.rvx, g.rvy, g.rvz};
@@ -212,14 +221,34 @@ __global__ __launch_bounds__(64) void k_sid_N(GeoView g, const int32_t *__restri
     sid_setup(s, p0, p1, g.org, g.h, N);
     AccT acc = 0;
     if (s.hit) {
+        // This lane's part of the traversal, event to event: bound j of
+        // 1 << lg is the last plane crossing at or before j equal shares.  The
+        // entries of the parts are the whole walk's (its state after an event
+        // depends on the event's parameter alone).
+        auto share = [&](int j) {
+            const float p = s.amin + (s.amax - s.amin) * ((float)j / (float)(1 << lg));
+            return j == 0 || !(p > s.amin) ? s.amin : (j == 1 << lg || !(p < s.amax) ? s.amax : p);
+        };
+        auto event = [&](float p) {
+            if (!(p > s.amin) || !(p < s.amax)) return p;
+            float e = s.amin;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                if (s.st[a] == 0) continue;
+                const float before = sid_plane(s, a, sid_next_plane(s, a, p) - s.st[a]);
+                e = before > e && before <= p ? before : e;
+            }
+            return e;
+        };
+        const float ts = event(share(part)), te = event(share(part + 1));
         // next plane (as a float) and its parameter per axis; a plane beyond
         // the grid lies at or beyond amax, so it is never taken
-        float kf[3], tk[3], st[3], tcur = s.amin;
+        float kf[3], tk[3], st[3], tcur = ts;
         int64_t step[3], off = 0;
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
             const bool par = s.st[a] == 0;
-            const int kn = par ? 0 : sid_next_plane(s, a, s.amin);
+            const int kn = par ? 0 : sid_next_plane(s, a, ts);
             const int c = par ? s.cfix[a] : (s.st[a] > 0 ? kn - 1 : kn);
             kf[a] = (float)kn;
             st[a] = (float)s.st[a];
@@ -227,18 +256,18 @@ __global__ __launch_bounds__(64) void k_sid_N(GeoView g, const int32_t *__restri
             step[a] = s.st[a] * stride[a];
             off += c * stride[a];
         }
-        bool on = true;
+        bool on = ts < te;
         for (int left = N[0] + N[1] + N[2] + 4; on && left > 0; left -= 8) {
             float w[8];
             T v[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                float tnext = s.amax;
+                float tnext = te;
 #pragma unroll
                 for (int a = 0; a < 3; ++a) tnext = tk[a] < tnext ? tk[a] : tnext;
                 w[u] = on ? (tnext - tcur) * s.L : 0.f;
                 v[u] = x[off];
-                on = on && tnext < s.amax;
+                on = on && tnext < te;
 #pragma unroll
                 for (int a = 0; a < 3; ++a) {
                     const bool m = on && tk[a] == tnext;
@@ -253,7 +282,8 @@ __global__ __launch_bounds__(64) void k_sid_N(GeoView g, const int32_t *__restri
                 if (w[u] > 0) acc = fma((AccT)w[u], (AccT)v[u], acc);
         }
     }
-    y[k] = (T)acc;
+    acc = lane_sum(acc, 1 << lg);
+    if (part == 0) y[k] = (T)acc;
 }
 
 // T from the rays' parts inside boxes: a workgroup adds the parts of one work
@@ -396,14 +426,22 @@ static void dyn_apply(tv3_op *op, bool trans, const T *x, T *y, hipStream_t s) {
     const DynGeom &G = op->geo;
     const GeoView g = view(G);
     const int sid = G.mode == TV3_WEIGHT_SIDDON;
-    const unsigned rays64 = (unsigned)((g.P + 63) / 64), rays256 = (unsigned)((g.P + 255) / 256);
+    const unsigned rays256 = (unsigned)((g.P + 255) / 256);
     if (!trans) {
+        // up to eight lanes share a ray, until the chip has 16 wavefronts a CU
+        // (4,096 at 256 CUs).  us, one lane a ray -> this: Siddon 57 x 71 x 50,
+        // 9,408 rays 18.6 -> 13.2; 77 x 101 x 90, 90,150 33.6 -> 31.9; 121 x 101
+        // x 97, 147,456 55 -> 50; Bresenham 50^3, 9,408 8.7 -> 6.2; 64^3, 65,536
+        // 11.1 -> 10.2; twice as many lanes 36 and 53, 128^3 76 -> 83
+        int lg = 0;
+        while (lg < 3 && (g.P << lg) < (int64_t)op->ctx->num_cus * 16 * 64) ++lg;
+        const unsigned waves = (unsigned)(((g.P << lg) + 63) / 64);
         if (sid)
-            hipLaunchKernelGGL((k_sid_N<T, AccT>), dim3(rays64), dim3(64), 0, s, g, G.bundle.p, x,
-                               y);
+            hipLaunchKernelGGL((k_sid_N<T, AccT>), dim3(waves), dim3(64), 0, s, g, G.bundle.p, x, y,
+                               lg);
         else if (G.inside)
-            hipLaunchKernelGGL((k_bres_N<T, AccT>), dim3(rays64), dim3(64), 0, s, g, G.bundle.p,
-                               G.walk.p, x, y);
+            hipLaunchKernelGGL((k_bres_N<T, AccT>), dim3(waves), dim3(64), 0, s, g, G.bundle.p,
+                               G.walk.p, x, y, lg);
         else
             hipLaunchKernelGGL((k_clamped_N<T, AccT>), dim3(rays256), dim3(256), 0, s, g, x, y);
     } else {
