@@ -63,7 +63,7 @@ __device__ __forceinline__ uint16_t bf16_rne(float x) {
 }
 
 __global__ __launch_bounds__(512, 4) void k_gemm_rhs(const uint16_t *__restrict__ M,
-                                                  int64_t R, int64_t K, int S,
+                                                  int64_t R, int64_t K, int each, int more,
                                                   const float *__restrict__ X, int64_t ldx,
                                                   int G, float *__restrict__ part,
                                                   const int32_t *gate) {
@@ -75,8 +75,9 @@ __global__ __launch_bounds__(512, 4) void k_gemm_rhs(const uint16_t *__restrict_
     const int64_t tiles = R / kRows;
     const int64_t tile = blockIdx.x % tiles;
     const int s = (int)(blockIdx.x / tiles);
-    const int64_t kper = K / S;
-    const int64_t k_beg = (int64_t)s * kper, k_end = k_beg + kper;
+    // slice s of K: `each` chunks, one more in the first `more` slices
+    const int64_t nchunk = each + (s < more ? 1 : 0);
+    const int64_t k_beg = ((int64_t)s * each + min(s, more)) * kChunk;
     // this wavefront's 32-row band of M in operand order, lane's 16 bytes
     const uint16_t *mrow = M + (tile * (kRows / 32) + wave) * (K / 16) * 512 + lane * 8;
     // X staging: thread t converts 8 values of column t / 8 (columns >= G
@@ -89,7 +90,6 @@ __global__ __launch_bounds__(512, 4) void k_gemm_rhs(const uint16_t *__restrict_
     // multiplied: X's before the products, an operand of M as soon as its last
     // product is issued (into the same registers: two sets, and the totals,
     // would leave one workgroup a CU).
-    const int64_t nchunk = (k_end - k_beg) / kChunk;
     auto load_a = [&](int64_t c, int st) {
         const int64_t kc = k_beg + min(c, nchunk - 1) * kChunk;   // clamped: in range
         return *reinterpret_cast<const bf16x8 *>(mrow + (kc / 16 + st) * 512);
@@ -260,14 +260,16 @@ void gemm_rhs(const uint16_t *M, int64_t R, int64_t K, const float *X, int64_t l
               float *Y, int64_t ldy, const float *sub, int splits, float *part, hipStream_t s,
               const int32_t *gate) {
     TV3_REQUIRE(G > 0 && G <= kCols, TV3_E_ARG, "1 to 64 right-hand sides per product");
-    TV3_REQUIRE(gemm_rhs_shape_ok(R, K, splits), TV3_E_SHAPE,
-                "dense multi-RHS products need rows a multiple of 256 and K a multiple of "
-                "64 x splits");
+    TV3_REQUIRE(R > 0 && R % kRows == 0 && K % kChunk == 0 && splits > 0 && splits <= K / kChunk,
+                TV3_E_SHAPE,
+                "dense multi-RHS products need rows a multiple of 256 and K a multiple of 64, "
+                "with at least 64 values for each split");
     TV3_REQUIRE(ldx % 4 == 0, TV3_E_SHAPE,
                 "dense multi-RHS products need 16-byte aligned right-hand sides");
     const unsigned grid = (unsigned)((R / kRows) * splits);
-    hipLaunchKernelGGL(k_gemm_rhs, dim3(grid), dim3(kThreads), 0, s, M, R, K, splits, X, ldx, G,
-                       part, gate);
+    const int64_t chunks = K / kChunk;
+    hipLaunchKernelGGL(k_gemm_rhs, dim3(grid), dim3(kThreads), 0, s, M, R, K, (int)(chunks / splits),
+                       (int)(chunks % splits), X, ldx, G, part, gate);
     hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)(R / 8)), dim3(256), 0, s, part, R, splits,
                        G, Y, ldy, sub, gate);
 }

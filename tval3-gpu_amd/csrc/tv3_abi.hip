@@ -587,16 +587,22 @@ tv3_status tv3_matvec_multi(tv3_op *op, tv3_trans trans, int32_t nrhs, const flo
             TV3_HIP(hipGetLastError());
             return;
         }
-        // K splits (K a multiple of 64 splits): a workgroup a CU, and a second
-        // one where 2,048 values of K are left to each: every split writes and
-        // reads back R x 64 partial sums.  64 columns, A X, us, with 256, 512,
-        // 1024 workgroups: 4096 x 16384 45, 44, 57; 8192 x 32768 155, 150, 160;
-        // 2048 x 8192 20, 23, 32
+        // K splits, of whole 64-value chunks but not of equal lengths: about a
+        // workgroup a CU, two chunks or more each, and a second one a CU where
+        // 2,048 values of K are left to each: every split writes and reads back
+        // R x 64 partial sums.  64 columns, A X, us: 4096 x 16384 with 256, 512,
+        // 1024 workgroups 37, 43, 50; 8192 x 32768 155, 150, 160; 768 x 15104 (3
+        // tiles, 236 chunks) with 12 (the largest power of two that divides K),
+        // 144, 192, 288 workgroups 75, 16, 16, 20; 2304 x 12032 with 36, 216, 288
+        // 63, 23, 28; 1280 x 5376 with 20, 160, 240 31, 14, 15
         const int64_t tiles = R / gemm_rhs_rows(), cus = op->ctx->num_cus;
+        auto fits = [&](int64_t S) {
+            return 2 * S <= K / 64 &&
+                   (tiles * S <= cus || (tiles * S <= 2 * cus && K / S >= 2048));
+        };
         int splits = 1;
-        while (gemm_rhs_shape_ok(R, K, splits * 2) &&
-               (tiles * splits < cus || (tiles * splits < 2 * cus && K / (2 * splits) >= 2048)))
-            splits *= 2;
+        for (int64_t S = 2; S <= K / 64; S += S & (S - 1) ? S / 3 : S / 2)   // 2, 3, 4, 6, 8, 12
+            if (fits(S)) splits = (int)S;
         const size_t need = gemm_rhs_scratch(R, splits) * sizeof(float);
         if (op->ctx->scratch.bytes() < need) op->ctx->scratch.alloc(need);
         float *part = reinterpret_cast<float *>(op->ctx->scratch.p);
