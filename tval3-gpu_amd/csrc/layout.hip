@@ -894,6 +894,8 @@ void renumber_rows(tv3_ctx *ctx, const SparseRows &A, const std::vector<int32_t>
         throw tv3_error(TV3_E_FORMAT, "the fused solver needs F32, F16 or BF16 weights");
     TV3_HIP(hipGetLastError());
     build_transpose(ctx, N, L->AT);
+    // what launch_stream runs until a tuned or forced shape replaces it
+    build_row_blocks(ctx, L->AT, 2048);
 }
 
 FusedLayout &fused_layout(tv3_op *op, const int32_t dims[3], bool tune) {

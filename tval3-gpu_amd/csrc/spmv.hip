@@ -847,7 +847,6 @@ void build_transpose(tv3_ctx *ctx, const SparseRows &A, SparseRows &AT) {
     TV3_HIP(hipGetLastError());
     TV3_HIP(hipStreamSynchronize(s));
     AT.lanes = default_lanes(AT.rows, AT.nnz);
-    build_default_blocks(ctx, AT, false);
 }
 
 }  // namespace tv3

@@ -267,6 +267,12 @@ static void upload_rows(tv3_ctx *ctx, SparseRows &R, int64_t rows, int64_t cols,
     build_default_blocks(ctx, R, measurements);
 }
 
+// A^T of an operator built on the device, with a new operator's row blocks
+static void transpose_rows(tv3_ctx *ctx, const SparseRows &A, SparseRows &AT) {
+    build_transpose(ctx, A, AT);
+    build_default_blocks(ctx, AT, false);
+}
+
 tv3_status tv3_op_csr_create(tv3_ctx *ctx, int64_t m, int64_t n, int64_t nnz,
                              const int32_t *rowptr, const int32_t *col, const void *val,
                              tv3_dtype vt, const int32_t *cptr, const int32_t *crow,
@@ -294,7 +300,7 @@ tv3_status tv3_op_csr_create(tv3_ctx *ctx, int64_t m, int64_t n, int64_t nnz,
         op->m = m; op->n = n;
         upload_rows(ctx, op->A, m, n, nnz, rowptr, col, val, vt, true);
         if (has_csc) upload_rows(ctx, op->AT, n, m, nnz, cptr, crow, cval, vt, false);
-        else build_transpose(ctx, op->A, op->AT);
+        else transpose_rows(ctx, op->A, op->AT);
         TV3_HIP(hipStreamSynchronize(ctx->stream));
         *out = op.release();
     });
@@ -449,10 +455,10 @@ tv3_status tv3_op_hybrid_create(tv3_ctx *ctx, const tv3_geometry *geom, tv3_weig
             check_csr_host(m, n, nnz, rowptr, col, "CSR");
             TV3_REQUIRE(finite_host(val, vt, nnz), TV3_E_NONFINITE, "A holds NaN or Inf");
             upload_rows(ctx, A, m, n, nnz, rowptr, col, val, vt, false);
-            build_transpose(ctx, A, op->AT);
+            transpose_rows(ctx, A, op->AT);
         } else {                             // no matrix given: the geometry's own
             dynamic_materialize(op.get(), vt, A);
-            build_transpose(ctx, A, op->AT);
+            transpose_rows(ctx, A, op->AT);
         }
         TV3_HIP(hipStreamSynchronize(ctx->stream));
         *out = op.release();
@@ -474,7 +480,7 @@ tv3_status tv3_op_materialize(tv3_op *dyn, tv3_dtype vt, tv3_op **out) {
         op->kind = OpKind::CSR;
         op->m = dyn->m; op->n = dyn->n;
         dynamic_materialize(dyn, vt, op->A);
-        build_transpose(ctx, op->A, op->AT);
+        transpose_rows(ctx, op->A, op->AT);
         op->ray_order = geometry_ray_order(dyn->geo);
         *out = op.release();
     });

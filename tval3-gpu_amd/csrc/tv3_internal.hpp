@@ -436,6 +436,8 @@ size_t spmv_multi_scratch(const SparseRows &S);
 void spmv_multi(const SparseRows &S, int nrhs, const float *X, int64_t ldx, float *Y, int64_t ldy,
                 float *xt, hipStream_t s);
 // Stable device transpose of a CSR (rows ordered ascending within each column).
+// Its row blocks are the caller's choice: an operator's products and the fused
+// layout's run different kernels.
 void build_transpose(tv3_ctx *ctx, const SparseRows &A, SparseRows &AT);
 // exclusive scan of cnt[0..n) into out[0..n] (out[n] = total); returns total
 int64_t exclusive_scan_i32(tv3_ctx *ctx, const int32_t *cnt, int32_t *out, int64_t n);
