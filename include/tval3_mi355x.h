@@ -223,8 +223,9 @@ tv3_status tv3_matvec_noalloc(tv3_op *op, tv3_trans trans, const float *x_dev, f
  * any other operator gives tv3_matvec's result per column, a dense one and a
  * sparse one in row blocks from one reading of the matrix for up to eight
  * columns (the sparse one with a workspace of eight vectors kept with the
- * operator; one column at a time under stream capture).  Asynchronous on
- * stream. */
+ * operator; under stream capture one column at a time for a sparse operator,
+ * and as many as the context's workspace holds for a dense one's A X).
+ * Asynchronous on stream. */
 tv3_status tv3_matvec_multi(tv3_op *op, tv3_trans trans, int32_t nrhs, const float *X_dev,
                             int64_t ldx, float *Y_dev, int64_t ldy, void *stream);
 

@@ -215,33 +215,53 @@ __global__ __launch_bounds__(256) void k_gemv_t(int64_t m, int64_t n, int64_t ld
 
 }  // namespace
 
+// Column slabs of A x: enough workgroups for four a CU, as far as the columns
+// go; never more than the min(128, ceil(n / 64)) that a workspace of the
+// caller's is checked for.
+static int64_t most_slabs(int64_t n) {
+    const int64_t slabs = std::min<int64_t>(128, (n + 63) / 64), per = (n + slabs - 1) / slabs;
+    return (n + per - 1) / per;
+}
+static int64_t slabs_of(const tv3_op *op, int W) {
+    const int64_t tiles = (op->m + 64 * W - 1) / (64 * W), n = op->n;
+    const int64_t ks = std::min(most_slabs(n),
+                                std::max<int64_t>(1, (4 * op->ctx->num_cus + tiles - 1) / tiles));
+    const int64_t per = (n + ks - 1) / ks;
+    return (n + per - 1) / per;
+}
+// rows a lane of A x loads at once
+template <typename V> static int run_n(int64_t m) { return m >= run_of<V>() ? run_of<V>() : 1; }
+
 // G vectors (1 <= G <= KT).  ws: the split-K partials of A x go to this
 // workspace of ws_bytes (the allocation-free path, one vector) instead of the
-// context's, which grows on demand.
+// context's, which grows on demand to what the launch uses.  Under stream
+// capture it cannot grow: then as many slabs as it holds, at least one, which
+// needs none.
 template <typename V, int W, int KT, typename T, typename AccT>
 static void gemv_n(tv3_op *op, int G, const T *x, int64_t ldx, T *y, int64_t ldy, hipStream_t s,
                    void *ws, size_t ws_bytes) {
     const V *A = reinterpret_cast<const V *>(op->dense.p);
     const int64_t m = op->m, n = op->n, lda = op->lda;
-    // the workspace a caller provides is checked for min(128, ceil(n / 64))
-    // slabs; the launch uses no more than those
-    int64_t slabs = std::min<int64_t>(128, (n + 63) / 64);
-    slabs = (n + (n + slabs - 1) / slabs - 1) / ((n + slabs - 1) / slabs);
-    const size_t need = sizeof(AccT) * (size_t)slabs * (size_t)m;
-    if (ws)
-        TV3_REQUIRE(need <= ws_bytes, TV3_E_UNSUPPORTED,
-                    "dense A x needs " + std::to_string(need) + " bytes of partial sums; the "
+    if (ws) {
+        const size_t most = sizeof(AccT) * (size_t)most_slabs(n) * (size_t)m;
+        TV3_REQUIRE(most <= ws_bytes, TV3_E_UNSUPPORTED,
+                    "dense A x needs " + std::to_string(most) + " bytes of partial sums; the "
                     "allocation-free path holds " + std::to_string(ws_bytes));
-    // enough workgroups for four a CU, as far as the columns go
+    }
     const int64_t tiles = (m + 64 * W - 1) / (64 * W);
-    int64_t ks = std::min(slabs, std::max<int64_t>(1, (4 * op->ctx->num_cus + tiles - 1) / tiles));
-    const int64_t cols_per = (n + ks - 1) / ks;
-    ks = (n + cols_per - 1) / cols_per;
+    int64_t ks = slabs_of(op, W);
     AccT *part = reinterpret_cast<AccT *>(ws);
     if (!ws && ks > 1) {
-        if (op->ctx->scratch.bytes() < KT * need) op->ctx->scratch.alloc(KT * need);
-        part = reinterpret_cast<AccT *>(op->ctx->scratch.p);
+        DevBuf<uint8_t> &held = op->ctx->scratch;
+        const size_t slab = sizeof(AccT) * (size_t)m * (size_t)G;
+        if (held.bytes() < slab * ks) {
+            if (capturing(s)) ks = std::max<int64_t>(1, held.bytes() / slab);
+            else held.alloc(slab * ks);
+        }
+        part = reinterpret_cast<AccT *>(held.p);
     }
+    const int64_t cols_per = (n + ks - 1) / ks;
+    ks = (n + cols_per - 1) / cols_per;
     hipLaunchKernelGGL((k_gemv_n_part<V, W, KT, T, AccT>), dim3((unsigned)tiles, (unsigned)ks),
                        dim3(256), 0, s, m, n, lda, A, x, ldx, G, part, y, ldy, cols_per);
     if (ks > 1)
@@ -262,7 +282,7 @@ static void gemv(tv3_op *op, bool trans, int G, const T *x, int64_t ldx, T *y, i
                  hipStream_t s, void *ws = nullptr, size_t ws_bytes = 0) {
     constexpr int W = run_of<V>();
     if (!trans) {
-        if (op->m >= W) gemv_n<V, W, KT, T, AccT>(op, G, x, ldx, y, ldy, s, ws, ws_bytes);
+        if (run_n<V>(op->m) == W) gemv_n<V, W, KT, T, AccT>(op, G, x, ldx, y, ldy, s, ws, ws_bytes);
         else gemv_n<V, 1, KT, T, AccT>(op, G, x, ldx, y, ldy, s, ws, ws_bytes);
     } else {
         // columns per wavefront: as many as leave eight wavefronts a CU
@@ -282,15 +302,21 @@ static void gemv(tv3_op *op, bool trans, const T *x, T *y, hipStream_t s, void *
 }
 
 // Several vectors, each with its single product's additions in the same
-// order (same bits): a reading of A serves up to eight.  2047 x 8190 FP32, 8
+// order (same bits): a reading of A serves up to eight, fewer where a capture
+// leaves too little workspace.  2047 x 8190 FP32, 8
 // vectors, A X 448 -> 20 us and A^T R 105 -> 18 us (26 four at a time); 64
 // vectors 3579 -> 155 and 831 -> 137 us; 4000 x 16001 BF16, 8 vectors, 571 ->
 // 34 and 342 -> 47 us (one at a time, before).
 template <typename V>
 static void gemv_multi(tv3_op *op, bool trans, int nrhs, const float *X, int64_t ldx, float *Y,
                        int64_t ldy, hipStream_t s) {
+    int most = 8;
+    if (!trans && capturing(s)) {   // as many as find room for all their slabs
+        const size_t one = sizeof(float) * (size_t)(slabs_of(op, run_n<V>(op->m)) * op->m);
+        most = (int)std::max<size_t>(1, std::min<size_t>(8, op->ctx->scratch.bytes() / one));
+    }
     for (int j = 0; j < nrhs;) {
-        const int left = nrhs - j;
+        const int left = std::min(nrhs - j, most);
         const float *x = X + j * ldx;
         float *y = Y + j * ldy;
         if (left == 1) {
@@ -300,9 +326,9 @@ static void gemv_multi(tv3_op *op, bool trans, int nrhs, const float *X, int64_t
         } else if (left <= 4) {
             gemv<V, 4, float, float>(op, trans, left, x, ldx, y, ldy, s);
         } else {
-            gemv<V, 8, float, float>(op, trans, std::min(left, 8), x, ldx, y, ldy, s);
+            gemv<V, 8, float, float>(op, trans, left, x, ldx, y, ldy, s);
         }
-        j += std::min(left, 8);
+        j += left;
     }
 }
 
