@@ -165,6 +165,12 @@ static tv3_status solve_host(tv3_ctx *ctx, tv3_op *op, const tv3_opts *opts,
         if (ctx->host_ws.bytes() < need) ctx->host_ws.alloc(need);
         T *bd = reinterpret_cast<T *>(ctx->host_ws.p), *Ud = bd + pad(op->m),
           *Utd = Ut ? Ud + pad(n) : nullptr;
+        // the caller may free b, U and U_true when this returns or throws (a
+        // NaN in b is found before anything waits): no copy is left queued
+        struct Drained {
+            hipStream_t s;
+            ~Drained() { (void)hipStreamSynchronize(s); }
+        } drained{s};
         TV3_HIP(hipMemcpyAsync(bd, b, sizeof(T) * op->m, hipMemcpyHostToDevice, s));
         if (opts->warm_start)
             TV3_HIP(hipMemcpyAsync(Ud, U, sizeof(T) * n, hipMemcpyHostToDevice, s));
@@ -180,7 +186,7 @@ static tv3_status solve_host(tv3_ctx *ctx, tv3_op *op, const tv3_opts *opts,
             solve_plain<double>(ctx, op, *opts, dims, bd, Ud, Utd, info, hist, b);
         }
         TV3_HIP(hipMemcpyAsync(U, Ud, sizeof(T) * n, hipMemcpyDeviceToHost, s));
-        TV3_HIP(hipStreamSynchronize(s));
+        TV3_HIP(hipStreamSynchronize(s));   // reports what went wrong
     });
     if (info) {
         info->outer_secs =
