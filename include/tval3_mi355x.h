@@ -195,6 +195,13 @@ tv3_status tv3_op_csr_download(tv3_op *op, int32_t *rowptr, int32_t *col, double
  * x, y device pointers; y is fully overwritten; asynchronous on stream
  * (a hipStream_t; NULL is the null stream, as for the reference's
  * stream = 0 default; pass tv3_ctx_stream(ctx) for the context stream).
+ * Products on several streams may be in flight at once: each of the first
+ * three streams of a workspace (a context's for dense products) has a buffer
+ * of its own, further ones wait for each other (finish a stream's products
+ * before destroying it).  Products recorded into graphs
+ * share one more buffer, so two graphs with dense products of one context must
+ * not be replayed at the same time; tv3_matvec allocates where a workspace has
+ * to grow, also under stream capture.
  * mulChain is a multi-GPU hint and has no counterpart here. */
 tv3_status tv3_matvec(tv3_op *op, tv3_trans trans, const float *x_dev, float *y_dev,
                       void *stream);
@@ -223,8 +230,7 @@ tv3_status tv3_matvec_noalloc(tv3_op *op, tv3_trans trans, const float *x_dev, f
  * any other operator gives tv3_matvec's result per column, a dense one and a
  * sparse one in row blocks from one reading of the matrix for up to eight
  * columns (the sparse one with a workspace of eight vectors kept with the
- * operator; under stream capture one column at a time for a sparse operator,
- * and as many as the context's workspace holds for a dense one's A X).
+ * operator; one column at a time for a sparse operator under stream capture).
  * Asynchronous on stream. */
 tv3_status tv3_matvec_multi(tv3_op *op, tv3_trans trans, int32_t nrhs, const float *X_dev,
                             int64_t ldx, float *Y_dev, int64_t ldy, void *stream);

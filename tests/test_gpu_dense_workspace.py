@@ -1,5 +1,5 @@
 """The workspace of dense products A X: what the launch's column slabs need,
-and products recorded into a graph, where it cannot grow.  A graph is replayed
+and products recorded into a graph, whatever ran before.  A graph is replayed
 several times with eager products between, every replay compared."""
 import numpy as np
 import pytest
@@ -68,3 +68,38 @@ def test_products_under_capture(m, n, dtype, first):
         torch.cuda.synchronize()
         assert torch.equal(Y.double(), (A @ X.double())) and torch.equal(y.double(), A @ x.double()), k
         torch.cuda.synchronize()
+
+
+def test_graph_keeps_its_workspace():
+    # eager products, larger ones too, on the replaying stream and on another
+    # while a graph's products are in flight; a second graph whose products
+    # need a larger workspace.  Random values: the eager product's bits.
+    import torch
+    assert torch.cuda.is_available()
+    ctx = api.Context(0)
+    rng = np.random.default_rng(5)
+    small, large = (api.DenseOperator(ctx, np.asfortranarray(
+        rng.normal(size=(m, n)).astype(np.float32)), "f32") for m, n in ((700, 3000), (1500, 9000)))
+    g = torch.Generator(device="cuda").manual_seed(1)
+    xs, xl = (torch.randn(8, n, device="cuda", generator=g).t() for n in (3000, 9000))
+    ys, yl = small.mat_mat_mul(xs), large.mat_mat_mul(xl)
+    outs, outl = torch.zeros_like(ys), torch.zeros_like(yl)
+    torch.cuda.synchronize()
+    graphs = []
+    for op, x, y in ((small, xs, outs), (large, xl, outl)):
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[-1]):
+            op.mat_mat_mul(x, y)
+    other = torch.cuda.Stream()
+    for k in range(4):
+        outs.zero_()
+        outl.zero_()
+        torch.cuda.synchronize()
+        graphs[0].replay()
+        graphs[1].replay()
+        with torch.cuda.stream(other):
+            a = large.mat_mat_mul(xl)
+        b = small.mat_mat_mul(xs)
+        torch.cuda.synchronize()
+        for got, want in ((outs, ys), (outl, yl), (a, yl), (b, ys)):
+            assert torch.equal(got, want), k

@@ -19,6 +19,7 @@
 // values of x in registers serve C loads of A (with one column, x is 2 bytes
 // of L1 traffic per byte of a BF16 matrix and set the pace).
 #include <algorithm>
+#include <optional>
 
 #include "lanes.hpp"
 #include "tv3_internal.hpp"
@@ -229,14 +230,10 @@ static int64_t slabs_of(const tv3_op *op, int W) {
     const int64_t per = (n + ks - 1) / ks;
     return (n + per - 1) / per;
 }
-// rows a lane of A x loads at once
-template <typename V> static int run_n(int64_t m) { return m >= run_of<V>() ? run_of<V>() : 1; }
 
 // G vectors (1 <= G <= KT).  ws: the split-K partials of A x go to this
 // workspace of ws_bytes (the allocation-free path, one vector) instead of the
-// context's, which grows on demand to what the launch uses.  Under stream
-// capture it cannot grow: then as many slabs as it holds, at least one, which
-// needs none.
+// context's, which grows on demand to what the launch uses.
 template <typename V, int W, int KT, typename T, typename AccT>
 static void gemv_n(tv3_op *op, int G, const T *x, int64_t ldx, T *y, int64_t ldy, hipStream_t s,
                    void *ws, size_t ws_bytes) {
@@ -249,19 +246,13 @@ static void gemv_n(tv3_op *op, int G, const T *x, int64_t ldx, T *y, int64_t ldy
                     "allocation-free path holds " + std::to_string(ws_bytes));
     }
     const int64_t tiles = (m + 64 * W - 1) / (64 * W);
-    int64_t ks = slabs_of(op, W);
+    const int64_t ks = slabs_of(op, W), cols_per = (n + ks - 1) / ks;
     AccT *part = reinterpret_cast<AccT *>(ws);
+    std::optional<StreamScratch::Lease> lease;
     if (!ws && ks > 1) {
-        DevBuf<uint8_t> &held = op->ctx->scratch;
-        const size_t slab = sizeof(AccT) * (size_t)m * (size_t)G;
-        if (held.bytes() < slab * ks) {
-            if (capturing(s)) ks = std::max<int64_t>(1, held.bytes() / slab);
-            else held.alloc(slab * ks);
-        }
-        part = reinterpret_cast<AccT *>(held.p);
+        lease.emplace(op->ctx->scratch.take(s, sizeof(AccT) * (size_t)(ks * m) * (size_t)G));
+        part = reinterpret_cast<AccT *>(lease->p);
     }
-    const int64_t cols_per = (n + ks - 1) / ks;
-    ks = (n + cols_per - 1) / cols_per;
     hipLaunchKernelGGL((k_gemv_n_part<V, W, KT, T, AccT>), dim3((unsigned)tiles, (unsigned)ks),
                        dim3(256), 0, s, m, n, lda, A, x, ldx, G, part, y, ldy, cols_per);
     if (ks > 1)
@@ -282,7 +273,7 @@ static void gemv(tv3_op *op, bool trans, int G, const T *x, int64_t ldx, T *y, i
                  hipStream_t s, void *ws = nullptr, size_t ws_bytes = 0) {
     constexpr int W = run_of<V>();
     if (!trans) {
-        if (run_n<V>(op->m) == W) gemv_n<V, W, KT, T, AccT>(op, G, x, ldx, y, ldy, s, ws, ws_bytes);
+        if (op->m >= W) gemv_n<V, W, KT, T, AccT>(op, G, x, ldx, y, ldy, s, ws, ws_bytes);
         else gemv_n<V, 1, KT, T, AccT>(op, G, x, ldx, y, ldy, s, ws, ws_bytes);
     } else {
         // columns per wavefront: as many as leave eight wavefronts a CU
@@ -302,21 +293,15 @@ static void gemv(tv3_op *op, bool trans, const T *x, T *y, hipStream_t s, void *
 }
 
 // Several vectors, each with its single product's additions in the same
-// order (same bits): a reading of A serves up to eight, fewer where a capture
-// leaves too little workspace.  2047 x 8190 FP32, 8
+// order (same bits): a reading of A serves up to eight.  2047 x 8190 FP32, 8
 // vectors, A X 448 -> 20 us and A^T R 105 -> 18 us (26 four at a time); 64
 // vectors 3579 -> 155 and 831 -> 137 us; 4000 x 16001 BF16, 8 vectors, 571 ->
 // 34 and 342 -> 47 us (one at a time, before).
 template <typename V>
 static void gemv_multi(tv3_op *op, bool trans, int nrhs, const float *X, int64_t ldx, float *Y,
                        int64_t ldy, hipStream_t s) {
-    int most = 8;
-    if (!trans && capturing(s)) {   // as many as find room for all their slabs
-        const size_t one = sizeof(float) * (size_t)(slabs_of(op, run_n<V>(op->m)) * op->m);
-        most = (int)std::max<size_t>(1, std::min<size_t>(8, op->ctx->scratch.bytes() / one));
-    }
     for (int j = 0; j < nrhs;) {
-        const int left = std::min(nrhs - j, most);
+        const int left = std::min(nrhs - j, 8);
         const float *x = X + j * ldx;
         float *y = Y + j * ldy;
         if (left == 1) {

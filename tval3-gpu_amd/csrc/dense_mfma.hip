@@ -293,6 +293,7 @@ void dense_operand_order(tv3_op *op, hipStream_t s) {
                        (const uint16_t *)op->dense.p, op->lda, 1, op->n, op->m,
                        (uint16_t *)oT.p);
     TV3_HIP(hipGetLastError());
+    TV3_HIP(hipStreamSynchronize(s));    // the next product may run on another stream
     op->dense_oN = std::move(oN);
     op->dense_oT = std::move(oT);
 }

@@ -248,7 +248,6 @@ void tv3_ctx_destroy(tv3_ctx *ctx) {
     ctx->batch_session.reset();
     ctx->plain_ws.release();
     ctx->host_ws.release();
-    ctx->scratch.release();
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -575,18 +574,19 @@ tv3_status tv3_matvec_multi(tv3_op *op, tv3_trans trans, int32_t nrhs, const flo
         const int64_t R = yl, K = xl;
         const bool mfma = op->kind == OpKind::DENSE && op->dtype == TV3_BF16 && R % 256 == 0 &&
                           K % 64 == 0 && op->lda % 8 == 0 && ldx % 4 == 0;
-        // a sparse matrix in row blocks is read once for up to eight vectors; the
-        // workspace needs its order kept over streams, which a capture cannot
+        // a sparse matrix in row blocks is read once for up to eight vectors; not
+        // under capture, which can neither grow the workspace nor keep its order
         const SparseRows *S = op->kind == OpKind::CSR ? (T ? &op->AT : &op->A)
                               : op->kind == OpKind::HYBRID && T ? &op->AT : nullptr;
         if (S && nrhs > 1 && spmv_multi_ok(*S) && !capturing(s)) {
-            float *xt = reinterpret_cast<float *>(
-                op->multi_ws.acquire(s, spmv_multi_scratch(*S) * sizeof(float)));
+            const StreamTurn turn(&op->multi_order, s);
+            const size_t need = spmv_multi_scratch(*S) * sizeof(float);
+            if (op->multi_ws.bytes() < need) op->multi_ws.alloc(need);
+            float *xt = reinterpret_cast<float *>(op->multi_ws.p);
             int32_t j = 0;
             for (; nrhs - j > 1; j += 8)
                 spmv_multi(*S, std::min(8, nrhs - j), X + j * ldx, ldx, Y + j * ldy, ldy, xt, s);
             if (j < nrhs) spmv_csr(*S, X + j * ldx, Y + j * ldy, s);
-            op->multi_ws.release(s);
             return;
         }
         if (!mfma && op->kind == OpKind::DENSE) {
@@ -616,8 +616,8 @@ tv3_status tv3_matvec_multi(tv3_op *op, tv3_trans trans, int32_t nrhs, const flo
         for (int64_t S = 2; S <= K / 64; S += S & (S - 1) ? S / 3 : S / 2)   // 2, 3, 4, 6, 8, 12
             if (fits(S)) splits = (int)S;
         const size_t need = gemm_rhs_scratch(R, splits) * sizeof(float);
-        if (op->ctx->scratch.bytes() < need) op->ctx->scratch.alloc(need);
-        float *part = reinterpret_cast<float *>(op->ctx->scratch.p);
+        const StreamScratch::Lease lease = op->ctx->scratch.take(s, need);
+        float *part = reinterpret_cast<float *>(lease.p);
         dense_operand_order(op, s);
         const uint16_t *M = (const uint16_t *)(T ? op->dense_oT.p : op->dense_oN.p);
         for (int32_t c = 0; c < nrhs; c += 64)

@@ -5,6 +5,7 @@
 // library and become tv3_status codes at the C ABI (tv3_abi.cpp).
 #pragma once
 
+#include <algorithm>
 #include <atomic>
 
 #include <hip/hip_bf16.h>
@@ -92,30 +93,6 @@ struct PinnedBuf {
     }
 };
 
-// Workspace of an object's calls that may run on several streams: acquire
-// makes the stream wait for the last use, release marks the end of this one.
-// Grown on demand (freeing the smaller buffer waits for the device), kept
-// until the object is destroyed.  Not for a stream that is being captured.
-struct SharedScratch {
-    DevBuf<uint8_t> buf;
-    hipEvent_t done = nullptr;
-    bool used = false;
-    SharedScratch() = default;
-    SharedScratch(const SharedScratch &) = delete;
-    SharedScratch &operator=(const SharedScratch &) = delete;
-    ~SharedScratch() { if (done) (void)hipEventDestroy(done); }
-    uint8_t *acquire(hipStream_t s, size_t bytes) {
-        if (!done) TV3_HIP(hipEventCreateWithFlags(&done, hipEventDisableTiming));
-        if (used) TV3_HIP(hipStreamWaitEvent(s, done, 0));
-        if (buf.bytes() < bytes) buf.alloc(bytes);
-        return buf.p;
-    }
-    void release(hipStream_t s) {
-        TV3_HIP(hipEventRecord(done, s));
-        used = true;
-    }
-};
-
 inline bool capturing(hipStream_t s) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &st) != hipSuccess) {
@@ -124,6 +101,92 @@ inline bool capturing(hipStream_t s) {
     }
     return st != hipStreamCaptureStatusNone;
 }
+
+// The order of calls that use one buffer from several streams: a call's stream
+// waits for the last use, and the end of the call is the next one's wait.  Not
+// for a stream that is being captured.  Costs about 4 us a call (a barrier on
+// the device).
+struct StreamOrder {
+    hipEvent_t done = nullptr;
+    bool used = false;
+    StreamOrder() = default;
+    StreamOrder(const StreamOrder &) = delete;
+    StreamOrder &operator=(const StreamOrder &) = delete;
+    ~StreamOrder() { if (done) (void)hipEventDestroy(done); }
+    void enter(hipStream_t s) {
+        if (!done) TV3_HIP(hipEventCreateWithFlags(&done, hipEventDisableTiming));
+        if (used) TV3_HIP(hipStreamWaitEvent(s, done, 0));
+    }
+    void leave(hipStream_t s) {
+        if (hipEventRecord(done, s) == hipSuccess) used = true;
+    }
+};
+
+// one call's turn in it (order may be NULL), ended where the call ends or throws
+struct StreamTurn {
+    StreamOrder *order;
+    hipStream_t s;
+    StreamTurn(StreamOrder *order, hipStream_t s) : order(order), s(s) {
+        if (order) order->enter(s);
+    }
+    StreamTurn(StreamTurn &&o) noexcept : order(o.order), s(o.s) { o.order = nullptr; }
+    StreamTurn &operator=(const StreamTurn &) = delete;
+    ~StreamTurn() { if (order) order->leave(s); }
+};
+
+// The workspaces of products that may run on several streams at once, grown
+// on demand (freeing the smaller buffer waits for the device) and kept until
+// their owner is destroyed.  The first kOwned streams have a buffer each, in
+// whose order they use it; any further stream takes turns on one more.  Calls
+// that a capture records share a buffer that nothing else uses, and one that
+// grows leaves the smaller to the graphs that hold its address: graphs of one
+// owner's products are not replayed at the same time.
+//
+// A buffer has at least 4 MiB: one of 2 MiB (8192 x 16384 BF16, A x) took 430
+// us to come by, 4 MiB 280, and it grows less often.
+struct StreamScratch {
+    static constexpr int kOwned = 3;
+    static constexpr size_t kLeast = size_t(4) << 20;
+    struct Own {
+        bool taken = false;
+        hipStream_t stream = nullptr;
+        DevBuf<uint8_t> buf;
+    } own[kOwned];
+    DevBuf<uint8_t> rest;
+    StreamOrder order;
+    std::vector<DevBuf<uint8_t>> recorded;     // the last is in use
+
+    struct Lease {
+        uint8_t *p;
+        StreamTurn turn;
+    };
+    Lease take(hipStream_t s, size_t bytes) {
+        bytes = std::max(bytes, kLeast);
+        if (capturing(s)) {
+            if (recorded.empty() || recorded.back().bytes() < bytes) {
+                // in the default mode an allocation would end the capture
+                hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+                TV3_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+                struct Restore {
+                    hipStreamCaptureMode mode;
+                    ~Restore() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+                } restore{mode};
+                recorded.emplace_back(bytes);
+            }
+            return {recorded.back().p, StreamTurn(nullptr, s)};
+        }
+        for (Own &o : own) {
+            if (o.taken && o.stream != s) continue;
+            o.taken = true;
+            o.stream = s;
+            if (o.buf.bytes() < bytes) o.buf.alloc(bytes);
+            return {o.buf.p, StreamTurn(nullptr, s)};
+        }
+        StreamTurn turn(&order, s);
+        if (rest.bytes() < bytes) rest.alloc(bytes);
+        return {rest.p, std::move(turn)};
+    }
+};
 
 inline size_t dtype_size(tv3_dtype t) {
     switch (t) {
@@ -392,7 +455,7 @@ struct tv3_ctx {
     // and U_true, grown to the largest solve so far (a solve waits for its
     // stream before it returns, and a context serves one host thread)
     tv3::DevBuf<uint8_t> plain_ws, host_ws;
-    tv3::DevBuf<uint8_t> scratch;   // general workspace (grown on demand)
+    tv3::StreamScratch scratch;     // partial sums of dense products
     std::unique_ptr<tv3::CtxSession> batch_session;   // the last batched solve, for reuse
 };
 
@@ -410,7 +473,8 @@ struct tv3_op {
     int64_t lda = 0;
     tv3::DevBuf<uint8_t> dense_oN, dense_oT;   // A and A^T in MFMA operand order (multi-RHS
                                                // products), built on demand
-    tv3::SharedScratch multi_ws;               // sparse products of several vectors
+    tv3::DevBuf<uint8_t> multi_ws;             // sparse products of several vectors,
+    tv3::StreamOrder multi_order;              // one call at a time
     // DYNAMIC / HYBRID
     tv3::DynGeom geo;
     // CSR built from a geometry: the locality order of its rays (may be empty)
