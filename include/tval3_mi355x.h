@@ -195,13 +195,13 @@ tv3_status tv3_op_csr_download(tv3_op *op, int32_t *rowptr, int32_t *col, double
  * x, y device pointers; y is fully overwritten; asynchronous on stream
  * (a hipStream_t; NULL is the null stream, as for the reference's
  * stream = 0 default; pass tv3_ctx_stream(ctx) for the context stream).
- * Products on several streams may be in flight at once: each of the first
- * three streams of a workspace (a context's for dense products) has a buffer
- * of its own, further ones wait for each other (finish a stream's products
- * before destroying it).  Products recorded into graphs
- * share one more buffer, so two graphs with dense products of one context must
- * not be replayed at the same time; tv3_matvec allocates where a workspace has
- * to grow, also under stream capture.
+ * Products on several streams may be in flight at once.  Dense products use a
+ * workspace of their context, matrix-free Siddon products in tiles one of their
+ * operator: its first three streams have a buffer each, further ones wait for
+ * each other (finish a stream's products before destroying it).  Products
+ * recorded into graphs share one more buffer, so two graphs that hold products
+ * of one workspace must not be replayed at the same time.  tv3_matvec allocates
+ * where a workspace has to grow, also under stream capture.
  * mulChain is a multi-GPU hint and has no counterpart here. */
 tv3_status tv3_matvec(tv3_op *op, tv3_trans trans, const float *x_dev, float *y_dev,
                       void *stream);
@@ -214,8 +214,9 @@ tv3_status tv3_matvec_f64(tv3_op *op, tv3_trans trans, const double *x_dev, doub
  * a static device array of 16 MiB per GPU (set up by tv3_ctx_create) instead
  * of the context's workspace; a dense A x that needs more (rows times column
  * slabs, min(128, ceil(cols/64)) slabs, 4 bytes each) returns
- * TV3_E_UNSUPPORTED.  Every other product uses no scratch.  Results equal
- * tv3_matvec's bit for bit.  All calls on one GPU share that array: calls
+ * TV3_E_UNSUPPORTED.  A matrix-free Siddon operator in tiles uses the buffer its
+ * fused solves use; every other product uses no scratch.  Results equal
+ * tv3_matvec's bit for bit.  All calls on one GPU share those: calls
  * that overlap on one GPU (two streams, two host threads) race. */
 tv3_status tv3_matvec_noalloc(tv3_op *op, tv3_trans trans, const float *x_dev, float *y_dev,
                               void *stream);

@@ -6,7 +6,7 @@ products the operator's copies as well."""
 import numpy as np
 import pytest
 
-from tval3_amd import api
+from tval3_amd import api, workload as wl
 
 pytestmark = pytest.mark.gpu
 
@@ -78,3 +78,56 @@ def test_matrix_core_first_product_on_each_stream():
     torch.cuda.synchronize()
     want = torch.from_numpy(A).cuda().double() @ X.double()
     assert torch.equal(a.double(), want) and torch.equal(b.double(), want)
+
+
+def _tiles(ctx):
+    # 32^3 voxels, 16,384 rays: tile products of some 20 us
+    return api.DynamicOperator(ctx, wl.transducer_geometry(64, 256, dims=(32, 32, 32), seed=3),
+                               "siddon")
+
+
+def test_siddon_tiles():
+    import torch
+    assert torch.cuda.is_available()
+    op = _tiles(api.Context(0))
+    xs = [_cols(op.n, 1, s)[:, 0].contiguous() for s in range(3)]
+    rs = [_cols(op.m, 1, s)[:, 0].contiguous() for s in range(3)]
+    _check([lambda x=x: op.mat_vec_mul(x) for x in xs] +
+           [lambda r=r: op.mat_vec_mul(r, trans=True) for r in rs])
+    # without an allocation: one call after the other, the same bits
+    for x, r in zip(xs, rs):
+        for v, trans in ((x, False), (r, True)):
+            y = torch.empty(op.n if trans else op.m, device="cuda")
+            op.mat_vec_mul_noalloc(v, y, trans=trans)
+            assert torch.equal(y, op.mat_vec_mul(v, trans=trans))
+
+
+def test_siddon_tiles_beside_a_solve_and_a_graph():
+    import torch
+    assert torch.cuda.is_available()
+    ctx = api.Context(0)
+    op = _tiles(ctx)
+    x, r = _cols(op.n, 1, 1)[:, 0].contiguous(), _cols(op.m, 1, 2)[:, 0].contiguous()
+    b = np.linspace(0.5, 1.5, op.m).astype(np.float32)
+    o = api.default_opts(maxit=4, tol=0.0, tol_inn=0.0, solver="fused")
+    want = op.mat_vec_mul(x), op.mat_vec_mul(r, trans=True)
+    U = api.tval3_gpu_3d(ctx, op, b, (32, 32, 32), o)[0]
+    y, z = torch.zeros_like(want[0]), torch.zeros_like(want[1])
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        op.mat_vec_mul(x, y)
+        op.mat_vec_mul(r, z, trans=True)
+    other = torch.cuda.Stream()
+    for k in range(4):
+        y.zero_()
+        z.zero_()
+        torch.cuda.synchronize()
+        for _ in range(5):
+            graph.replay()
+        with torch.cuda.stream(other):
+            got = [(op.mat_vec_mul(x), op.mat_vec_mul(r, trans=True)) for _ in range(20)]
+        assert (api.tval3_gpu_3d(ctx, op, b, (32, 32, 32), o)[0] == U).all(), k
+        torch.cuda.synchronize()
+        for g in got + [(y, z)]:
+            assert torch.equal(g[0], want[0]) and torch.equal(g[1], want[1]), k

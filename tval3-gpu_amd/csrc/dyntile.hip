@@ -18,6 +18,7 @@
 // positions of its entries there (ray order).
 #include <algorithm>
 #include <numeric>
+#include <optional>
 
 // The entries one A^T box keeps in LDS where a workgroup may hold 160 KiB
 // (15360 otherwise): 19456 entries (76 KiB) let two workgroups share a CU,
@@ -426,7 +427,7 @@ std::unique_ptr<FusedLayout> build_dyn_layout(tv3_op *op) {
     R.lanes = per_ray > 24 ? 16 : per_ray > 12 ? 8 : 4;
     upload_vec(ctx, R.ptr, rptr);
     upload_vec(ctx, R.seg, rseg);
-    R.part.alloc(nsegF > 0 ? nsegF : 1);
+    R.part.alloc(std::max<int64_t>({nsegF, m, 1}));      // or r: see dyn_tile_apply
     // ray end points in internal order -> traversal records on the device
     std::vector<float> ends(6 * (m > 0 ? m : 1), 0.f);
     for (int64_t i = 0; i < m; ++i) {
@@ -448,7 +449,8 @@ std::unique_ptr<FusedLayout> build_dyn_layout(tv3_op *op) {
         TV3_HIP(hipGetLastError());
         TV3_HIP(hipStreamSynchronize(ctx->stream));
     }
-    D->rin.alloc(m > 0 ? m : 1);
+    D->work_bytes = R.part.bytes();
+    D->work.reserve(D->work_bytes);
     TV3_HIP(hipStreamSynchronize(ctx->stream));
     // the matrices themselves are not kept: sizes only
     for (SparseRows *S : {&L->A, &L->AT}) {
@@ -462,18 +464,24 @@ std::unique_ptr<FusedLayout> build_dyn_layout(tv3_op *op) {
     return L;
 }
 
-bool dyn_tile_apply(tv3_op *op, bool trans, const float *x, float *y, hipStream_t s) {
+bool dyn_tile_apply(tv3_op *op, bool trans, const float *x, float *y, hipStream_t s, bool noalloc) {
     FusedLayout *F = op->fused.get();
     if (!F || !F->dyn) return false;
     // natural order in and out without passes of its own, except r: A x stages
     // its boxes from x as it is, and the sums are stored through the maps
     DynTiles &D = *F->dyn;
+    std::optional<StreamScratch::Lease> lease;
+    float *work = F->RS.part.p;              // the segments' sums, or r
+    if (!noalloc) {
+        lease.emplace(D.work.take(s, D.work_bytes));
+        work = reinterpret_cast<float *>(lease->p);
+    }
     if (!trans) {
-        launch_dyn_N<true, float>(D, x, F->RS.part.p, nullptr, s);
-        launch_seg_sum(F->RS, EpiScatter{y, F->r_int2nat.p}, s);
+        launch_dyn_N<true, float>(D, x, work, nullptr, s);
+        launch_seg_sum(F->RS, work, EpiScatter{y, F->r_int2nat.p}, s);
     } else {
-        permute_gather(x, F->r_int2nat.p, D.rin.p, op->m, s);
-        launch_dyn_T<float>(D, D.rin.p, EpiScatter{y, F->v_int2nat.p}, s);
+        permute_gather(x, F->r_int2nat.p, work, op->m, s);
+        launch_dyn_T<float>(D, work, EpiScatter{y, F->v_int2nat.p}, s);
     }
     TV3_HIP(hipGetLastError());
     return true;

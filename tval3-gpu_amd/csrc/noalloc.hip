@@ -2,14 +2,15 @@
 // device allocation, for callers that cannot allocate (code under HIP graph
 // capture, tight serving loops, harnesses that forbid hipMalloc).
 //
-// Of the products tv3_matvec runs, only the dense A x uses scratch memory:
-// the split-K partial sums of its column slabs (dense.hip), which tv3_matvec
-// keeps in a context workspace grown by hipMalloc.  Here they go to a
+// Of the products tv3_matvec runs, the dense A x uses scratch memory that
+// grows: the split-K partial sums of its column slabs (dense.hip), which
+// tv3_matvec keeps in workspaces of the context.  Here they go to a
 // file-scope device array of fixed size instead.  Each GPU holds its own copy
 // of the array until the process ends; its address on a device is looked up
 // once, with that device current, when the first context on the device is
-// created (tv3_ctx_create), and kept per device.  Every other product (CSR,
-// dense A^T x, dynamic, hybrid) uses no scratch and is called as is.
+// created (tv3_ctx_create), and kept per device.  A matrix-free operator in
+// tiles uses its layout's own buffer, which the solver uses too.  Every other
+// product (CSR, dense A^T x, hybrid) uses no scratch and is called as is.
 #include <mutex>
 
 #include "tv3_internal.hpp"
@@ -67,7 +68,8 @@ tv3_status tv3_matvec_noalloc(tv3_op *op, tv3_trans trans, const float *x, float
             TV3_REQUIRE(ws != nullptr, TV3_E_INTERNAL,
                         "the allocation-free scratch of this device is not set up");
             dense_gemv_ws(op, x, y, s, ws, kScratchBytes);
-        } else {
+        } else if (!(op->kind == OpKind::DYNAMIC &&
+                     dyn_tile_apply(op, trans == TV3_T, x, y, s, /*noalloc=*/true))) {
             op_apply(op, trans == TV3_T, x, y, s);
         }
         TV3_HIP(hipGetLastError());

@@ -831,8 +831,9 @@ inline int seg_sum_blocks(const SegSum &R) {
     return (int)ng;
 }
 
+// part: the segments' sums (R.part, or a workspace of as many)
 template <typename Epi>
-void launch_seg_sum(const SegSum &R, const Epi &epi, hipStream_t s) {
+void launch_seg_sum(const SegSum &R, const float *part, const Epi &epi, hipStream_t s) {
     constexpr int NLB = kSegSumNLB;
     const int L = R.lanes;
     const int64_t nl = seg_sum_logical(R);
@@ -841,13 +842,17 @@ void launch_seg_sum(const SegSum &R, const Epi &epi, hipStream_t s) {
 #define TV3_SCASE(LL)                                                                     \
     case LL:                                                                              \
         hipLaunchKernelGGL((k_seg_sum<LL, NLB, Epi>), dim3(g), dim3(256), 0, s, R.rows,     \
-                           R.ptr.p, R.seg.p, R.part.p, epi, nl);                          \
+                           R.ptr.p, R.seg.p, part, epi, nl);                          \
         break;
     switch (L) {
         TV3_SCASE(2) TV3_SCASE(4) TV3_SCASE(8) TV3_SCASE(16) TV3_SCASE(32)
     default: throw tv3_error(TV3_E_ARG, "segment-sum lanes must be a power of two in [2, 32]");
     }
 #undef TV3_SCASE
+}
+template <typename Epi>
+void launch_seg_sum(const SegSum &R, const Epi &epi, hipStream_t s) {
+    launch_seg_sum(R, R.part.p, epi, s);
 }
 
 // A x of a fused layout (rows = rays) with epilogue epi; `active` (may be

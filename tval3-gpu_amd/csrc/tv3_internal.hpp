@@ -160,6 +160,8 @@ struct StreamScratch {
         uint8_t *p;
         StreamTurn turn;
     };
+    // the first stream's buffer, allocated ahead of its first call
+    void reserve(size_t bytes) { own[0].buf.alloc(std::max(bytes, kLeast)); }
     Lease take(hipStream_t s, size_t bytes) {
         bytes = std::max(bytes, kLeast);
         if (capturing(s)) {
@@ -383,7 +385,10 @@ struct DynTiles {
     DevBuf<uint32_t> pptr;           // n + 1: padded starts of the voxel rows
     DevBuf<uint16_t> pos;            // per voxel row its entries' positions in its bwd
                                      // box, ray order, padded to 4 with the position ne
-    DevBuf<float> rin;               // a caller's r in internal ray order (m)
+    // A caller's product: the segments' sums, or r in internal ray order.  (The
+    // solver and the allocation-free products use SegSum::part.)
+    StreamScratch work;
+    size_t work_bytes = 0;
 };
 
 // The fused solver's internal layout of a sparse operator: voxels numbered by
@@ -568,7 +573,8 @@ void renumber_rows(tv3_ctx *ctx, const SparseRows &A, const std::vector<int32_t>
 std::unique_ptr<FusedLayout> build_dyn_layout(tv3_op *op);
 // y = A x / A^T x of a matrix-free operator by its tile products, natural
 // order in and out; false when it has none (FP32 vectors)
-bool dyn_tile_apply(tv3_op *op, bool trans, const float *x, float *y, hipStream_t s);
+bool dyn_tile_apply(tv3_op *op, bool trans, const float *x, float *y, hipStream_t s,
+                    bool noalloc = false);
 // panel forms of a prebuilt A^T (rows = voxels in tiles of 512 rows, sources =
 // rays), one per row-block size in blks; false when a panel would need more
 // distinct rays than its local indices address or the weights are not F32,
