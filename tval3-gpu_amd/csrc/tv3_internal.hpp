@@ -142,11 +142,15 @@ struct StreamTurn {
 // grows leaves the smaller to the graphs that hold its address: graphs of one
 // owner's products are not replayed at the same time.
 //
-// A buffer has at least 4 MiB: one of 2 MiB (8192 x 16384 BF16, A x) took 430
-// us to come by, 4 MiB 280, and it grows less often.
+// A buffer above 1 MiB has at least 4 MiB: one of 2 MiB (8192 x 16384 BF16,
+// A x) made the first product take 430 us, 4 MiB 280; smaller ones come from
+// the runtime's own blocks (1638 x 4096 FP32, 0.4 MB: first pass 55 us, 92 with
+// 4 MiB).
 struct StreamScratch {
     static constexpr int kOwned = 3;
-    static constexpr size_t kLeast = size_t(4) << 20;
+    static size_t rounded(size_t bytes) {
+        return bytes > (size_t(1) << 20) ? std::max(bytes, size_t(4) << 20) : bytes;
+    }
     struct Own {
         bool taken = false;
         hipStream_t stream = nullptr;
@@ -161,9 +165,9 @@ struct StreamScratch {
         StreamTurn turn;
     };
     // the first stream's buffer, allocated ahead of its first call
-    void reserve(size_t bytes) { own[0].buf.alloc(std::max(bytes, kLeast)); }
+    void reserve(size_t bytes) { own[0].buf.alloc(rounded(bytes)); }
     Lease take(hipStream_t s, size_t bytes) {
-        bytes = std::max(bytes, kLeast);
+        bytes = rounded(bytes);
         if (capturing(s)) {
             if (recorded.empty() || recorded.back().bytes() < bytes) {
                 // in the default mode an allocation would end the capture
