@@ -240,7 +240,9 @@ tv3_status tv3_matvec_multi(tv3_op *op, tv3_trans trans, int32_t nrhs, const flo
 /* tval3_gpu_3d(U, A, b, opts, Ut, pagelocked, mainGPU, numGPUs, gpuArray)
  * (3d/tval3_gpu_3d.cpp:1673-1745, core loop :1088-1345) for float data.
  * b_host: m floats; U_host: n floats (output; input too if opts->warm_start);
- * Ut_host: n floats or NULL (info->rel_error); hist may be NULL. */
+ * Ut_host: n floats or NULL (info->rel_error); hist may be NULL.  The plain
+ * solver's vectors (33 of n, 8 of m) and a host solve's device copies stay with
+ * the context until it is destroyed, at the largest solve's size. */
 tv3_status tv3_solve(tv3_ctx *ctx, tv3_op *op, const tv3_opts *opts, const int32_t dims[3],
                      const float *b_host, float *U_host, const float *Ut_host, tv3_info *info,
                      tv3_history *hist);

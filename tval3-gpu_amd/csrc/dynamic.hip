@@ -167,9 +167,11 @@ __device__ __forceinline__ void ray_ends(const GeoView &g, int64_t k, R p0[3], R
 // share a ray's steps, one behind the other (rays in bundles of neighbours, so
 // the lanes of a wavefront gather near each other), and gather eight voxels at
 // a time; one at a time, each step waited for its gather.  At 128^3 with
-// 262,144 rays 206 -> 77 us, now bound by the gathers' line look-ups (4 to 32
-// at a time, bundles of 4^2 to 32^2 rays and workgroups of 64 to 1024 threads
-// all take 77-79 us; x in bricks of 4 x 4 x 2 voxels 70, and 6 for the copy).
+// 262,144 rays 206 -> 77 us, now bound by the lines of the gathers: 19.6M L1
+// accesses (0.4 a clock and CU), 13.5M of them on to L2 (22 TB/s; vector issue
+// takes 13 us).  4 to 32 at a time, bundles of 4^2 to 32^2 rays and workgroups
+// of 64 to 1024 threads all take 77-79 us; x in bricks of 4 x 4 x 2 voxels 70,
+// and 6 for the copy.
 template <typename T, typename AccT>
 __global__ __launch_bounds__(64) void k_bres_N(GeoView g, const int32_t *__restrict__ bundle,
                                                const int4 *__restrict__ walk,
@@ -202,7 +204,8 @@ __global__ __launch_bounds__(64) void k_bres_N(GeoView g, const int32_t *__restr
 }
 
 // N of a Siddon operator likewise: sid_walk's steps with eight gathers at a
-// time (77 x 101 x 90 voxels, 90,150 rays: 73 -> 32 us).  The Siddon operator
+// time (77 x 101 x 90 voxels, 90,150 rays: 73 -> 32 us, of which the vector
+// instructions take 24).  The Siddon operator
 // is the FP32 traversal: FP64 products accumulate its weights in FP64 (the
 // same matrix in both precisions).
 template <typename T, typename AccT>
@@ -291,9 +294,10 @@ __global__ __launch_bounds__(64) void k_sid_N(GeoView g, const int32_t *__restri
 // adds it to a cleared y, whole lines at a time).  The sums are FP64 for FP32
 // vectors too: an LDS FP64 add serves a wavefront in 22 clocks, an FP32 add
 // in 196 (measured, random addresses), which at first bound the kernel: 134
-// us at 128^3 with 262,144 Bresenham rays against 44 us now (1025 us with one
-// memory atomic per entry).  Parts of equal length are neighbours in the
-// list, so the lanes of a wavefront end together.
+// us at 128^3 with 262,144 Bresenham rays against 44 us now, of which LDS is
+// busy 24 and vector issue 21 (1025 us with one memory atomic per entry).
+// Parts of equal length are neighbours in the list, so the lanes of a wavefront
+// end together.
 template <bool SID, typename T>
 __global__ __launch_bounds__(kBoxThreads) void k_box_T(GeoView g, int nby, int nbx,
                                                        const int4 *__restrict__ items,

@@ -160,11 +160,12 @@ __device__ __forceinline__ double row_fma(const double2 *wx, int a, int e, int l
 // row (a voxel next to a transducer) is summed lane by lane, J gathers in
 // flight.
 //
-// Bound by the line fills of the gathers (L2 -> L1, 128 B each, ~30 TB/s)
-// and, where x outgrows an L2 slice, by its misses.  us, against 2048-entry
+// Bound by the line fills of the gathers (L2 -> L1, 128 B each: 23.5M for
+// either product at 128^3, 28 TB/s in A^T) and, where x outgrows an L2 slice,
+// by its misses (A: 4.3M, 22 TB/s of fills; A^T 1.9M).  us, against 2048-entry
 // blocks of a 256-thread workgroup: 64^3 voxels x 65,536 rays FP32 weights
 // A^T 27.0 -> 18.0, A 17.2 -> 17.0; 128^3 x 262,144 FP16 A^T 130 -> 107,
-// A 149 -> 148, FP64 A^T 298 -> 186, A 300 -> 260 (k_csr_f64); A in natural
+// A 149 -> 148, FP64 A^T 298 -> 187, A 300 -> 260 (k_csr_f64); A in natural
 // block order (order_blocks).
 //
 // Acc = double also serves FP32 vectors whose row sums are rounded once: their

@@ -1,6 +1,7 @@
-// vec.hip -- kernels of the reference-shaped ("plain") TVAL3 loop: one kernel
-// per vector operation, reductions as FP64 block partials summed in a fixed
-// order.  Float and double instantiations.
+// vec.hip -- vector kernels of the reference-shaped ("plain") TVAL3 loop: the
+// operations between two host decisions share kernels, reductions are FP64 block
+// partials totalled on the device in a fixed order.  Float and double
+// instantiations.
 //
 // Reference kernels restated (3d/tval3_gpu_3d_kernels.cu): vec_add :75-108,
 // D :170-215, D^T :479-510, lam2/lam4 :724-771 (all three components, sigma
