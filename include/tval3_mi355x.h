@@ -199,9 +199,10 @@ tv3_status tv3_op_csr_download(tv3_op *op, int32_t *rowptr, int32_t *col, double
  * workspace of their context, matrix-free Siddon products in tiles one of their
  * operator: its first three streams have a buffer each, further ones wait for
  * each other (finish a stream's products before destroying it).  Products
- * recorded into graphs share one more buffer, so two graphs that hold products
- * of one workspace must not be replayed at the same time.  tv3_matvec allocates
- * where a workspace has to grow, also under stream capture.
+ * recorded into graphs share one more buffer, so products of one workspace must
+ * not lie on parallel branches of a graph, nor in graphs that are replayed at
+ * the same time.  tv3_matvec allocates where a workspace has to grow, also under
+ * stream capture.
  * mulChain is a multi-GPU hint and has no counterpart here. */
 tv3_status tv3_matvec(tv3_op *op, tv3_trans trans, const float *x_dev, float *y_dev,
                       void *stream);
